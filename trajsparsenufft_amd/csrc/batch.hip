@@ -17,7 +17,7 @@
 
 namespace tsn {
 int launch_split_panel_il(const float2* in, uint32_t rows, uint32_t coils, float scale, uint32_t* out,
-                          hipStream_t stream, int values);
+                          hipStream_t stream, int values, bool lines);
 }  // namespace tsn
 
 using namespace tsn;
@@ -29,7 +29,7 @@ namespace {
 template <bool BF16>
 __global__ __launch_bounds__(256) void batch_split_kernel(const float2* const* __restrict__ meas,
                                                           const uint32_t* __restrict__ coils_of,
-                                                          const uint32_t* __restrict__ m_of, uint32_t blocks_max,
+                                                          const uint32_t* __restrict__ m_of, bool lines,
                                                           float scale, uint32_t* __restrict__ panels,
                                                           uint64_t panel_stride) {
   const uint32_t z = blockIdx.y;
@@ -37,6 +37,7 @@ __global__ __launch_bounds__(256) void batch_split_kernel(const float2* const* _
   const uint32_t blocks = (coils + kCoilsPerBlock - 1) / kCoilsPerBlock;
   const uint64_t total = static_cast<uint64_t>(blocks) * m * kN;
   uint32_t* out = panels + z * panel_stride;
+  const bool two_lines = lines && blocks == 2;  // both blocks of a row in one 128-byte line
   for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < total;
        g += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
     const int n = static_cast<int>(g & 15);
@@ -57,9 +58,8 @@ __global__ __launch_bounds__(256) void batch_split_kernel(const float2* const* _
       w = static_cast<uint32_t>(__builtin_bit_cast(uint16_t, h)) |
           (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, r)) << 16);
     }
-    out[g] = w;
+    out[two_lines ? (static_cast<uint64_t>(row) * 2 + b) * kN + n : g] = w;
   }
-  (void)blocks_max;
 }
 
 // x_z (column-major [n1][n0]) -> x_out[z] ([n0][n1]); history sqrt(rho) and
@@ -89,6 +89,7 @@ struct tsn_batch {
   tsn_plan_config cfg{};
   int device = 0;
   uint32_t problems = 0, cmax = 0, bmax = 0, mmax = 0, pixels = 0, vec_blocks = 0, grid = 0;
+  bool lines = false;  // problems of 9..16 coils keep line-row panels (kLines; see kMaxLineCols)
   std::vector<uint32_t> coils, m;
   std::vector<const tsn_direction*> fwd, adj;
   InterpBatch ib_fwd[2], ib_adj[2];  // parts of one and of two coil blocks
@@ -165,6 +166,7 @@ FftArgs batch_fft_args(const tsn_batch* bt) {
   a.panel_il = bt->pan_il;
   a.grid = bt->grid_buf;
   a.t_inv = bt->t_inv;
+  a.panel_lines = bt->lines ? 1u : 0u;
   a.grid_blocked = 1;  // each problem's rows compact (<= 8 coils) or in 8-coil blocks
   a.image_stride = bt->pixels;
   a.smaps_stride = static_cast<uint64_t>(bt->pixels) * bt->cmax;
@@ -189,10 +191,10 @@ int enqueue_batch_cg(tsn_batch* bt, uint32_t iterations, hipStream_t s) {
   const dim3 split_grid(std::min<uint64_t>(div_up(total, 256), 4096), S);
   if (bt->cfg.precision == TSN_PREC_SPLITBF16)
     hipLaunchKernelGGL(batch_split_kernel<true>, split_grid, dim3(256), 0, s, bt->meas_tab, bt->coils_dev,
-                       bt->m_dev, bt->bmax, norm, bt->smp_il, sample_stride(bt));
+                       bt->m_dev, bt->lines, norm, bt->smp_il, sample_stride(bt));
   else
     hipLaunchKernelGGL(batch_split_kernel<false>, split_grid, dim3(256), 0, s, bt->meas_tab, bt->coils_dev,
-                       bt->m_dev, bt->bmax, norm, bt->smp_il, sample_stride(bt));
+                       bt->m_dev, bt->lines, norm, bt->smp_il, sample_stride(bt));
   for (const InterpBatch& ib : bt->ib_adj)
     if (ib.n_problems) TSN_CHECK(launch_interp_batch(ib, kind, 1, true, 1.0f, s));
   // b written straight into p (r0 = p0 = b, x0 = 0), with the per-column
@@ -316,8 +318,8 @@ int build_interp_tables(tsn_batch* bt) {
   }
   for (int k = 0; k < 2; ++k) {
     if (bt->parts_fwd[k].empty()) continue;
-    TSN_CHECK(interp_batch_build(bt->parts_fwd[k], &bt->ib_fwd[k], bt->member_group, bt->coil_waves, bt->depth));
-    TSN_CHECK(interp_batch_build(bt->parts_adj[k], &bt->ib_adj[k], bt->member_group, bt->coil_waves, bt->depth));
+    TSN_CHECK(interp_batch_build(bt->parts_fwd[k], &bt->ib_fwd[k], bt->lines, bt->member_group, bt->coil_waves, bt->depth));
+    TSN_CHECK(interp_batch_build(bt->parts_adj[k], &bt->ib_adj[k], bt->lines, bt->member_group, bt->coil_waves, bt->depth));
   }
   return TSN_OK;
 }
@@ -457,6 +459,7 @@ int tsn_batch_create(const tsn_plan_config* cfg, const tsn_batch_problem* proble
     bt->mmax = std::max(bt->mmax, q.forward->h.output_size);
   }
   bt->bmax = div_up(bt->cmax, kCoilsPerBlock);
+  bt->lines = bt->grid <= kMaxLineCols && bt->mmax <= kMaxLineCols;
   const size_t px = bt->pixels, S = count;
   int rc = TSN_OK;
   auto A = [&](auto** ptr, size_t n) {

@@ -24,7 +24,9 @@ struct FftArgs {
   // coils, up to 8) or in 8-coil chunk blocks of 64-byte rows; without
   // grid_blocked, grid and panel32 rows are cstride wide.
   float2* t_fwd;           // rows [K0][n1]
-  uint32_t* panel_il;      // [block][K0*K1][16] hi | res << 16
+  uint32_t* panel_il;      // [block][K0*K1][16] hi | res << 16; with panel_lines, problems above 8 coils
+                           // hold both blocks of a row together: [K0*K1][32]
+  uint32_t panel_lines;
   float2* panel32;         // rows [K0*K1]
   const float2* grid;      // rows [K0*K1]
   float2* t_inv;           // rows [n1][K0]

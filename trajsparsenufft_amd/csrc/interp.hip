@@ -28,6 +28,8 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 namespace tsn {
 
@@ -39,7 +41,6 @@ enum OutMode { kOutCoilMajor = 0, kOutRowMajor = 1, kOutSplit16 = 2, kOutSplit16
 // Tile kinds: FP16 tiles x FP16 hi + residual on smfmac, the same on dense
 // MFMA, FP16 hi only, and BF16 tiles x BF16 hi + residual on smfmac.
 enum TileKind { kSparseSplit = 0, kDenseSplit = 1, kSparseHi = 2, kSparseSplitBF16 = 3 };
-
 
 struct InterpArgs {
   const WorkItem* items;
@@ -66,7 +67,8 @@ struct InterpArgs {
   float* out_f32;         // float2 output (coil- or row-major)
   _Float16* out_hi;       // split output panel blocks
   _Float16* out_res;
-  uint32_t* out_il;       // interleaved split output panel blocks
+  uint32_t* out_il;       // interleaved split output panel blocks, or line rows
+  uint32_t lines;         // one wave per coil block (WB = 2): the interleaved panels hold line rows, not blocks
   // row-major float2 output: (row, coil) at float2 (coil >> 3) * out_bs +
   // row * out_rs + (coil & 7) ([row][coils]: out_rs = coils, out_bs = 8)
   uint32_t out_rs;
@@ -98,9 +100,10 @@ struct InterpProblem {
   uint32_t coil_base;   // first coil of this block
   const uint32_t* panel_il;  // this block's input panel [n_cols][16]
   float* out_f32;       // the problem's float2 output
-  uint32_t* out_il;     // this block's split output panel [n_out][16]
+  uint32_t* out_il;     // this block's split output panel
   uint32_t out_rs;      // row-major output strides (as InterpArgs)
   uint64_t out_bs;
+  uint32_t lines;       // both panels hold two coil blocks as 128-byte line rows
 };
 
 // Global-space view of a plain pointer.  The kernel's loads and stores after
@@ -127,7 +130,8 @@ __device__ __forceinline__ InterpArgs problem_args(const InterpArgs& a, uint32_t
   v.coils = q.coils;
   v.coil_base = q.coil_base;
   v.panel_il = q.panel_il;
-  v.panel_stride = static_cast<uint64_t>(q.n_cols) * kN;  // block b's input panel follows at b strides
+  v.panel_stride = static_cast<uint64_t>(q.n_cols) * kN;
+  v.lines = q.lines;
   v.out_f32 = q.out_f32;
   v.out_il = q.out_il;
   v.out_rs = q.out_rs;
@@ -172,7 +176,7 @@ __device__ __forceinline__ float dc_apply(const InterpArgs& a, float v, uint32_t
   return dc_residual(v, y, a.dc_scale, w);
 }
 
-template <int OM, bool CONJ, bool ACC>
+template <int OM, bool CONJ, bool ACC, int WB>
 __device__ __forceinline__ void interp_epilogue(const InterpArgs& a, const int4& rows, int b,
                                                 const float4_t& acc_re, const float4_t& acc_im,
                                                 int lane) {
@@ -191,7 +195,9 @@ __device__ __forceinline__ void interp_epilogue(const InterpArgs& a, const int4&
     if (row < 0) continue;
     if constexpr (OM == kOutSplitBF16IL || OM == kOutSplit16IL) {
       if (a.dc_meas) v = dc_apply(a, v, coil, row, part);
-      glb(a.out_il)[(static_cast<size_t>(b) * a.n_out + row) * kN + n] = split_word<OM == kOutSplitBF16IL>(v);
+      const size_t o = WB > 1 && a.lines ? (static_cast<size_t>(row) * 2 + b) * kN
+                                         : (static_cast<size_t>(b) * a.n_out + row) * kN;
+      glb(a.out_il)[o + n] = split_word<OM == kOutSplitBF16IL>(v);
     } else if constexpr (OM == kOutSplit16) {
       asm volatile("" : "+v"(v));  // split the FP32 value (see split_word)
       const _Float16 hi = static_cast<_Float16>(v);
@@ -207,6 +213,70 @@ __device__ __forceinline__ void interp_epilogue(const InterpArgs& a, const int4&
       if constexpr (ACC) v += glb(a.out_f32)[o];
       glb(a.out_f32)[o] = v;
     }
+  }
+}
+
+// The epilogue of both coil blocks of kLines panels.  Accumulator b of lane n
+// of a quarter is word w = 4 (n & 7) + 2 (n >> 3) + b of the 32-word row (see
+// fetch_ops): part (n >> 1) & 1 (Re or Im) of coil 8 ((n >> 2) & 1) + 4 (n & 1)
+// + 2 (n >> 3) + b, and lane n ^ 2 holds the coil's other part.  Split outputs
+// write the two words with one 8-byte store (128 contiguous bytes a row);
+// float2 outputs exchange accumulators so that the Re lane holds both parts of
+// its b = 0 coil and the Im lane both parts of its b = 1 coil, one 8-byte store
+// each.
+template <int OM, bool CONJ, bool ACC>
+__device__ __forceinline__ void interp_epilogue_lines(const InterpArgs& a, const int4& rows,
+                                                      const float4_t (&acc_re)[2], const float4_t (&acc_im)[2],
+                                                      int lane) {
+  const uint32_t n = lane & 15;
+  const bool im = (n >> 1) & 1u;
+  const uint32_t coil0 = a.coil_base + ((n >> 2) & 1u) * kCoilsPerBlock + 4 * (n & 1) + 2 * (n >> 3);
+  const int rr[4] = {rows.x, rows.y, rows.z, rows.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = rr[i];
+    if constexpr (OM == kOutSplitBF16IL || OM == kOutSplit16IL) {
+      float v[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const float other = __shfl_xor(acc_im[b][i], 2);
+        v[b] = (im == CONJ ? acc_re[b][i] - other : acc_re[b][i] + other) * a.scale;
+      }
+      if (row < 0) continue;
+      if (a.dc_meas) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) v[b] = dc_apply(a, v[b], coil0 + b, row, im ? 1 : 0);
+      }
+      const u32x2_t w = {split_word<OM == kOutSplitBF16IL>(v[0]), split_word<OM == kOutSplitBF16IL>(v[1])};
+      glb(reinterpret_cast<u32x2_t*>(a.out_il))[static_cast<size_t>(row) * kN + 2 * (n & 7) + (n >> 3)] = w;
+    } else {
+      const float re = im ? acc_re[1][i] : acc_re[0][i], iv = im ? acc_im[1][i] : acc_im[0][i];
+      const float ore = __shfl_xor(im ? acc_re[0][i] : acc_re[1][i], 2);
+      const float oim = __shfl_xor(im ? acc_im[0][i] : acc_im[1][i], 2);
+      const float rr_ = im ? ore : re, ri = im ? oim : iv;  // the Re channel's sums
+      const float ir = im ? re : ore, ii = im ? iv : oim;   // the Im channel's sums
+      float2_t v = {(CONJ ? rr_ + ii : rr_ - ii) * a.scale, (CONJ ? ir - ri : ir + ri) * a.scale};
+      const uint32_t coil = coil0 + (im ? 1u : 0u);
+      if (row < 0 || coil >= a.coils) continue;
+      size_t o;
+      if constexpr (OM == kOutCoilMajor) o = static_cast<size_t>(coil) * a.n_out + row;
+      else o = (coil >> 3) * a.out_bs + static_cast<size_t>(row) * a.out_rs + (coil & 7);
+      auto* out = glb(reinterpret_cast<float2_t*>(a.out_f32));
+      if constexpr (ACC) v += out[o];
+      out[o] = v;
+    }
+  }
+}
+
+// Rows of a group from the wave's accumulators (or from summed chunk slots).
+template <int NB, int IL, int OM, bool CONJ, bool ACC, int WB>
+__device__ __forceinline__ void write_group(const InterpArgs& a, const int4& rows, const float4_t (&acc_re)[NB],
+                                            const float4_t (&acc_im)[NB], int lane) {
+  if constexpr (IL == kLines) {
+    interp_epilogue_lines<OM, CONJ, ACC>(a, rows, acc_re, acc_im, lane);
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) interp_epilogue<OM, CONJ, ACC, WB>(a, rows, b, acc_re[b], acc_im[b], lane);
   }
 }
 
@@ -229,8 +299,8 @@ struct TileRsrc {
   rsrc_t cols, a, idx, dense, rows, hi[NB], res[NB];
 };
 
-template <int NB, bool IL>
-__device__ __forceinline__ TileRsrc<NB> make_tile_rsrc(const InterpArgs& a) {
+template <int NB, int IL, int WB>
+__device__ __forceinline__ TileRsrc<NB> make_tile_rsrc(const InterpArgs& a, uint32_t end_cut = 0) {
   TileRsrc<NB> r;
   const uint64_t tiles = a.n_tiles;
   r.cols = make_rsrc(a.tile_cols, tiles * kK * 4);
@@ -240,8 +310,10 @@ __device__ __forceinline__ TileRsrc<NB> make_tile_rsrc(const InterpArgs& a) {
   r.rows = make_rsrc(a.group_rows, static_cast<uint64_t>(a.n_groups) * 64);
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    if constexpr (IL) {
-      r.hi[b] = make_rsrc(a.panel_il + b * a.panel_stride, a.panel_stride * 4);
+    if constexpr (IL != kHalves) {
+      // (WB = 2: panel_il already points at the wave's block, to the panel's end in line rows)
+      if constexpr (IL == kLines) r.hi[b] = make_rsrc(a.panel_il, a.panel_stride * 8);
+      else r.hi[b] = make_rsrc(a.panel_il + b * a.panel_stride, a.panel_stride * (WB > 1 && a.lines ? 8 : 4) - end_cut);
       r.res[b] = r.hi[b];
     } else {
       r.hi[b] = make_rsrc(a.panel_hi + b * a.panel_stride, a.panel_stride * 2);
@@ -293,11 +365,17 @@ __device__ __forceinline__ void stage_cols(const TileRsrc<NB>& r, int first, int
 
 // Column words of the unit's k-th tile from the stage (the 16 lanes of a
 // quarter read the same 32 bytes: LDS broadcast).
+template <int IL>
 __device__ __forceinline__ TileCols staged_cols(const uint32_t* stage, int k, int lane) {
-  const u32x4_t* p = reinterpret_cast<const u32x4_t*>(stage + k * kK) + (lane >> 4) * 2;
   TileCols c;
-  c.c0 = p[0];
-  c.c1 = p[1];
+  if constexpr (IL == kLines) {  // four columns a lane (fetch_ops)
+    c.c0 = reinterpret_cast<const u32x4_t*>(stage + k * kK)[lane >> 3];
+    c.c1 = c.c0;
+  } else {
+    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(stage + k * kK) + (lane >> 4) * 2;
+    c.c0 = p[0];
+    c.c1 = p[1];
+  }
   return c;
 }
 
@@ -305,25 +383,43 @@ __device__ __forceinline__ TileCols staged_cols(const uint32_t* stage, int k, in
 // raw gathered panel words (kept unpacked until the multiply so no wait is
 // forced before then).  IL: one dword (hi | res << 16) per row; otherwise one
 // zero-extended half per row for hi (w[0..7]) and for the residual (w[8..15]).
-template <int NB, bool IL>
+template <int NB, int IL>
 struct TileOps {
   u32x4_t a0, a1;
   uint32_t idx, last;
   uint32_t w[NB][IL ? 8 : 16];
 };
 
-template <int KIND, int NB, bool IL>
-__device__ __forceinline__ void fetch_ops(const TileRsrc<NB>& r, int t, const TileCols& c, int lane,
+template <int KIND, int NB, int IL, int WB>
+__device__ __forceinline__ void fetch_ops(const TileRsrc<NB>& r, int t, const TileCols& c, int lane, uint32_t shift,
                                           TileOps<NB, IL>& o) {
   const uint32_t n = lane & 15;
   const uint32_t cw[8] = {c.c0.x, c.c0.y, c.c0.z, c.c0.w, c.c1.x, c.c1.y, c.c1.z, c.c1.w};
+  if constexpr (IL == kLines) {
+    // Whole 128-byte lines, 16 bytes a lane: lanes n < 8 of quarter q read its
+    // columns 8q .. 8q + 3, lanes n >= 8 columns 8q + 4 .. 8q + 7, words
+    // 4 (n & 7) .. + 3 of each (mma_tile exchanges half of them with lane
+    // n ^ 8).  Rows of 128 bytes in L2, 32 columns a step, 16 waves a CU: 80
+    // cycles a CU, against 104 as two 64-byte halves in 4-byte loads and 140
+    // in 8-byte loads.
+    static_assert(NB == 2, "line rows hold two coil blocks");
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32x4_t v =
+          __builtin_amdgcn_raw_buffer_load_b128(r.hi[0], static_cast<int>((cw[j] << 2) | ((n & 7) << 4)), 0, 0);
+      o.w[0][j] = v.x;
+      o.w[1][j] = v.y;
+      o.w[0][4 + j] = v.z;
+      o.w[1][4 + j] = v.w;
+    }
+  } else {
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if constexpr (IL) {
-        // row byte offset in the interleaved panel: column * 64 + n * 4
-        const uint32_t off = (cw[j] << 1) | (n << 2);
+      if constexpr (IL == kBlocks) {
+        // row byte offset in the interleaved panel: column * 64 (128 in line rows) + n * 4
+        const uint32_t off = (cw[j] << (WB > 1 ? shift : 1u)) | (n << 2);
         o.w[b][j] = __builtin_amdgcn_raw_buffer_load_b32(r.hi[b], static_cast<int>(off), 0, 0);
       } else {
         const uint32_t off = (j == 2 ? (cw[j] & 0x7FFFFFFFu) : cw[j]) | (n << 1);
@@ -332,6 +428,7 @@ __device__ __forceinline__ void fetch_ops(const TileRsrc<NB>& r, int t, const Ti
                                           : __builtin_amdgcn_raw_buffer_load_b16(r.res[b], static_cast<int>(off), 0, 0);
       }
     }
+  }
   }
   if constexpr (KIND == kDenseSplit) {
     o.a0 = __builtin_amdgcn_raw_buffer_load_b128(r.dense, lane * 32, t * (64 * 32), 0);
@@ -356,11 +453,25 @@ __device__ __forceinline__ half8_t pack_halves(const uint32_t* w, uint32_t sel) 
 }
 constexpr uint32_t kSelLo = 0x05040100u, kSelHi = 0x07060302u;
 
-template <int KIND, int NB, bool IL>
-__device__ __forceinline__ void mma_tile(const TileOps<NB, IL>& o, float4_t (&acc_re)[NB],
+// Exchange between lanes n and n ^ 8 of each 16-lane row: lanes n < 8 take the
+// partner's x into y, lanes n >= 8 the partner's y into x.
+__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {
+  constexpr int kRor8 = 0x128;  // DPP row rotate by 8
+  const uint32_t x0 = x, y0 = y;
+  y = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(y0), static_cast<int>(x0), kRor8, 0xF, 0x3, false));
+  x = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(x0), static_cast<int>(y0), kRor8, 0xF, 0xC, false));
+}
+
+template <int KIND, int NB, int IL>
+__device__ __forceinline__ void mma_tile(TileOps<NB, IL>& o, float4_t (&acc_re)[NB],
                                          float4_t (&acc_im)[NB]) {
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
+    if constexpr (IL == kLines) {
+      // every lane gets words 4 (n & 7) + 2 (n >> 3) + b of all 8 columns
+#pragma unroll
+      for (int j = 0; j < 4; ++j) swap_halves(o.w[b][j], o.w[b][4 + j]);
+    }
     const half8_t hi = pack_halves(o.w[b], kSelLo);
     half8_t res;
     if constexpr (IL) res = pack_halves(o.w[b], kSelHi);
@@ -400,7 +511,7 @@ __device__ __forceinline__ void mma_tile(const TileOps<NB, IL>& o, float4_t (&ac
 // interleaved panel, 0 for two coil blocks of separate panels or of
 // dense-control tiles, else 1 (deeper stages measured no faster and cost
 // occupancy).
-template <int KIND, int NB, bool IL>
+template <int KIND, int NB, int IL>
 struct PipeDepth {
   static constexpr int value = (IL && NB == 1 && KIND != kDenseSplit) ? 2
                                : (NB == 2 && (!IL || KIND == kDenseSplit)) ? 0
@@ -421,7 +532,7 @@ struct PipeDepth {
 // (loaded one group ahead) and resets the accumulators; with 0 (a chunk of a
 // long group) everything accumulates.  One loop for both keeps the kernel's
 // register count at that of the regular units.
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int D>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB, int D>
 __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc<NB>& r, int first, int end,
                                              int group, int group_end, uint32_t last_mask, float4_t (&acc_re)[NB],
                                              float4_t (&acc_im)[NB], int lane, const uint32_t* stage) {
@@ -435,7 +546,7 @@ __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc
   const int n = end - first;
   const int last = end - 1;
   auto tile = [&](int i) { return min(first + i, last); };
-  auto cols_of = [&](int i) { return staged_cols(stage, tile(i) - first, lane); };
+  auto cols_of = [&](int i) { return staged_cols<IL>(stage, tile(i) - first, lane); };
   last_mask = __builtin_amdgcn_readfirstlane(last_mask);
   int4 rows = load_rows(r, g, lane);
   TileCols cols[U];
@@ -447,7 +558,7 @@ __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < D; ++i) {
-    fetch_ops<KIND, NB, IL>(r, tile(i), cols[i % U], lane, ops[i % U]);
+    fetch_ops<KIND, NB, IL, WB>(r, tile(i), cols[i % U], lane, 1u + a.lines, ops[i % U]);
     __builtin_amdgcn_sched_barrier(0);
   }
   for (int base = 0; base < n; base += U) {
@@ -459,13 +570,13 @@ __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc
       // the end, so no loaded register is merged across a branch
       cols[(j + D + 1) % U] = cols_of(i + D + 1);
       __builtin_amdgcn_sched_barrier(0);
-      fetch_ops<KIND, NB, IL>(r, tile(i + D), cols[(j + D) % U], lane, ops[(j + D) % U]);
+      fetch_ops<KIND, NB, IL, WB>(r, tile(i + D), cols[(j + D) % U], lane, 1u + a.lines, ops[(j + D) % U]);
       if (i < n) {
         mma_tile<KIND, NB, IL>(ops[j], acc_re, acc_im);
         if (__builtin_amdgcn_readfirstlane(ops[j].last) & last_mask) {
+          write_group<NB, IL, OM, CONJ, ACC, WB>(a, rows, acc_re, acc_im, lane);
 #pragma unroll
           for (int b = 0; b < NB; ++b) {
-            interp_epilogue<OM, CONJ, ACC>(a, rows, b, acc_re[b], acc_im[b], lane);
             acc_re[b] = float4_t{0.f, 0.f, 0.f, 0.f};
             acc_im[b] = float4_t{0.f, 0.f, 0.f, 0.f};
           }
@@ -502,7 +613,7 @@ constexpr uint32_t kMaxSlots = (1u << 31) / (kSlotFloats * 4);
 // WB > 1 (one wave per coil block of the entry): wave wb publishes its
 // accumulators as block wb, the group's last arrival of all chunks and waves
 // adds the slots of every block; a holds the unshifted (block 0) arguments.
-template <int OM, bool CONJ, bool ACC, int NB, int WB = 1>
+template <int OM, bool CONJ, bool ACC, int NB, int IL, int WB = 1>
 __device__ __forceinline__ void chunk_finish(const InterpArgs& a, const ChunkItem& c, float4_t (&acc_re)[NB],
                                              float4_t (&acc_im)[NB], int lane, int wb = 0) {
   // slot layout: [coil block][re, im][lane][4] floats; slot offsets stay below
@@ -529,6 +640,7 @@ __device__ __forceinline__ void chunk_finish(const InterpArgs& a, const ChunkIte
   const int first = static_cast<int>(c.slot0 * kSlotFloats * 4);
   const int4 rows = group_rows_of(a, static_cast<uint32_t>(c.group), lane);
   const uint32_t n = c.n_chunks;
+  float4_t sum_re[NB * WB], sum_im[NB * WB];
 #pragma unroll
   for (int b = 0; b < NB * WB; ++b) {
     float4_t re = float4_t{0.f, 0.f, 0.f, 0.f}, im = re;
@@ -556,8 +668,10 @@ __device__ __forceinline__ void chunk_finish(const InterpArgs& a, const ChunkIte
         }
       }
     }
-    interp_epilogue<OM, CONJ, ACC>(a, rows, b, re, im, lane);
+    sum_re[b] = re;
+    sum_im[b] = im;
   }
+  write_group<NB * WB, IL, OM, CONJ, ACC, WB>(a, rows, sum_re, sum_im, lane);
 }
 
 // One wave per block, one entry of the launch order each (a regular unit, a
@@ -573,12 +687,12 @@ __device__ __forceinline__ void chunk_finish(const InterpArgs& a, const ChunkIte
 // (the arguments by value: a reference to the kernel's by-value argument
 // would make the compiler copy it to scratch and read it back through flat
 // loads)
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int WB, int D>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB, int D>
 __device__ __forceinline__ void tiles_entry(InterpArgs a) {
   static_assert(WB == 1 || NB == 1, "one wave per coil block covers one block");
   __shared__ uint32_t stages[WB][kStageWords];
   const int lane = threadIdx.x & 63;
-  const int wb = WB > 1 ? static_cast<int>(threadIdx.x >> 6) : 0;
+  const int wb = WB > 1 ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)) : 0;
   uint32_t* stage = stages[wb];
   float4_t acc_re[NB], acc_im[NB];
 #pragma unroll
@@ -600,41 +714,44 @@ __device__ __forceinline__ void tiles_entry(InterpArgs a) {
     if (a.problems) problem = glb(a.item_problem)[entry];
   }
   InterpArgs v = a;
-  if constexpr (IL) {
+  if constexpr (IL != kHalves) {
     if (a.problems) v = problem_args(a, problem);
   }
   // this wave's coil block: input panel, output coils and split-panel block
   InterpArgs vw = v;
+  uint32_t end_cut = 0;
   if constexpr (WB > 1) {
-    vw.panel_il = v.panel_il ? v.panel_il + wb * v.panel_stride : nullptr;
+    // separate blocks, or this block's half of every line row
+    vw.lines = __builtin_amdgcn_readfirstlane(v.lines);
+    end_cut = vw.lines ? wb * kN * 4 : 0;
+    vw.panel_il = v.panel_il ? v.panel_il + wb * (vw.lines ? static_cast<uint64_t>(kN) : v.panel_stride) : nullptr;
     vw.panel_hi = v.panel_hi ? v.panel_hi + wb * v.panel_stride : nullptr;
     vw.panel_res = v.panel_res ? v.panel_res + wb * v.panel_stride : nullptr;
     vw.coil_base = v.coil_base + wb * kCoilsPerBlock;
     const size_t out_block = static_cast<size_t>(wb) * v.n_out * kN;
-    vw.out_il = v.out_il ? v.out_il + out_block : nullptr;
+    vw.out_il = v.out_il ? v.out_il + (vw.lines ? static_cast<size_t>(wb) * kN : out_block) : nullptr;
     vw.out_hi = v.out_hi ? v.out_hi + out_block : nullptr;
     vw.out_res = v.out_res ? v.out_res + out_block : nullptr;
   }
   if (u.tile_begin == u.tile_end) {  // empty group: zero rows
     const int4 rows = group_rows_of(vw, static_cast<uint32_t>(u.group), lane);
-#pragma unroll
-    for (int b = 0; b < NB; ++b) interp_epilogue<OM, CONJ, ACC>(vw, rows, b, acc_re[b], acc_im[b], lane);
+    write_group<NB, IL, OM, CONJ, ACC, WB>(vw, rows, acc_re, acc_im, lane);
     return;
   }
-  const TileRsrc<NB> r = make_tile_rsrc<NB, IL>(vw);
+  const TileRsrc<NB> r = make_tile_rsrc<NB, IL, WB>(vw, end_cut);
   stage_cols(r, u.tile_begin, u.tile_end - u.tile_begin, stage, lane);
-  stream_tiles<KIND, NB, IL, OM, CONJ, ACC, D>(vw, r, u.tile_begin, u.tile_end, u.group, u.group_end,
+  stream_tiles<KIND, NB, IL, OM, CONJ, ACC, WB, D>(vw, r, u.tile_begin, u.tile_end, u.group, u.group_end,
                                                is_chunk ? 0u : 1u, acc_re, acc_im, lane, stage);
-  if (is_chunk) chunk_finish<OM, CONJ, ACC, NB, WB>(v, c, acc_re, acc_im, lane, wb);
+  if (is_chunk) chunk_finish<OM, CONJ, ACC, NB, IL, WB>(v, c, acc_re, acc_im, lane, wb);
 }
 
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int WB = 1>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB = 1>
 __global__ __launch_bounds__(64 * WB) void interp_tiles_kernel(InterpArgs a) {
   tiles_entry<KIND, NB, IL, OM, CONJ, ACC, WB, PipeDepth<KIND, NB, IL>::value>(a);
 }
 
 // The same with another pipeline depth D (the autotuner's alternatives).
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int WB, int D>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB, int D>
 __global__ __launch_bounds__(64 * WB) void interp_tiles_depth_kernel(InterpArgs a) {
   tiles_entry<KIND, NB, IL, OM, CONJ, ACC, WB, D>(a);
 }
@@ -672,9 +789,6 @@ struct CsrArgs {
 // A row of several chunks publishes one partial per chunk to a slot, and the
 // wave that counts the row's last arrival adds the slots in chunk order and
 // writes the row (the slot protocol of the packed kernel's long groups).
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
-
 template <bool CONJ>
 __device__ __forceinline__ void cmac(float2_t v, float2_t x, bool valid, float& re, float& im) {
   float pr, pi;
@@ -891,8 +1005,8 @@ constexpr uint32_t kSplitRows = 64;
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void split_panel_il_kernel(const float2* __restrict__ in, uint32_t rows,
-                                                             uint32_t coils, float scale,
-                                                             uint32_t* __restrict__ out) {
+                                                             uint32_t coils, float scale, uint32_t row_words,
+                                                             uint64_t block_words, uint32_t* __restrict__ out) {
   __shared__ float2 tile[kSplitRows][kCoilsPerBlock + 1];
   const uint32_t row0 = blockIdx.x * kSplitRows, b = blockIdx.y;
 #pragma unroll
@@ -909,7 +1023,7 @@ __global__ __launch_bounds__(256) void split_panel_il_kernel(const float2* __res
     const uint32_t r = w / kN, n = w % kN, row = row0 + r;
     if (row >= rows) continue;
     const float2 x = tile[r][n & 7];
-    out[(static_cast<size_t>(b) * rows + row) * kN + n] = split_word<BF16>((n < 8 ? x.x : x.y) * scale);
+    out[b * block_words + static_cast<size_t>(row) * row_words + n] = split_word<BF16>((n < 8 ? x.x : x.y) * scale);
   }
 }
 
@@ -946,14 +1060,14 @@ __global__ __launch_bounds__(256) void dc_residual_kernel(const float* __restric
 // plans and batches make with interleaved panels (forward into a split
 // panel, adjoint into float2 rows), one wave per entry: 1 or 3 tiles ahead
 // for one coil block, 2 for two.
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int WB>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB>
 struct AltDepths {
   static constexpr bool kPlanLaunch = IL && KIND != kDenseSplit && !ACC && WB == 1 &&
                                       ((OM == kOutRowMajor && CONJ) ||
                                        ((OM == kOutSplit16IL || OM == kOutSplitBF16IL) && !CONJ));
 };
 
-template <int KIND, int NB, bool IL, int OM, bool CONJ, bool ACC, int WB>
+template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB>
 static void launch_both(const InterpArgs& a, hipStream_t s) {
   const uint32_t blocks = a.n_chunks + a.n_items;
   if (!blocks) return;
@@ -981,7 +1095,7 @@ static void launch_both(const InterpArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((interp_tiles_kernel<KIND, NB, IL, OM, CONJ, ACC, WB>), dim3(blocks), dim3(64 * WB), 0, s, a);
 }
 
-template <int KIND, int NB, bool IL, int OM, int WB = 1>
+template <int KIND, int NB, int IL, int OM, int WB = 1>
 static void launch_tiles_om(const InterpArgs& a, bool conj, bool acc, hipStream_t s) {
   constexpr bool kAccOk = OM != kOutSplit16 && OM != kOutSplit16IL && OM != kOutSplitBF16IL;
   if (conj) {
@@ -996,7 +1110,7 @@ static void launch_tiles_om(const InterpArgs& a, bool conj, bool acc, hipStream_
 // Interleaved panels (plan-internal) pair with FP32 or interleaved split
 // output; separate panels with FP32 or separate split output (checked by
 // launch_interp).  WB = 2: two coil blocks, one wave each (NB = 1).
-template <int KIND, int NB, bool IL, int WB = 1>
+template <int KIND, int NB, int IL, int WB = 1>
 static void launch_tiles_nb(const InterpArgs& a, int om, bool conj, bool acc, hipStream_t s) {
   if constexpr (IL) {
     if (om == kOutCoilMajor) launch_tiles_om<KIND, NB, IL, kOutCoilMajor, WB>(a, conj, acc, s);
@@ -1010,37 +1124,45 @@ static void launch_tiles_nb(const InterpArgs& a, int om, bool conj, bool acc, hi
   }
 }
 
-// Interleaved panels of two coil blocks: one wave for both blocks
-// (coil_waves 1) or one wave per block (coil_waves 2).
+// Line-row panels (plans and batches of 9..16 coils), one wave for both coil
+// blocks: the launches those make (forward into a split panel or, for a plan's
+// forward operator, coil-major float2; adjoint into float2 rows).
 template <int KIND>
-static void launch_tiles_il2(const InterpArgs& a, int om, bool conj, bool acc, uint32_t coil_waves,
-                             hipStream_t s) {
-  if (coil_waves == 2) launch_tiles_nb<KIND, 1, true, 2>(a, om, conj, acc, s);
-  else launch_tiles_nb<KIND, 2, true>(a, om, conj, acc, s);
+static int launch_lines(const InterpArgs& a, int om, bool conj, bool acc, hipStream_t s) {
+  constexpr int kSplitOut = KIND == kSparseSplitBF16 ? kOutSplitBF16IL : kOutSplit16IL;
+  if (acc) return fail(TSN_ERR_ARGUMENT, "line-row panels do not accumulate");
+  if (om == kOutSplit16IL && !conj) launch_both<KIND, 2, kLines, kSplitOut, false, false, 1>(a, s);
+  else if (om == kOutRowMajor && conj) launch_both<KIND, 2, kLines, kOutRowMajor, true, false, 1>(a, s);
+  else if (om == kOutCoilMajor && !conj) launch_both<KIND, 2, kLines, kOutCoilMajor, false, false, 1>(a, s);
+  else return fail(TSN_ERR_ARGUMENT, "line-row panels do not write output mode %d here", om);
+  return TSN_OK;
 }
 
+// Two coil blocks of interleaved panels: one wave for both (coil_waves 1) or
+// one wave per block (coil_waves 2, either panel layout).
 template <int KIND>
-static void launch_tiles(const InterpArgs& a, bool il, int om, bool conj, bool acc, uint32_t coil_waves,
-                         hipStream_t s) {
+static int launch_tiles(const InterpArgs& a, int panels, int om, bool conj, bool acc, uint32_t coil_waves,
+                        hipStream_t s) {
   const bool two = a.coils > kCoilsPerBlock;
-  if constexpr (KIND == kSparseSplitBF16) {  // interleaved panels only (checked by launch_interp)
-    if (two) launch_tiles_il2<KIND>(a, om, conj, acc, coil_waves, s);
-    else launch_tiles_nb<KIND, 1, true>(a, om, conj, acc, s);
-    return;
+  if (panels == kHalves) {
+    if constexpr (KIND != kSparseSplitBF16) {  // BF16 tiles take interleaved panels (checked by launch_interp)
+      if (two) launch_tiles_nb<KIND, 2, kHalves>(a, om, conj, acc, s);
+      else launch_tiles_nb<KIND, 1, kHalves>(a, om, conj, acc, s);
+    }
+    return TSN_OK;
   }
-  if (il) {
-    if (two) launch_tiles_il2<KIND>(a, om, conj, acc, coil_waves, s);
-    else launch_tiles_nb<KIND, 1, true>(a, om, conj, acc, s);
-  } else {
-    if (two) launch_tiles_nb<KIND, 2, false>(a, om, conj, acc, s);
-    else launch_tiles_nb<KIND, 1, false>(a, om, conj, acc, s);
-  }
+  if (!two) launch_tiles_nb<KIND, 1, kBlocks>(a, om, conj, acc, s);
+  else if (coil_waves == 2) launch_tiles_nb<KIND, 1, kBlocks, 2>(a, om, conj, acc, s);
+  else if (panels == kLines) return launch_lines<KIND>(a, om, conj, acc, s);
+  else launch_tiles_nb<KIND, 2, kBlocks>(a, om, conj, acc, s);
+  return TSN_OK;
 }
 
 static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                               int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                              _Float16* out_hi, _Float16* out_res, hipStream_t stream, bool interleaved,
+                              _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
                               uint32_t* out_il, const DcTerms* dc, const ChunkScratch* scratch) {
+  const bool interleaved = panels != kHalves;
   if (!d || d->csr) return fail(TSN_ERR_ARGUMENT, "interpolation needs a packed (non-CSR) direction");
   if (coils == 0 || coils > static_cast<uint32_t>(kMaxCoils))
     return fail(TSN_ERR_ARGUMENT, "coils must be in 1..16 (got %u)", coils);
@@ -1059,6 +1181,9 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
     return fail(TSN_ERR_ARGUMENT, "tile value format of the direction does not match the interpolation variant");
   if (kind == kSparseSplitBF16 && !interleaved)
     return fail(TSN_ERR_ARGUMENT, "BF16 tiles take an interleaved split panel");
+  const bool lines = panels == kLines && coils > static_cast<uint32_t>(kCoilsPerBlock);
+  if (lines && d->h.n_cols > kMaxLineCols)
+    return fail(TSN_ERR_ARGUMENT, "line-row panels hold at most %u columns (got %u)", kMaxLineCols, d->h.n_cols);
   InterpArgs a{};
   a.items = d->items;
   a.n_items = d->n_items;
@@ -1079,9 +1204,10 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
   a.panel_hi = static_cast<const _Float16*>(hi);
   a.panel_res = static_cast<const _Float16*>(res);
   a.panel_il = static_cast<const uint32_t*>(hi);
-  a.panel_stride = static_cast<uint64_t>(d->h.n_cols) * kN;
   a.coils = coils;
   a.n_out = d->h.output_size;
+  a.panel_stride = static_cast<uint64_t>(d->h.n_cols) * kN;
+  a.lines = lines ? 1u : 0u;
   a.scale = scale;
   a.out_f32 = out_f32;
   a.out_hi = out_hi;
@@ -1098,11 +1224,12 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
   }
   a.depth = d->pipe_depth;
   const uint32_t cw = d->coil_waves;
-  if (kind == kSparseSplit) launch_tiles<kSparseSplit>(a, interleaved, out_mode, conj, accumulate, cw, stream);
-  else if (kind == kDenseSplit) launch_tiles<kDenseSplit>(a, interleaved, out_mode, conj, accumulate, cw, stream);
+  if (kind == kSparseSplit) TSN_CHECK(launch_tiles<kSparseSplit>(a, panels, out_mode, conj, accumulate, cw, stream));
+  else if (kind == kDenseSplit)
+    TSN_CHECK(launch_tiles<kDenseSplit>(a, panels, out_mode, conj, accumulate, cw, stream));
   else if (kind == kSparseSplitBF16)
-    launch_tiles<kSparseSplitBF16>(a, interleaved, out_mode, conj, accumulate, cw, stream);
-  else launch_tiles<kSparseHi>(a, interleaved, out_mode, conj, accumulate, cw, stream);
+    TSN_CHECK(launch_tiles<kSparseSplitBF16>(a, panels, out_mode, conj, accumulate, cw, stream));
+  else TSN_CHECK(launch_tiles<kSparseHi>(a, panels, out_mode, conj, accumulate, cw, stream));
   TSN_HIP(hipGetLastError());
   return TSN_OK;
 }
@@ -1111,17 +1238,17 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
 // pointers sized by the caller; panels hold ceil(coils/8) blocks.
 int launch_interp(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                   int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, bool interleaved,
+                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
                   uint32_t* out_il, const ChunkScratch* scratch) {
   return launch_interp_impl(d, kind, hi, res, coils, out_mode, conj, accumulate, scale, out_f32, out_hi, out_res,
-                            stream, interleaved, out_il, nullptr, scratch);
+                            stream, panels, out_il, nullptr, scratch);
 }
 
 int launch_interp_dc(const tsn_direction* d, int kind, const uint32_t* panel, uint32_t coils, float scale,
-                     const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch) {
+                     const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch, int panels) {
   if (!dc.y) return fail(TSN_ERR_ARGUMENT, "missing measurements");
   return launch_interp_impl(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, scale, nullptr, nullptr,
-                            nullptr, s, true, out_il, &dc, scratch);
+                            nullptr, s, panels, out_il, &dc, scratch);
 }
 
 int launch_dc_residual(const float2* pred, uint32_t rows, uint32_t coils, const DcTerms& dc, bool bf16,
@@ -1240,7 +1367,7 @@ int launch_split_panel(const float2* in, uint32_t rows, uint32_t coils, float sc
 }
 
 int launch_split_panel_il(const float2* in, uint32_t rows, uint32_t coils, float scale, uint32_t* out,
-                          hipStream_t stream, int values) {
+                          hipStream_t stream, int values, bool lines) {
   if (!in || !out || rows == 0) return fail(TSN_ERR_ARGUMENT, "bad split arguments");
   if (coils == 0 || coils > static_cast<uint32_t>(kMaxCoils))
     return fail(TSN_ERR_ARGUMENT, "coils must be in 1..16 (got %u)", coils);
@@ -1248,10 +1375,13 @@ int launch_split_panel_il(const float2* in, uint32_t rows, uint32_t coils, float
     return fail(TSN_ERR_ARGUMENT, "unknown value format %d", values);
   const uint32_t blocks = div_up(coils, kCoilsPerBlock);
   const dim3 grid(div_up(rows, kSplitRows), blocks);
+  lines = lines && blocks == 2;
+  const uint32_t rw = lines ? 2 * kN : kN;
+  const uint64_t bw = lines ? static_cast<uint64_t>(kN) : static_cast<uint64_t>(rows) * kN;
   if (values == TSN_VALUES_BF16)
-    hipLaunchKernelGGL(split_panel_il_kernel<true>, grid, dim3(256), 0, stream, in, rows, coils, scale, out);
+    hipLaunchKernelGGL(split_panel_il_kernel<true>, grid, dim3(256), 0, stream, in, rows, coils, scale, rw, bw, out);
   else
-    hipLaunchKernelGGL(split_panel_il_kernel<false>, grid, dim3(256), 0, stream, in, rows, coils, scale, out);
+    hipLaunchKernelGGL(split_panel_il_kernel<false>, grid, dim3(256), 0, stream, in, rows, coils, scale, rw, bw, out);
   TSN_HIP(hipGetLastError());
   return TSN_OK;
 }
@@ -1601,8 +1731,8 @@ static int upload_pack(const HostPack& p, tsn_direction** out) {
 
 constexpr uint32_t kMemberGroup = 8;  // default member group (batch autotuner candidate)
 
-int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* out, uint32_t member_group,
-                       uint32_t coil_waves, uint32_t depth) {
+int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* out, bool lines,
+                       uint32_t member_group, uint32_t coil_waves, uint32_t depth) {
   *out = InterpBatch{};
   if (depth > 3) return fail(TSN_ERR_ARGUMENT, "pipeline depth must be 0 (default) or 1..3");
   if (member_group == 0) member_group = kMemberGroup;
@@ -1611,6 +1741,7 @@ int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* o
   const int values = parts[0].dir->values;
   const uint32_t blocks = parts[0].blocks;
   if (blocks != 1 && blocks != 2) return fail(TSN_ERR_ARGUMENT, "a batch part covers 1 or 2 coil blocks");
+  lines = lines && blocks == 2;
   std::vector<InterpProblem> probs;
   for (const InterpBatchPart& p : parts) {
     const tsn_direction* d = p.dir;
@@ -1627,6 +1758,9 @@ int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* o
     q.n_groups = d->h.groups;
     q.n_out = d->h.output_size;
     q.n_cols = d->h.n_cols;
+    q.lines = lines ? 1u : 0u;
+    if (lines && q.n_cols > kMaxLineCols)
+      return fail(TSN_ERR_ARGUMENT, "line-row panels hold at most %u columns (got %u)", kMaxLineCols, q.n_cols);
     q.coils = p.coils;
     q.coil_base = p.coil_base;
     q.panel_il = p.panel_il;
@@ -1694,6 +1828,7 @@ int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* o
   for (const std::vector<uint32_t>& v : xcd_entries) order.insert(order.end(), v.begin(), v.end());
   InterpBatch b;
   b.blocks = blocks;
+  b.lines = lines;
   b.coil_waves = coil_waves;
   b.depth = depth;
   b.member_group = member_group;
@@ -1734,25 +1869,27 @@ void interp_batch_free(InterpBatch* b) {
   *b = InterpBatch{};
 }
 
-template <int KIND, int NB, int WB = 1>
-static void launch_batch_nb(const InterpArgs& a, int out_mode, bool conj, hipStream_t s) {
-  if (out_mode == kOutRowMajor) launch_tiles_om<KIND, NB, true, kOutRowMajor, WB>(a, conj, false, s);
-  else if (KIND == kSparseSplitBF16) launch_tiles_om<KIND, NB, true, kOutSplitBF16IL, WB>(a, conj, false, s);
-  else launch_tiles_om<KIND, NB, true, kOutSplit16IL, WB>(a, conj, false, s);
-}
-
+// One wave per entry, or (two coil blocks) one per block; entries of two
+// blocks in separate panels always take the latter.
 template <int KIND>
-static void launch_batch_kind(const InterpArgs& a, uint32_t blocks, uint32_t coil_waves, int out_mode, bool conj,
-                              hipStream_t s) {
-  if (blocks == 2 && coil_waves == 2) launch_batch_nb<KIND, 1, 2>(a, out_mode, conj, s);
-  else if (blocks == 2) launch_batch_nb<KIND, 2>(a, out_mode, conj, s);
-  else launch_batch_nb<KIND, 1>(a, out_mode, conj, s);
+static void launch_batch_kind(const InterpArgs& a, const InterpBatch& b, int out_mode, bool conj, hipStream_t s) {
+  constexpr int kSplitOut = KIND == kSparseSplitBF16 ? kOutSplitBF16IL : kOutSplit16IL;
+  if (b.blocks == 2 && (b.coil_waves == 2 || !b.lines)) {
+    if (conj) launch_both<KIND, 1, kBlocks, kOutRowMajor, true, false, 2>(a, s);
+    else launch_both<KIND, 1, kBlocks, kSplitOut, false, false, 2>(a, s);
+  } else if (b.blocks == 2) {
+    if (conj) launch_both<KIND, 2, kLines, kOutRowMajor, true, false, 1>(a, s);
+    else launch_both<KIND, 2, kLines, kSplitOut, false, false, 1>(a, s);
+  } else {
+    if (conj) launch_both<KIND, 1, kBlocks, kOutRowMajor, true, false, 1>(a, s);
+    else launch_both<KIND, 1, kBlocks, kSplitOut, false, false, 1>(a, s);
+  }
 }
 
 int launch_interp_batch(const InterpBatch& b, int kind, int out_mode, bool conj, float scale, hipStream_t s) {
   if (!b.problems) return fail(TSN_ERR_ARGUMENT, "empty interpolation batch");
-  if (out_mode != kOutRowMajor && out_mode != kOutSplit16IL)
-    return fail(TSN_ERR_ARGUMENT, "batched interpolation writes row-major float2 or split panels");
+  if (out_mode != (conj ? kOutRowMajor : kOutSplit16IL))
+    return fail(TSN_ERR_ARGUMENT, "batched interpolation writes split panels (forward) or row-major float2 (adjoint)");
   if ((kind == kSparseSplitBF16) != (b.values == TSN_VALUES_BF16))
     return fail(TSN_ERR_ARGUMENT, "tile value format of the batch does not match the interpolation variant");
   if (kind == kDenseSplit && !b.dense) return fail(TSN_ERR_ARGUMENT, "batch has no dense-control tiles");
@@ -1770,11 +1907,11 @@ int launch_interp_batch(const InterpBatch& b, int kind, int out_mode, bool conj,
   a.coils = kCoilsPerBlock;  // replaced per problem
   a.depth = b.depth;
   switch (kind) {
-    case kSparseSplit: launch_batch_kind<kSparseSplit>(a, b.blocks, b.coil_waves, out_mode, conj, s); break;
-    case kDenseSplit: launch_batch_kind<kDenseSplit>(a, b.blocks, b.coil_waves, out_mode, conj, s); break;
-    case kSparseHi: launch_batch_kind<kSparseHi>(a, b.blocks, b.coil_waves, out_mode, conj, s); break;
+    case kSparseSplit: launch_batch_kind<kSparseSplit>(a, b, out_mode, conj, s); break;
+    case kDenseSplit: launch_batch_kind<kDenseSplit>(a, b, out_mode, conj, s); break;
+    case kSparseHi: launch_batch_kind<kSparseHi>(a, b, out_mode, conj, s); break;
     case kSparseSplitBF16:
-      launch_batch_kind<kSparseSplitBF16>(a, b.blocks, b.coil_waves, out_mode, conj, s);
+      launch_batch_kind<kSparseSplitBF16>(a, b, out_mode, conj, s);
       break;
     default: return fail(TSN_ERR_ARGUMENT, "unknown interpolation kind %d", kind);
   }
@@ -1853,7 +1990,7 @@ int tsn_interp_noalloc(const tsn_direction* d, const void* hi, const void* res, 
     TSN_HIP(hipGetLastError());
   }
   return launch_interp(d, res ? kSparseSplit : kSparseHi, hi, res, coils, out_layout, conjugate != 0,
-                       accumulate != 0, scale, static_cast<float*>(out), nullptr, nullptr, s, false, nullptr,
+                       accumulate != 0, scale, static_cast<float*>(out), nullptr, nullptr, s, kHalves, nullptr,
                        d->n_chunks ? &chunk : nullptr);
 }
 
@@ -1948,7 +2085,7 @@ int tsn_direction_autotune(tsn_direction* d, uint32_t coils, void* stream, uint3
     rc = schedule_units(d, c.unit);
     auto launch = [&]() {
       return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, 1.0f, nullptr, nullptr,
-                           nullptr, s, true, out);
+                           nullptr, s, d->h.n_cols <= kMaxLineCols ? kLines : kBlocks, out);
     };
     for (int i = 0; rc == TSN_OK && i < 3; ++i) rc = launch();
     if (rc != TSN_OK) break;
@@ -2149,7 +2286,7 @@ int tsn_interp(const tsn_direction* d, const void* hi, const void* res, void* ou
     return fail(TSN_ERR_ARGUMENT, "unknown output layout %d", out_layout);
   return launch_interp(d, res ? kSparseSplit : kSparseHi, hi, res, coils, out_layout, conjugate != 0,
                        accumulate != 0, scale, static_cast<float*>(out), nullptr, nullptr,
-                       static_cast<hipStream_t>(stream), false, nullptr);
+                       static_cast<hipStream_t>(stream), kHalves, nullptr);
 }
 
 int tsn_interp_dense(const tsn_direction* d, const void* hi, const void* res, void* out,
@@ -2161,7 +2298,7 @@ int tsn_interp_dense(const tsn_direction* d, const void* hi, const void* res, vo
   TSN_CHECK(ensure_dense_tiles(d));
   return launch_interp(d, kDenseSplit, hi, res, coils, out_layout, conjugate != 0, accumulate != 0,
                        scale, static_cast<float*>(out), nullptr, nullptr,
-                       static_cast<hipStream_t>(stream), false, nullptr);
+                       static_cast<hipStream_t>(stream), kHalves, nullptr);
 }
 
 int tsn_interp_f32(const tsn_direction* d, const void* in, void* out, uint32_t coils, int conjugate,
@@ -2180,10 +2317,10 @@ int tsn_interp_il(const tsn_direction* d, const void* panel, void* out, uint32_t
   if (out_layout == TSN_OUT_SPLIT_IL) {
     if (accumulate) return fail(TSN_ERR_ARGUMENT, "a split-panel output cannot accumulate");
     return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, conjugate != 0, false, scale, nullptr,
-                         nullptr, nullptr, static_cast<hipStream_t>(stream), true, static_cast<uint32_t*>(out));
+                         nullptr, nullptr, static_cast<hipStream_t>(stream), kBlocks, static_cast<uint32_t*>(out));
   }
   return launch_interp(d, kind, panel, nullptr, coils, out_layout, conjugate != 0, accumulate != 0, scale,
-                       static_cast<float*>(out), nullptr, nullptr, static_cast<hipStream_t>(stream), true, nullptr);
+                       static_cast<float*>(out), nullptr, nullptr, static_cast<hipStream_t>(stream), kBlocks, nullptr);
 }
 
 int tsn_interp_dc(const tsn_direction* d, const void* panel, const void* measurements, int measurement_layout,
@@ -2210,14 +2347,14 @@ int tsn_interp_dc(const tsn_direction* d, const void* panel, const void* measure
   auto* out = static_cast<uint32_t*>(out_panel);
   if (mode == TSN_DC_FUSED) return launch_interp_dc(d, kind, static_cast<const uint32_t*>(panel), coils, scale, dc, out, s);
   TSN_CHECK(launch_interp(d, kind, panel, nullptr, coils, kOutRowMajor, false, false, scale,
-                          static_cast<float*>(workspace), nullptr, nullptr, s, true, nullptr));
+                          static_cast<float*>(workspace), nullptr, nullptr, s, kBlocks, nullptr));
   return launch_dc_residual(static_cast<const float2*>(workspace), rows, coils, dc, bf16, out, s);
 }
 
 int tsn_split_panel_il(const void* in, uint32_t rows, uint32_t coils, float scale, int values, void* panel,
                        void* stream) {
   return launch_split_panel_il(static_cast<const float2*>(in), rows, coils, scale,
-                               static_cast<uint32_t*>(panel), static_cast<hipStream_t>(stream), values);
+                               static_cast<uint32_t*>(panel), static_cast<hipStream_t>(stream), values, false);
 }
 
 int tsn_split_panel(const void* in, uint32_t rows, uint32_t coils, float scale, void* hi, void* res,

@@ -23,7 +23,7 @@
 
 namespace tsn {
 int launch_split_panel_il(const float2* in, uint32_t rows, uint32_t coils, float scale, uint32_t* out,
-                          hipStream_t stream, int values);
+                          hipStream_t stream, int values, bool lines);
 int launch_split_panel(const float2* in, uint32_t rows, uint32_t coils, float scale, _Float16* hi,
                        _Float16* res, hipStream_t stream);
 }  // namespace tsn
@@ -56,6 +56,7 @@ struct tsn_plan {
   double* rho = nullptr;
   uint32_t rho_cap = 0;
   int* status = nullptr;
+  int panels = kBlocks;  // layout of pan_il and smp_il: kLines for 9..16 coils (see kMaxLineCols)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -96,6 +97,7 @@ FftArgs fft_args(const tsn_plan* pl) {
   a.t_inv = pl->t_inv;
   // the packed variants' adjoint writes the grid in the FFT's chunk layout;
   // the FP32 CSR kernels gather and write [row][coils] rows
+  a.panel_lines = pl->panels == kLines ? 1u : 0u;
   a.grid_blocked = pl->cfg.precision == TSN_PREC_FP32 ? 0u : 1u;
   return a;
 }
@@ -144,10 +146,10 @@ int op_forward_samples(tsn_plan* pl, float2* out_coil_major, hipStream_t s) {
   }
   if (out_coil_major)
     return launch_interp(pl->fwd, interp_kind(pl), pl->pan_il, nullptr, pl->cfg.coils, 0, false, false, scale,
-                         reinterpret_cast<float*>(out_coil_major), nullptr, nullptr, s, true, nullptr,
+                         reinterpret_cast<float*>(out_coil_major), nullptr, nullptr, s, pl->panels, nullptr,
                          &pl->fwd_chunks);
   return launch_interp(pl->fwd, interp_kind(pl), pl->pan_il, nullptr, pl->cfg.coils, 3, false, false, scale,
-                       nullptr, nullptr, nullptr, s, true, pl->smp_il, &pl->fwd_chunks);
+                       nullptr, nullptr, nullptr, s, pl->panels, pl->smp_il, &pl->fwd_chunks);
 }
 
 // sample panels -> grid (conjugate transpose interpolation)
@@ -158,7 +160,7 @@ int op_adjoint_grid(tsn_plan* pl, hipStream_t s) {
   // row-major (mode 1) up to 8 coils, 8-coil blocks of rows (mode 5) above
   return launch_interp(pl->adj, interp_kind(pl), pl->smp_il, nullptr, pl->cfg.coils,
                        pl->cfg.coils > static_cast<uint32_t>(kCoilsPerBlock) ? 5 : 1, true, false, 1.0f, reinterpret_cast<float*>(pl->grid),
-                       nullptr, nullptr, s, true, nullptr, &pl->adj_chunks);
+                       nullptr, nullptr, s, pl->panels, nullptr, &pl->adj_chunks);
 }
 
 // grid -> image (column-major) with combine, scale, regulariser, dot partial
@@ -192,7 +194,7 @@ int op_load_samples(tsn_plan* pl, const float2* samples, float scale, hipStream_
     return TSN_OK;
   }
   return launch_split_panel_il(samples, pl->m, pl->cfg.coils, scale, pl->smp_il, s,
-                               is_bf16(pl) ? TSN_VALUES_BF16 : TSN_VALUES_FP16);
+                               is_bf16(pl) ? TSN_VALUES_BF16 : TSN_VALUES_FP16, pl->panels == kLines);
 }
 
 int transpose_image(const float2* in, uint32_t rows, uint32_t cols, float scale, float2* out, hipStream_t s) {
@@ -329,6 +331,7 @@ int tsn_plan_create(const tsn_plan_config* cfg, const tsn_direction* fwd, const 
   pl->adj = adj;
   pl->m = fwd->h.output_size;
   pl->blocks = div_up(c.coils, kCoilsPerBlock);
+  if (pl->blocks == 2 && grid <= kMaxLineCols && pl->m <= kMaxLineCols) pl->panels = kLines;
   pl->pixels = c.image0 * c.image1;
   pl->vec_blocks = div_up(pl->pixels, kVecThreads);
   const size_t px = pl->pixels;
@@ -453,7 +456,7 @@ int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measuremen
     dc.row_stride = 2 * coils;
     dc.coil_stride = 2;
     TSN_CHECK(launch_interp_dc(pl->fwd, interp_kind(pl), pl->pan_il, coils, grid_norm(pl), dc, pl->smp_il, s,
-                               &pl->fwd_chunks));
+                               &pl->fwd_chunks, pl->panels));
   }
   TSN_CHECK(op_adjoint_grid(pl, s));
   TSN_CHECK(op_adjoint_image(pl, pl->ap, nullptr, 0.0f, 1.0f, nullptr, s));

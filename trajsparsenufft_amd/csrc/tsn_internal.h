@@ -39,6 +39,20 @@ static_assert(kCsrChunkEntries <= kCsrStageEntries, "a chunk must fit the LDS st
 // Device column words of packed tiles hold column * 32 (a byte offset) below
 // bit 31, so a pack may have at most 2^26 columns.
 constexpr uint32_t kMaxDeviceCols = 1u << 26;
+// Input panels of the packed interpolation: separate FP16 hi and residual
+// panels; interleaved words hi | res << 16 in coil blocks [block][row][16]; or,
+// for two coil blocks, the same words with both blocks of a row in one 128-byte
+// line [row][32], block 0 first (plans and batches of 9..16 coils).  Why lines:
+// L2 serves 128-byte lines, so gathering the 64-byte row of each block on its
+// own moved every line twice (8.1 M L2 requests per launch at 110,839 tiles /
+// 16 coils, 5.5 M now).  Measured at 768^2 / 460,800 samples / 16 coils,
+// separate blocks -> lines: forward 96 -> 68.5 us, adjoint 90 -> 73.5 us (what
+// is left moves 5.1 TB/s past L2); eight such frames 701 -> 488 and 608 -> 500
+// us per step; 512^2 / 11 coils / spiral 30.7 -> 24.9 and 20.4 -> 19.0 us.
+enum PanelMode { kHalves = 0, kBlocks = 1, kLines = 2 };
+// Byte offsets of line rows (column * 128) are 32-bit; plans and batches with
+// more columns keep separate blocks.
+constexpr uint32_t kMaxLineCols = 1u << 25;
 // Per-tile operand offsets are signed 32-bit buffer offsets: sparse operands
 // (1 KiB per tile) hold 2^21 tiles, expanded dense-control tiles (2 KiB) 2^20.
 constexpr uint32_t kMaxDeviceTiles = 1u << 21;
@@ -194,7 +208,7 @@ struct InterpBatchPart {
   uint32_t* out_il;          // the first block's interleaved split output panel [n_out][16]
   uint32_t coils;            // coils of the problem
   uint32_t coil_base;        // first coil of the first block
-  uint32_t blocks = 1;       // coil blocks of the part (1 or 2; block 1's panels follow block 0's)
+  uint32_t blocks = 1;       // coil blocks of the part (1 or 2; block 1's panels follow block 0's or share its rows)
 };
 
 // Device tables of a batched launch: XCD x runs piece x of every direction's
@@ -210,6 +224,7 @@ struct InterpBatch {
   uint32_t* order = nullptr;     // launch order of units and chunks (kChunkTag marks a chunk)
   uint32_t n_problems = 0, n_items = 0, n_chunks = 0;
   uint32_t blocks = 1;  // coil blocks per part (every part of a batch has the same)
+  bool lines = false;   // two blocks: both panels hold 128-byte line rows
   uint32_t coil_waves = kDefaultCoilWaves;  // parts of two blocks: 1 wave for both, or 2 (one per block)
   uint32_t depth = 0;                       // tiles in flight ahead of the multiply (0: the kernel's default)
   uint32_t member_group = 0;                // parts sharing a direction that follow each entry
@@ -219,8 +234,9 @@ struct InterpBatch {
 // member_group: parts sharing a direction that follow each of its entries
 // (0 = the default, 8); coil_waves: waves per entry of two-block parts;
 // depth: tiles in flight ahead of the multiply (0 = the kernel's default).
-int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* out, uint32_t member_group = 0,
-                       uint32_t coil_waves = kDefaultCoilWaves, uint32_t depth = 0);
+// lines: the panels of parts of two coil blocks hold line rows (kLines).
+int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* out, bool lines,
+                       uint32_t member_group = 0, uint32_t coil_waves = kDefaultCoilWaves, uint32_t depth = 0);
 void interp_batch_free(InterpBatch* b);
 // kind: 0 split FP16, 1 dense control, 2 FP16 hi only, 3 split BF16; out_mode:
 // 1 row-major float2, 3 interleaved split (FP16 or BF16 as the kind).
@@ -241,11 +257,12 @@ struct ChunkScratch {
 int launch_interp_csr(const tsn_direction* d, const float2* in, uint32_t coils, int out_mode, bool conj,
                       bool accumulate, float scale, float2* out, hipStream_t stream,
                       const ChunkScratch* scratch = nullptr, bool out_prezeroed = false);
-// Packed interpolation (kind and out_mode as below); scratch null: the
-// direction's own.
+// Packed interpolation (kind and out_mode as below); panels: PanelMode of the
+// input and of an interleaved split output (kLines of up to 8 coils is
+// kBlocks); scratch null: the direction's own.
 int launch_interp(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                   int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, bool interleaved,
+                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
                   uint32_t* out_il, const ChunkScratch* scratch = nullptr);
 
 // Data-consistency terms: residual (prediction - scale * y) * w per sample
@@ -262,7 +279,8 @@ struct DcTerms {
 // its sparse operands on first use (idempotent; not for concurrent callers).
 int ensure_dense_tiles(const tsn_direction* d);
 int launch_interp_dc(const tsn_direction* d, int kind, const uint32_t* panel, uint32_t coils, float scale,
-                     const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch = nullptr);
+                     const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch = nullptr,
+                     int panels = kBlocks);
 // The same residual from stored predictions float2 [rows][coils].
 int launch_dc_residual(const float2* pred, uint32_t rows, uint32_t coils, const DcTerms& dc, bool bf16,
                        uint32_t* out_il, hipStream_t s);
