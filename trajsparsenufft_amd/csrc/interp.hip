@@ -15,9 +15,14 @@
 // over several waves and reduced deterministically; block -> item mapping
 // keeps Morton-adjacent groups on one XCD (shared L2).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <mutex>
+#include <new>
 #include <numeric>
+#include <system_error>
+#include <thread>
+#include <type_traits>
 
 #include "tsn_internal.h"
 
@@ -758,14 +763,15 @@ __global__ __launch_bounds__(64 * WB) void interp_tiles_depth_kernel(InterpArgs 
 
 
 struct CsrArgs {
-  const uint32_t* row_ptr;
+  const CsrBlock* blocks;
+  uint32_t n_blocks;
+  const CsrRound* rounds;  // rounds after the first of each block
   const int32_t* row_ids;
-  const int32_t* cols;
-  const float2* vals;
-  const CsrItem* items;
-  uint32_t n_items;
-  float2* partials;    // [slots][kMaxCoils] partial sums of long-row chunks
-  uint32_t* counters;  // one arrival counter per row of several chunks, zero between launches
+  const uint32_t* cols;    // distinct columns of each round
+  const float2* vals;      // [steps][64] entry values (see CsrBlock)
+  const uint32_t* idx;     // [ceil(steps / 4)][64] local columns, one byte a step
+  float2* partials;        // [slots][kMaxCoils] partial sums of long-row chunks
+  uint32_t* counters;      // one arrival counter per group of long rows, zero between launches
   const float2* in;
   uint32_t n_cols;
   uint32_t coils;
@@ -775,79 +781,72 @@ struct CsrArgs {
   uint32_t skip_empty;  // the output's empty rows already hold zeros: runs of empty rows write nothing
 };
 
-// Plain FP32 path.  One wave per block takes one work item: a run of at most
-// kCsrRowsPerItem consecutive short rows (each at most kCsrShortEntries
-// entries), or one chunk of a longer row (at most kCsrChunkEntries entries).
-// The item's column ids and FP32 complex coefficients are contiguous in the
-// CSR arrays; the wave copies them into LDS with coalesced loads, all issued
-// before the first wait.  LPR lanes (one coil each) then work on a row: the
-// lane groups of a run take its rows, the lane groups of a chunk stride its
-// entries and are summed in a fixed butterfly order.  Each group reads the
-// column ids of a batch of entries from LDS (one broadcast address per group),
-// issues all of the batch's gathers of input rows float2 [row][coils] and then
-// accumulates in entry order, so a row's sum never depends on the schedule.
-// A row of several chunks publishes one partial per chunk to a slot, and the
-// wave that counts the row's last arrival adds the slots in chunk order and
-// writes the row (the slot protocol of the packed kernel's long groups).
-template <bool CONJ>
-__device__ __forceinline__ void cmac(float2_t v, float2_t x, bool valid, float& re, float& im) {
-  float pr, pi;
-  if (CONJ) {
-    pr = v.x * x.x + v.y * x.y;
-    pi = v.x * x.y - v.y * x.x;
+// Plain FP32 path.  A block of four waves takes one CsrBlock: rows neighbouring
+// in k-space, in rounds of at most kCsrCols distinct input rows that their
+// entries name.  A round copies those input rows (float2 [row][coils]) into LDS
+// once and forms every product from there: neighbouring rows share most of
+// their columns, so an input row is fetched once per block instead of once per
+// entry (205,824 samples / 512^2 / 8 coils: 47 MB of gathers a launch instead
+// of 474 MB).  Four lanes (a quad) work on a row, CPL coils each; lane k of the
+// quad holds entries 4t + k, so one coalesced load brings 4 entries of 16 rows,
+// and the quad shares them by DPP broadcasts folded into the arithmetic (no LDS
+// traffic but the input rows, one 16-byte read a lane and entry at 8 coils).
+// Values and one-byte local columns stream from memory, the next four steps
+// loaded ahead.
+// Rows of up to kCsrShortEntries entries are summed in entry order.  Chunks (at
+// most kCsrChunkEntries entries) of longer rows take four quads, quad p the
+// entries p mod 4, in 16 / CPL strided partial sums combined in a fixed tree;
+// the chunks of a row publish partial sums that the last arrival adds in chunk
+// order (the slot protocol of the packed kernel's long groups).  No sum depends
+// on the schedule.
+// Measured against one lane group per row that gathered every entry from memory
+// (512^2 / 8 coils): forward 43-46 -> 21 us, adjoint
+// 59-65 -> 27.5 us, sums bit for bit the same.
+template <int CTRL>
+__device__ __forceinline__ float quad_bcast(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), CTRL, 0xF, 0xF, true));
+}
+
+template <int CPL>
+struct CsrCoils {
+  float2_t v[CPL];
+};
+
+// acc += v * x (conj(v) * x) for the CPL coils of a lane: each product rounded
+// as a multiply and a fused multiply-add, then added.
+template <int CPL, bool CONJ>
+__device__ __forceinline__ void csr_mac(float vr, float vi, const CsrCoils<CPL>& x, CsrCoils<CPL>& acc) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const float a = vi * x.v[c].y, b = vi * x.v[c].x;
+    acc.v[c].x += __builtin_fmaf(vr, x.v[c].x, CONJ ? a : -a);
+    acc.v[c].y += __builtin_fmaf(vr, x.v[c].y, CONJ ? -b : b);
+  }
+}
+
+// Entry 4t + K of the quad's row: lane K's value and local column.
+template <int CPL, bool CONJ, int K>
+__device__ __forceinline__ void csr_entry(const char* stage, float2_t val, uint32_t at, uint32_t lane_off,
+                                          CsrCoils<CPL>& acc) {
+  constexpr int kCtrl = K * 0x55;  // quad_perm [K, K, K, K]
+  const uint32_t o = quad_bcast<kCtrl>(at) + lane_off;
+  CsrCoils<CPL> x;
+  if constexpr (CPL == 1) {
+    x.v[0] = *reinterpret_cast<const float2_t*>(stage + o);
   } else {
-    pr = v.x * x.x - v.y * x.y;
-    pi = v.x * x.y + v.y * x.x;
-  }
-  re = valid ? re + pr : re;
-  im = valid ? im + pi : im;
-}
-
-// One batch: the gathers of entries e0, e0 + step, ... (B of them, those at or
-// past end masked) are all issued before the first is used; the coefficients
-// are read from LDS only when the products are formed, so a batch holds just
-// its gathered rows in registers.
-template <bool CONJ, int B>
-__device__ __forceinline__ void csr_batch(const int32_t* s_col, const float2_t* s_val, uint32_t e0, uint32_t end,
-                                          uint32_t step, rsrc_t in, uint32_t lane_off, uint32_t row_bytes,
-                                          float& re, float& im) {
-  float2_t x[B];
 #pragma unroll
-  for (int i = 0; i < B; ++i) {
-    const uint32_t e = e0 + i * step;
-    const uint32_t col = static_cast<uint32_t>(s_col[e < end ? e : e0]);
-    x[i] = __builtin_bit_cast(float2_t, __builtin_amdgcn_raw_buffer_load_b64(in, col * row_bytes + lane_off, 0, 0));
-  }
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int i = 0; i < B; ++i) {
-    const uint32_t e = e0 + i * step;
-    cmac<CONJ>(s_val[e < end ? e : e0], x[i], e < end, re, im);
-  }
-}
-
-// Entries first, first + step, ... < end of the LDS stage, in entry order:
-// batches of 24 while more than 16 remain, then of 16 or 8 (a 36-entry row:
-// 24 + 16, two memory round trips; 24 keeps the kernel at 5 waves per SIMD,
-// where 32 needed 112 registers and 4 waves, measured no faster).
-template <bool CONJ>
-__device__ __forceinline__ void csr_row_sum(const int32_t* s_col, const float2_t* s_val, uint32_t first, uint32_t end,
-                                            uint32_t step, rsrc_t in, uint32_t lane_off, uint32_t row_bytes,
-                                            float& re, float& im) {
-  uint32_t e0 = first;
-  while (e0 < end) {
-    const uint32_t left = (end - e0 + step - 1) / step;
-    if (left > 16) {
-      csr_batch<CONJ, 24>(s_col, s_val, e0, end, step, in, lane_off, row_bytes, re, im);
-      e0 += 24 * step;
-    } else if (left > 8) {
-      csr_batch<CONJ, 16>(s_col, s_val, e0, end, step, in, lane_off, row_bytes, re, im);
-      e0 += 16 * step;
-    } else {
-      csr_batch<CONJ, 8>(s_col, s_val, e0, end, step, in, lane_off, row_bytes, re, im);
-      e0 += 8 * step;
+    for (int c = 0; c < CPL; c += 2) {
+      const float4_t q = *reinterpret_cast<const float4_t*>(stage + o + c * 8);
+      x.v[c] = float2_t{q.x, q.y};
+      x.v[c + 1] = float2_t{q.z, q.w};
     }
   }
+  csr_mac<CPL, CONJ>(quad_bcast<kCtrl>(val.x), quad_bcast<kCtrl>(val.y), x, acc);
 }
 
 template <int OM, bool ACC>
@@ -861,114 +860,197 @@ __device__ __forceinline__ void csr_store(const CsrArgs& a, int32_t row, uint32_
   glb(out)[o] = v;
 }
 
-template <int LPR, int OM, bool CONJ, bool ACC>
-__global__ __launch_bounds__(64) void interp_csr_kernel(CsrArgs a) {
-  constexpr int G = 64 / LPR;  // lane groups per wave
-  __shared__ int32_t s_col[kCsrStageEntries];
-  __shared__ float2_t s_val[kCsrStageEntries];
-  const uint32_t lane = threadIdx.x;
-  const CsrItem it = a.items[xcd_remap(blockIdx.x, gridDim.x)];
-  const uint32_t n = it.e_end - it.e_begin;
-  const uint32_t g = lane / LPR, c = lane % LPR;
-  const bool active = c < a.coils;
-  const bool chunk = it.n_chunks != 0;
-  if (n == 0) {
-    // a run of empty rows (at most kCsrEmptyRunRows): zeros, unless the
-    // output holds them already or the launch accumulates; every row id is
-    // loaded before the first store
-    if (ACC || a.skip_empty) return;
-    constexpr int kPer = (kCsrEmptyRunRows + G - 1) / G;
-    int32_t orow[kPer];
+// The entries of one round of the wave's quads.  STRIDED: entry i of a quad
+// goes to sum i mod NA, else all to sum 0.
+template <int CPL, bool CONJ, bool STRIDED, int NA>
+__device__ __forceinline__ void csr_round(const float2_t* vals, const uint32_t* idx, uint32_t steps,
+                                          const char* stage, uint32_t lane_off, float2_t (&val)[4], uint32_t at,
+                                          CsrCoils<CPL> (&acc)[NA]) {
+  float2_t next_val[4];
+  uint32_t next_at = 0;
+  for (uint32_t t0 = 0; t0 < steps; t0 += 4) {
+    if (t0 + 4 < steps) {
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) orow[k] = glb(a.row_ids)[min(it.row_begin + g + k * G, it.row_end - 1)];
+      for (int i = 0; i < 4; ++i) next_val[i] = glb(vals)[static_cast<size_t>(min(t0 + 4 + i, steps - 1)) * 64];
+      next_at = glb(idx)[static_cast<size_t>(t0 / 4 + 1) * 64];
+    }
 #pragma unroll
-    for (int k = 0; k < kPer; ++k)
-      if (it.row_begin + g + k * G < it.row_end && active) csr_store<OM, false>(a, orow[k], c, 0.f, 0.f);
-    return;
-  }
-  // the group's row of a run (its first; runs hold at most G rows when LPR <= 8)
-  const uint32_t row = chunk ? it.row_begin : min(it.row_begin + g, it.row_end - 1);
-  const uint32_t rb = glb(a.row_ptr)[row], re_ = glb(a.row_ptr)[row + 1];
-  const int32_t out_row = glb(a.row_ids)[row];
-  // stage the item's entries (clamped loads, every one issued before the first wait)
-  int32_t cbuf[kCsrStageEntries / 64];
-  float2_t vbuf[kCsrStageEntries / 64];
-#pragma unroll
-  for (int i = 0; i < kCsrStageEntries / 64; ++i) {
-    const uint32_t e = it.e_begin + min(i * 64 + lane, n - 1);
-    cbuf[i] = glb(a.cols)[e];
-    vbuf[i] = glb(reinterpret_cast<const float2_t*>(a.vals))[e];
-  }
-#pragma unroll
-  for (int i = 0; i < kCsrStageEntries / 64; ++i) {
-    s_col[i * 64 + lane] = cbuf[i];
-    s_val[i * 64 + lane] = vbuf[i];
-  }
-  __syncthreads();
-  const uint32_t row_bytes = a.coils * 8;
-  const rsrc_t in = make_rsrc(a.in, static_cast<uint64_t>(a.n_cols) * row_bytes);
-  const uint32_t lane_off = (active ? c : 0) * 8;
-  float re = 0.f, im = 0.f;
-  if (!chunk) {
-    uint32_t r = it.row_begin + g, b = rb, e = re_;
-    int32_t orow = out_row;
-    while (r < it.row_end) {
-      re = 0.f;
-      im = 0.f;
-      csr_row_sum<CONJ>(s_col, s_val, b - it.e_begin, e - it.e_begin, 1, in, lane_off, row_bytes, re, im);
-      if (active) csr_store<OM, ACC>(a, orow, c, re, im);
-      r += G;
-      if (r < it.row_end) {
-        b = glb(a.row_ptr)[r];
-        e = glb(a.row_ptr)[r + 1];
-        orow = glb(a.row_ids)[r];
+    for (int i = 0; i < 4; ++i) {
+      if (t0 + i < steps) {
+        const uint32_t o = ((at >> (8 * i)) & 0xFFu) * (4 * CPL * 8);
+        csr_entry<CPL, CONJ, 0>(stage, val[i], o, lane_off, acc[0]);
+        csr_entry<CPL, CONJ, 1>(stage, val[i], o, lane_off, acc[STRIDED ? 1 % NA : 0]);
+        csr_entry<CPL, CONJ, 2>(stage, val[i], o, lane_off, acc[STRIDED ? 2 % NA : 0]);
+        csr_entry<CPL, CONJ, 3>(stage, val[i], o, lane_off, acc[STRIDED ? 3 % NA : 0]);
       }
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) val[i] = next_val[i];
+    at = next_at;
+  }
+}
+
+template <int CPL, int OM, bool CONJ, bool ACC>
+__global__ __launch_bounds__(256) void interp_csr_kernel(CsrArgs a) {
+  constexpr int kCoils = 4 * CPL;  // coils of an LDS row
+  constexpr int kSums = 4 / CPL;   // strided sums of a quad
+  __shared__ __align__(16) float2_t stage[(kCsrCols + 1) * kCoils];
+  __shared__ uint32_t last_arrival;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, l = tid & 3u, quad = tid >> 2;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const CsrBlock it = a.blocks[xcd_remap(blockIdx.x, gridDim.x)];
+  if (it.n_rounds == 0) {
+    // a run of empty rows (at most kCsrEmptyRunRows): zeros, unless the output
+    // holds them already or the launch accumulates
+    if (ACC || a.skip_empty) return;
+    for (uint32_t o = tid; o < it.n_rows * kCoils; o += 256) {
+      const uint32_t c = o % kCoils;
+      if (c < a.coils) csr_store<OM, false>(a, glb(a.row_ids)[it.row0 + o / kCoils], c, 0.f, 0.f);
+    }
     return;
   }
-  // one chunk of a long row: the groups stride the entries, then a butterfly over the groups
-  csr_row_sum<CONJ>(s_col, s_val, g, n, G, in, lane_off, row_bytes, re, im);
+  const uint32_t row_bytes = a.coils * 8;
+  const rsrc_t in = make_rsrc(a.in, static_cast<uint64_t>(a.n_cols) * row_bytes);
+  const uint32_t lane_off = l * CPL * 8;
+  CsrCoils<CPL> acc[kSums];
 #pragma unroll
-  for (int off = LPR; off < 64; off <<= 1) {
-    re += __shfl_xor(re, off);
-    im += __shfl_xor(im, off);
+  for (int k = 0; k < kSums; ++k)
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) acc[k].v[c] = float2_t{0.f, 0.f};
+  if (tid < kCoils) stage[tid] = float2_t{0.f, 0.f};  // row 0: the column of padding entries
+  CsrRound rd = it.first;
+  for (uint32_t k = 0;;) {
+    // the round's column ids, its first entries, then the rows the ids name
+    uint32_t cid[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cid[i] = glb(a.cols)[rd.col0 + min(i * 64 + quad, rd.n_cols - 1u)];
+    uint32_t ent = rd.ent0, ix = rd.idx0;
+    for (uint32_t i = 0; i < w; ++i) {
+      const uint32_t t = (rd.steps >> (8 * i)) & 0xFFu;
+      ent += t;
+      ix += (t + 3) / 4;
+    }
+    const uint32_t steps = (rd.steps >> (8 * w)) & 0xFFu;
+    const float2_t* vals = reinterpret_cast<const float2_t*>(a.vals) + static_cast<size_t>(ent) * 64 + lane;
+    const uint32_t* idx = a.idx + static_cast<size_t>(ix) * 64 + lane;
+    float2_t val[4];
+    uint32_t at = 0;
+    if (steps) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) val[i] = glb(vals)[static_cast<size_t>(min(static_cast<uint32_t>(i), steps - 1)) * 64];
+      at = glb(idx)[0];
+    }
+    // (lanes past the problem's coils read the next row or, past the end,
+    // zeros; their sums are never stored)
+    u32x4_t g[4][CPL == 4 ? 2 : 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t o = cid[i] * row_bytes + lane_off;
+      if constexpr (CPL == 1) {
+        const u32x2_t v = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(in, o, 0, 0));
+        g[i][0] = u32x4_t{v.x, v.y, 0u, 0u};
+      } else {
+#pragma unroll
+        for (int c = 0; c < CPL / 2; ++c) g[i][c] = __builtin_amdgcn_raw_buffer_load_b128(in, o + c * 16, 0, 0);
+      }
+    }
+    if (k) __syncthreads();  // every wave is done with the last round's stage
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t r = i * 64 + quad;
+      if (r >= rd.n_cols) continue;
+      float2_t* to = stage + (r + 1) * kCoils + l * CPL;
+      if constexpr (CPL == 1) {
+        *to = __builtin_bit_cast(float2_t, u32x2_t{g[i][0].x, g[i][0].y});
+      } else {
+#pragma unroll
+        for (int c = 0; c < CPL / 2; ++c) reinterpret_cast<u32x4_t*>(to)[c] = g[i][c];
+      }
+    }
+    __syncthreads();
+    const char* base = reinterpret_cast<const char*>(stage);
+    if (it.n_chunks == 0) csr_round<CPL, CONJ, false, kSums>(vals, idx, steps, base, lane_off, val, at, acc);
+    else csr_round<CPL, CONJ, true, kSums>(vals, idx, steps, base, lane_off, val, at, acc);
+    if (++k == it.n_rounds) break;
+    rd = a.rounds[it.round0 + k - 1];
   }
+  if (it.n_chunks == 0) {  // quad q is row q
+    if (quad >= it.n_rows) return;
+    const int32_t row = glb(a.row_ids)[it.row0 + quad];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c)
+      if (l * CPL + c < a.coils) csr_store<OM, ACC>(a, row, l * CPL + c, acc[0].v[c].x, acc[0].v[c].y);
+    return;
+  }
+  // four quads a row: strided sum 4 a + p of quad p, added pairwise over p,
+  // then over a
+  CsrCoils<CPL> sum;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) {
+#pragma unroll
+      for (int off = 4; off < 16; off <<= 1) {
+        acc[k].v[c].x += __shfl_xor(acc[k].v[c].x, off);
+        acc[k].v[c].y += __shfl_xor(acc[k].v[c].y, off);
+      }
+    }
+    if constexpr (kSums == 4) sum.v[c] = (acc[0].v[c] + acc[1].v[c]) + (acc[2].v[c] + acc[3].v[c]);
+    else if constexpr (kSums == 2) sum.v[c] = acc[0].v[c] + acc[1].v[c];
+    else sum.v[c] = acc[0].v[c];
+  }
+  const uint32_t r = tid >> 4;
+  const bool owner = (quad & 3u) == 0 && r < it.n_rows;
   if (it.n_chunks == 1) {
-    if (g == 0 && active) csr_store<OM, ACC>(a, out_row, c, re, im);
+    if (!owner) return;
+    const int32_t row = glb(a.row_ids)[it.row0 + r];
+#pragma unroll
+    for (int c = 0; c < CPL; ++c)
+      if (l * CPL + c < a.coils) csr_store<OM, ACC>(a, row, l * CPL + c, sum.v[c].x, sum.v[c].y);
     return;
   }
+  // one chunk of the rows: publish, count, and the last arrival adds the
+  // chunks' slots in chunk order
   const rsrc_t slots = make_rsrc(a.partials, uint64_t{1} << 32);
-  if (g == 0 && active)
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, float2_t{re, im}), slots, c * 8,
-                                          static_cast<int>((it.slot0 + it.chunk) * kMaxCoils * 8), kCpolDevice);
-  __builtin_amdgcn_s_waitcnt(0);  // the slot stores acknowledged
-  asm volatile("" ::: "memory");
-  uint32_t arrived = 0;
-  if (lane == 0)
-    arrived = __hip_atomic_fetch_add(a.counters + it.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  arrived = __builtin_amdgcn_readfirstlane(arrived);
-  if (arrived + 1 != it.n_chunks) return;
-  asm volatile("" ::: "memory");
-  if (lane == 0) __hip_atomic_store(a.counters + it.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (g != 0 || !active) return;
-  float sr = 0.f, si = 0.f;
-  for (uint32_t q0 = 0; q0 < it.n_chunks; q0 += kSlotBatch) {
-    float2_t p[kSlotBatch];
+  if (owner) {
 #pragma unroll
-    for (uint32_t j = 0; j < kSlotBatch; ++j) {
-      const uint32_t q = min(q0 + j, it.n_chunks - 1);
-      p[j] = __builtin_bit_cast(float2_t, __builtin_amdgcn_raw_buffer_load_b64(
-                                            slots, c * 8, static_cast<int>((it.slot0 + q) * kMaxCoils * 8),
-                                            kCpolDevice));
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kSlotBatch; ++j) {
-      if (q0 + j >= it.n_chunks) break;
-      sr += p[j].x;
-      si += p[j].y;
-    }
+    for (int c = 0; c < CPL; ++c)
+      if (l * CPL + c < a.coils)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, sum.v[c]), slots,
+                                              (it.slot0 + it.chunk * it.n_rows + r) * (kMaxCoils * 8) +
+                                                  (l * CPL + c) * 8,
+                                              0, kCpolDevice);
   }
-  csr_store<OM, ACC>(a, out_row, c, sr, si);
+  __builtin_amdgcn_s_waitcnt(0);  // the wave's slot stores acknowledged
+  __syncthreads();
+  if (tid == 0)
+    last_arrival = __hip_atomic_fetch_add(a.counters + it.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
+                           it.n_chunks
+                       ? 1u
+                       : 0u;
+  __syncthreads();
+  if (!last_arrival) return;
+  asm volatile("" ::: "memory");
+  if (tid == 0) __hip_atomic_store(a.counters + it.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (uint32_t o = tid; o < it.n_rows * kCoils; o += 256) {
+    const uint32_t row = o / kCoils, c = o % kCoils;
+    if (c >= a.coils) continue;
+    float2_t v = float2_t{0.f, 0.f};
+    for (uint32_t q0 = 0; q0 < it.n_chunks; q0 += kSlotBatch) {
+      float2_t p[kSlotBatch];
+#pragma unroll
+      for (uint32_t j = 0; j < kSlotBatch; ++j)
+        p[j] = __builtin_bit_cast(
+            float2_t,
+            __builtin_amdgcn_raw_buffer_load_b64(
+                slots, (it.slot0 + min(q0 + j, it.n_chunks - 1u) * it.n_rows + row) * (kMaxCoils * 8) + c * 8, 0,
+                kCpolDevice));
+#pragma unroll
+      for (uint32_t j = 0; j < kSlotBatch; ++j)
+        if (q0 + j < it.n_chunks) v += p[j];
+    }
+    csr_store<OM, ACC>(a, glb(a.row_ids)[it.row0 + row], c, v.x, v.y);
+  }
 }
 
 // hi = RN16(v), res = RN16(v - hi), v = in * scale; in float2 [coil][rows];
@@ -1297,10 +1379,10 @@ int launch_dc_residual_rows(float2* rows_io, uint32_t rows, uint32_t coils, cons
   return TSN_OK;
 }
 
-template <int LPR, int OM>
+template <int CPL, int OM>
 static void launch_csr_om(const CsrArgs& a, bool conj, bool acc, hipStream_t s) {
 #define TSN_CSR(C, A) \
-  hipLaunchKernelGGL((interp_csr_kernel<LPR, OM, C, A>), dim3(a.n_items), dim3(64), 0, s, a)
+  hipLaunchKernelGGL((interp_csr_kernel<CPL, OM, C, A>), dim3(a.n_blocks), dim3(256), 0, s, a)
   if (conj) {
     if (acc) TSN_CSR(true, true); else TSN_CSR(true, false);
   } else {
@@ -1309,10 +1391,10 @@ static void launch_csr_om(const CsrArgs& a, bool conj, bool acc, hipStream_t s) 
 #undef TSN_CSR
 }
 
-template <int LPR>
-static void launch_csr_lpr(const CsrArgs& a, int om, bool conj, bool acc, hipStream_t s) {
-  if (om == kOutCoilMajor) launch_csr_om<LPR, kOutCoilMajor>(a, conj, acc, s);
-  else launch_csr_om<LPR, kOutRowMajor>(a, conj, acc, s);
+template <int CPL>
+static void launch_csr_cpl(const CsrArgs& a, int om, bool conj, bool acc, hipStream_t s) {
+  if (om == kOutCoilMajor) launch_csr_om<CPL, kOutCoilMajor>(a, conj, acc, s);
+  else launch_csr_om<CPL, kOutRowMajor>(a, conj, acc, s);
 }
 
 int launch_interp_csr(const tsn_direction* d, const float2* in, uint32_t coils, int out_mode,
@@ -1328,12 +1410,13 @@ int launch_interp_csr(const tsn_direction* d, const float2* in, uint32_t coils, 
   if (static_cast<uint64_t>(d->h.n_cols) * coils * 8 >= (uint64_t{1} << 32))
     return fail(TSN_ERR_ARGUMENT, "FP32 input of %u rows x %u coils exceeds 4 GiB", d->h.n_cols, coils);
   CsrArgs a{};
-  a.row_ptr = d->row_ptr;
+  a.blocks = d->csr_blocks;
+  a.n_blocks = d->n_csr_blocks;
   a.row_ids = d->row_ids;
-  a.cols = d->cols;
+  a.cols = d->csr_cols;
   a.vals = d->vals;
-  a.items = d->csr_items;
-  a.n_items = d->n_csr_items;
+  a.idx = d->csr_idx;
+  a.rounds = d->csr_rounds;
   a.partials = reinterpret_cast<float2*>(scratch ? scratch->partials : d->partials);
   a.counters = scratch ? scratch->counters : d->counters;
   if (d->n_slots && (!a.partials || !a.counters)) return fail(TSN_ERR_ARGUMENT, "missing chunk scratch");
@@ -1344,11 +1427,11 @@ int launch_interp_csr(const tsn_direction* d, const float2* in, uint32_t coils, 
   a.scale = scale;
   a.out = out;
   a.skip_empty = out_prezeroed ? 1u : 0u;
-  if (out_prezeroed || accumulate) a.n_items = d->n_csr_active_items;  // the trailing empty runs write nothing
-  if (a.n_items == 0) return TSN_OK;
-  if (coils <= 4) launch_csr_lpr<4>(a, out_mode, conj, accumulate, stream);
-  else if (coils <= 8) launch_csr_lpr<8>(a, out_mode, conj, accumulate, stream);
-  else launch_csr_lpr<16>(a, out_mode, conj, accumulate, stream);
+  if (out_prezeroed || accumulate) a.n_blocks = d->n_csr_active_blocks;  // the trailing empty runs write nothing
+  if (a.n_blocks == 0) return TSN_OK;
+  if (coils <= 4) launch_csr_cpl<1>(a, out_mode, conj, accumulate, stream);
+  else if (coils <= 8) launch_csr_cpl<2>(a, out_mode, conj, accumulate, stream);
+  else launch_csr_cpl<4>(a, out_mode, conj, accumulate, stream);
   TSN_HIP(hipGetLastError());
   return TSN_OK;
 }
@@ -1401,8 +1484,8 @@ static int device_copy(const T* host, size_t count, T** out, size_t* bytes) {
 static void release(tsn_direction* d) {
   if (!d) return;
   void* ptrs[] = {d->group_offsets, d->group_rows, d->tile_cols, d->tile_a, d->tile_idx,
-                  d->tile_dense, d->items, d->order, d->chunks, d->partials, d->counters, d->row_ptr, d->row_ids,
-                  d->cols, d->vals, d->csr_items};
+                  d->tile_dense, d->items, d->order, d->chunks, d->partials, d->counters, d->row_ids,
+                  d->csr_cols, d->vals, d->csr_idx, d->csr_rounds, d->csr_blocks};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (void* p : d->retired) (void)hipFree(p);
@@ -1526,45 +1609,241 @@ static int schedule_units(tsn_direction* d, uint32_t unit_tiles) {
 
 }  // namespace tsn
 
-// Work items of a CSR direction in row order: runs of consecutive rows of at
-// most kCsrShortEntries entries (at most kCsrRowsPerItem rows each), and each
-// longer row cut into ceil(entries / kCsrChunkEntries) chunks of equal size
-// (within one entry); a row of several chunks takes that many partial slots
-// and one arrival counter.  Empty rows form runs of their own (at most
-// kCsrEmptyRunRows rows) unless they follow a short row in a run.
-std::vector<tsn::CsrItem> tsn::csr_items(const std::vector<uint32_t>& ptr, uint32_t* slots, uint32_t* counters) {
-  std::vector<CsrItem> items;
-  *slots = 0;
-  *counters = 0;
-  const uint32_t rows = static_cast<uint32_t>(ptr.size()) - 1;
-  uint32_t t = 0;
-  while (t < rows) {
-    const uint32_t len = ptr[t + 1] - ptr[t];
-    if (len > static_cast<uint32_t>(kCsrShortEntries)) {
-      const uint32_t n = div_up(len, kCsrChunkEntries);
-      const uint32_t slot0 = n > 1 ? *slots : 0, counter = n > 1 ? *counters : 0;
-      if (n > 1) {
-        *slots += n;
-        *counters += 1;
-      }
-      for (uint32_t c = 0; c < n; ++c)
-        items.push_back(CsrItem{t, t + 1, ptr[t] + static_cast<uint32_t>(static_cast<uint64_t>(len) * c / n),
-                                ptr[t] + static_cast<uint32_t>(static_cast<uint64_t>(len) * (c + 1) / n), c, n,
-                                slot0, counter});
-      ++t;
-      continue;
-    }
-    const uint32_t start = t;
-    if (len == 0) {  // a run of empty rows
-      while (t < rows && t - start < static_cast<uint32_t>(kCsrEmptyRunRows) && ptr[t + 1] == ptr[t]) ++t;
-    } else {  // empty rows after the first stay in the run (cheap there)
-      while (t < rows && t - start < static_cast<uint32_t>(kCsrRowsPerItem) &&
-             ptr[t + 1] - ptr[t] <= static_cast<uint32_t>(kCsrShortEntries))
-        ++t;
-    }
-    items.push_back(CsrItem{start, t, ptr[start], ptr[t], 0, 0, 0, 0});
+namespace {
+
+// One lane quad of an FP32 block: entries base + stride i, i < count.
+struct CsrQuad {
+  uint32_t base, stride, count;
+};
+
+// Builds the blocks of one range of a direction's rows (csr_build).
+struct CsrBuilder {
+  const std::vector<uint32_t>& ptr;
+  const std::vector<int32_t>& cols;
+  const std::vector<float2>& vals;
+  const std::vector<int32_t>& rows;
+  tsn::CsrHost h;
+  std::vector<uint32_t> mark, place;  // group that last named a column; its index in uniq
+  std::vector<uint32_t> uniq;
+  uint32_t group = 0;
+
+  // The distinct columns of entries [b, e) that the group has not named yet.
+  uint32_t fresh(uint32_t b, uint32_t e) const {
+    uint32_t n = 0;
+    for (uint32_t k = b; k < e; ++k) n += mark[cols[k]] != group;
+    return n;
   }
-  return items;
+  void name(uint32_t b, uint32_t e) {
+    for (uint32_t k = b; k < e; ++k)
+      if (mark[cols[k]] != group) {
+        mark[cols[k]] = group;
+        uniq.push_back(static_cast<uint32_t>(cols[k]));
+      }
+  }
+
+  // One block of the quads (16 to a wave), whose entries name the columns uniq.
+  void emit(tsn::CsrBlock b, const CsrQuad* quads, uint32_t n_quads) {
+    std::sort(uniq.begin(), uniq.end());
+    const uint32_t u = static_cast<uint32_t>(uniq.size());
+    for (uint32_t i = 0; i < u; ++i) place[uniq[i]] = i;
+    b.n_rounds = tsn::div_up(u, tsn::kCsrCols);
+    b.round0 = static_cast<uint32_t>(h.rounds.size());
+    uint32_t at[64] = {};
+    for (uint32_t k = 0; k < b.n_rounds; ++k) {
+      const uint32_t u0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * k / b.n_rounds);
+      const uint32_t u1 = static_cast<uint32_t>(static_cast<uint64_t>(u) * (k + 1) / b.n_rounds);
+      tsn::CsrRound rd{};
+      rd.col0 = static_cast<uint32_t>(h.cols.size());
+      rd.n_cols = u1 - u0;
+      h.cols.insert(h.cols.end(), uniq.begin() + u0, uniq.begin() + u1);
+      rd.ent0 = static_cast<uint32_t>(h.vals.size() / 64);
+      rd.idx0 = static_cast<uint32_t>(h.idx.size() / 64);
+      for (uint32_t w = 0; w < 4; ++w) {
+        const uint32_t q0 = 16 * w, q1 = std::min(n_quads, q0 + 16);
+        // entry i of a quad sits at step i / 4 - at / 4, lane i mod 4 of the quad
+        uint32_t end[16] = {}, n = 0;
+        for (uint32_t q = q0; q < q1; ++q) {
+          const CsrQuad& qd = quads[q];
+          uint32_t i = at[q];
+          if (u1 == u) i = qd.count;
+          else
+            while (i < qd.count && place[cols[qd.base + qd.stride * i]] < u1) ++i;
+          end[q - q0] = i;
+          if (i > at[q]) n = std::max(n, (i - 1) / 4 - at[q] / 4 + 1);
+        }
+        rd.steps |= n << (8 * w);
+        const size_t v0 = h.vals.size(), i0 = h.idx.size();
+        h.vals.resize(v0 + static_cast<size_t>(n) * 64, make_float2(0.f, 0.f));
+        h.idx.resize(i0 + static_cast<size_t>(tsn::div_up(n, 4)) * 64, 0u);
+        for (uint32_t q = q0; q < q1; ++q) {
+          const CsrQuad& qd = quads[q];
+          const uint32_t first = at[q] / 4;
+          for (uint32_t i = at[q]; i < end[q - q0]; ++i) {
+            const uint32_t e = qd.base + qd.stride * i, t = i / 4 - first, lane = (q - q0) * 4 + (i & 3u);
+            h.vals[v0 + static_cast<size_t>(t) * 64 + lane] = vals[e];
+            h.idx[i0 + static_cast<size_t>(t / 4) * 64 + lane] |= (place[cols[e]] - u0 + 1) << (8 * (t & 3u));
+          }
+          at[q] = end[q - q0];
+        }
+      }
+      if (k == 0) b.first = rd;
+      else h.rounds.push_back(rd);
+    }
+    h.blocks.push_back(b);
+    uniq.clear();
+    ++group;
+  }
+
+  uint32_t length(uint32_t t) const { return ptr[t + 1] - ptr[t]; }
+
+  // The rows of perm[lo .. hi): long rows and short rows each form groups of
+  // consecutive rows, the long ones (blocks of several rounds) first.
+  void build(const std::vector<uint32_t>& perm, uint32_t lo, uint32_t hi) {
+    std::vector<uint32_t> small, large;
+    CsrQuad quads[64];
+    auto flush_small = [&]() {
+      if (small.empty()) return;
+      // longest first, so that the 16 rows of a wave are of similar length
+      std::stable_sort(small.begin(), small.end(), [&](uint32_t p, uint32_t q) { return length(p) > length(q); });
+      tsn::CsrBlock b{};
+      b.row0 = static_cast<uint32_t>(h.row_ids.size());
+      b.n_rows = static_cast<uint32_t>(small.size());
+      for (uint32_t r = 0; r < b.n_rows; ++r) {
+        h.row_ids.push_back(rows[small[r]]);
+        quads[r] = {ptr[small[r]], 1, length(small[r])};
+      }
+      emit(b, quads, b.n_rows);
+      small.clear();
+    };
+    auto flush_large = [&]() {
+      if (large.empty()) return;
+      tsn::CsrBlock b{};
+      b.row0 = static_cast<uint32_t>(h.row_ids.size());
+      b.n_rows = static_cast<uint32_t>(large.size());
+      b.n_chunks = tsn::div_up(length(large[0]), tsn::kCsrChunkEntries);
+      if (b.n_chunks > 1) {
+        b.slot0 = h.slots;
+        b.counter = h.counters;
+        h.slots += b.n_chunks * b.n_rows;
+        h.counters += 1;
+      }
+      for (uint32_t t : large) h.row_ids.push_back(rows[t]);
+      for (uint32_t c = 0; c < b.n_chunks; ++c) {
+        b.chunk = c;
+        for (uint32_t r = 0; r < b.n_rows; ++r) {
+          const uint32_t n = length(large[r]), t = ptr[large[r]];
+          const uint32_t e0 = t + static_cast<uint32_t>(static_cast<uint64_t>(n) * c / b.n_chunks);
+          const uint32_t e1 = t + static_cast<uint32_t>(static_cast<uint64_t>(n) * (c + 1) / b.n_chunks);
+          name(e0, e1);
+          for (uint32_t p = 0; p < 4; ++p) quads[4 * r + p] = {e0 + p, 4, (e1 - e0 + 3 - p) / 4};
+        }
+        emit(b, quads, 4 * b.n_rows);
+      }
+      large.clear();
+    };
+    for (uint32_t i = lo; i < hi; ++i) {
+      const uint32_t t = perm[i], n = length(t);
+      if (n <= tsn::kCsrShortEntries) continue;
+      if (large.size() == 16 || (!large.empty() && tsn::div_up(n, tsn::kCsrChunkEntries) !=
+                                                       tsn::div_up(length(large[0]), tsn::kCsrChunkEntries)))
+        flush_large();
+      large.push_back(t);
+    }
+    flush_large();
+    for (uint32_t i = lo; i < hi; ++i) {
+      const uint32_t t = perm[i], n = length(t);
+      if (n > tsn::kCsrShortEntries) continue;
+      if (small.size() == 64 || uniq.size() + fresh(ptr[t], ptr[t + 1]) > tsn::kCsrCols) flush_small();
+      name(ptr[t], ptr[t + 1]);
+      small.push_back(t);
+    }
+    flush_small();
+  }
+};
+
+}  // namespace
+
+// Launch order of an FP32 direction's blocks: XCD x runs the x-th of eight equal
+// ranges (xcd_remap), so the blocks are cut into eight contiguous runs of equal
+// work (steps, and a round's start counted as kCsrRoundSteps), each run's long
+// rows go first (blocks of several rounds last the longest), and shorter runs
+// are filled up with blocks of no rows.  512^2 / 8 coils adjoint: 30.1 -> 27.6 us
+// against equal block counts.
+static void csr_balance(std::vector<tsn::CsrBlock>* blocks, const std::vector<tsn::CsrRound>& rounds) {
+  constexpr uint32_t kCsrRoundSteps = 6;
+  auto longest = [](const tsn::CsrRound& r) {
+    uint32_t n = 0;
+    for (uint32_t w = 0; w < 4; ++w) n = std::max(n, (r.steps >> (8 * w)) & 0xFFu);
+    return n + kCsrRoundSteps;
+  };
+  auto work = [&](const tsn::CsrBlock& b) {
+    uint64_t n = longest(b.first);
+    for (uint32_t k = 1; k < b.n_rounds; ++k) n += longest(rounds[b.round0 + k - 1]);
+    return n;
+  };
+  uint64_t total = 0, done = 0;
+  for (const tsn::CsrBlock& b : *blocks) total += work(b);
+  std::vector<tsn::CsrBlock> runs[8];
+  for (const tsn::CsrBlock& b : *blocks) {
+    const uint64_t w = work(b);
+    runs[std::min<uint64_t>(7, (2 * done + w) * 4 / std::max<uint64_t>(total, 1))].push_back(b);
+    done += w;
+  }
+  size_t most = 0;
+  for (auto& r : runs) {
+    std::stable_partition(r.begin(), r.end(), [](const tsn::CsrBlock& b) { return b.n_chunks != 0; });
+    most = std::max(most, r.size());
+  }
+  blocks->clear();
+  for (auto& r : runs) {
+    r.resize(most, tsn::CsrBlock{});
+    blocks->insert(blocks->end(), r.begin(), r.end());
+  }
+}
+
+// Blocks of an FP32 direction.  Rows in the order `perm` (entries of row t:
+// ptr[t] .. ptr[t + 1] of cols and vals, ascending columns), cut into
+// up to kCsrParts ranges built side by side (false: out of memory).  In a range, short rows form groups of
+// up to 64 rows naming at most kCsrCols distinct columns (one round), long rows
+// groups of up to 16 rows of equally many chunks, one block per chunk.
+bool tsn::csr_build(const std::vector<uint32_t>& ptr, const std::vector<int32_t>& cols,
+                    const std::vector<float2>& vals, const std::vector<int32_t>& rows,
+                    const std::vector<uint32_t>& perm, uint32_t n_cols, std::vector<CsrHost>* out) {
+  const uint32_t n = static_cast<uint32_t>(perm.size());
+  // a range holds at least kCsrPartEntries entries: smaller ones cost more in
+  // groups cut short at their ends and in threads than they save
+  const uint32_t parts = static_cast<uint32_t>(
+      std::clamp<size_t>(cols.size() / kCsrPartEntries, 1, kCsrParts));
+  out->assign(parts, CsrHost{});
+  std::atomic<uint32_t> next{0};
+  std::atomic<bool> done{true};
+  auto work = [&]() {
+    try {
+      std::vector<uint32_t> mark(n_cols, 0xFFFFFFFFu), place(n_cols, 0u);
+      uint32_t group = 0;
+      for (uint32_t k; (k = next++) < parts;) {
+        CsrBuilder b{ptr, cols, vals, rows, {}, std::move(mark), std::move(place), {}, group};
+        b.build(perm, static_cast<uint32_t>(static_cast<uint64_t>(n) * k / parts),
+                static_cast<uint32_t>(static_cast<uint64_t>(n) * (k + 1) / parts));
+        (*out)[k] = std::move(b.h);
+        mark = std::move(b.mark);
+        place = std::move(b.place);
+        group = b.group;
+      }
+    } catch (const std::bad_alloc&) {
+      done = false;
+    }
+  };
+  const uint32_t threads = std::clamp(std::thread::hardware_concurrency(), 1u, parts);
+  std::vector<std::thread> pool;
+  try {
+    for (uint32_t i = 1; i < threads; ++i) pool.emplace_back(work);
+  } catch (const std::system_error&) {
+    // fewer helpers
+  }
+  work();
+  for (std::thread& t : pool) t.join();
+  return done;
 }
 
 std::vector<tsn::ChunkItem> tsn::long_chunks(const std::vector<uint32_t>& off, uint32_t problem, uint32_t slot_base,
@@ -2184,9 +2463,10 @@ int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** 
     h.active_rows = static_cast<uint32_t>(rows.size());
   }
   // Rows in Morton order of their k-space position (samples: the rounded grid
-  // coordinate; grid points: their own), so the contiguous range of work
-  // items each XCD runs covers a compact k-space region and its gathers stay
-  // in that XCD's L2.  Entries keep their order, so the sums do not change.
+  // coordinate; grid points: their own): a block's rows share columns, and the
+  // contiguous range of blocks each XCD runs covers a compact k-space region
+  // whose input rows stay in that XCD's L2.
+  std::vector<uint32_t> perm;
   {
     const uint32_t n = static_cast<uint32_t>(rows.size());
     std::vector<uint32_t> key(n);
@@ -2199,63 +2479,99 @@ int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** 
         key[t] = morton_key(g % kb->grid1, g / kb->grid1);
       }
     }
-    std::vector<uint32_t> perm(n);
+    perm.resize(n);
     std::iota(perm.begin(), perm.end(), 0u);
     std::stable_sort(perm.begin(), perm.end(), [&](uint32_t a, uint32_t b) { return key[a] < key[b]; });
-    std::vector<uint32_t> nptr(1, 0);
-    std::vector<int32_t> nrows(n), ncols(cols.size());
-    std::vector<float2> nvals(vals.size());
-    nptr.reserve(n + 1);
-    for (uint32_t i = 0; i < n; ++i) {
-      const uint32_t t = perm[i];
-      nrows[i] = rows[t];
-      const uint32_t b = ptr[t], e = ptr[t + 1], o = nptr.back();
-      std::copy(cols.begin() + b, cols.begin() + e, ncols.begin() + o);
-      std::copy(vals.begin() + b, vals.begin() + e, nvals.begin() + o);
-      nptr.push_back(o + (e - b));
-    }
-    ptr.swap(nptr);
-    rows.swap(nrows);
-    cols.swap(ncols);
-    vals.swap(nvals);
   }
+  std::vector<CsrHost> parts;
+  if (!csr_build(ptr, cols, vals, rows, perm, h.n_cols, &parts))
+    return fail(TSN_ERR_RUNTIME, "out of host memory");
+  // the parts one after the other: every block's offsets move by what precedes it
+  CsrHost host;  // blocks, rounds, row ids and columns of all parts; values and local columns stay in parts
+  uint32_t steps = 0, words = 0;
+  for (const CsrHost& q : parts) {
+    auto moved = [&](CsrRound r) {
+      r.col0 += static_cast<uint32_t>(host.cols.size());
+      r.ent0 += steps;
+      r.idx0 += words;
+      return r;
+    };
+    std::vector<CsrRound> more;
+    for (const CsrRound& r : q.rounds) more.push_back(moved(r));
+    for (CsrBlock b : q.blocks) {
+      b.first = moved(b.first);
+      b.round0 += static_cast<uint32_t>(host.rounds.size());
+      b.row0 += static_cast<uint32_t>(host.row_ids.size());
+      b.slot0 += host.slots;
+      b.counter += host.counters;
+      host.blocks.push_back(b);
+    }
+    host.rounds.insert(host.rounds.end(), more.begin(), more.end());
+    host.cols.insert(host.cols.end(), q.cols.begin(), q.cols.end());
+    host.row_ids.insert(host.row_ids.end(), q.row_ids.begin(), q.row_ids.end());
+    steps += static_cast<uint32_t>(q.vals.size() / 64);
+    words += static_cast<uint32_t>(q.idx.size() / 64);
+    host.slots += q.slots;
+    host.counters += q.counters;
+  }
+  csr_balance(&host.blocks, host.rounds);
+  const uint32_t active_blocks = static_cast<uint32_t>(host.blocks.size());
   // Output rows no entry reaches (grid points of the transpose no sample
-  // touches) follow as empty CSR rows in ascending order, so a launch that
-  // does not accumulate writes zeros there too (runs of empty rows).  Their
-  // items come last; a launch into an output already zero leaves them out.
-  const uint32_t active = static_cast<uint32_t>(rows.size());
-  if (active < h.output_size) {
+  // touches) follow as runs of empty rows in ascending order, so a launch that
+  // does not accumulate writes zeros there too; a launch into an output
+  // already zero leaves them out.
+  if (rows.size() < h.output_size) {
     std::vector<uint8_t> hit(h.output_size, 0);
     for (int32_t r : rows) hit[r] = 1;
-    for (uint32_t r = 0; r < h.output_size; ++r)
-      if (!hit[r]) {
-        rows.push_back(static_cast<int32_t>(r));
-        ptr.push_back(ptr.back());
+    for (uint32_t r = 0; r < h.output_size; ++r) {
+      if (hit[r]) continue;
+      if (host.blocks.size() == active_blocks || host.blocks.back().n_rows == kCsrEmptyRunRows) {
+        CsrBlock b{};
+        b.row0 = static_cast<uint32_t>(host.row_ids.size());
+        host.blocks.push_back(b);
       }
+      host.blocks.back().n_rows += 1;
+      host.row_ids.push_back(static_cast<int32_t>(r));
+    }
   }
-  uint32_t slots = 0, counters = 0;
-  const std::vector<CsrItem> items = csr_items(ptr, &slots, &counters);
-  uint32_t active_items = 0;  // items holding an active row: all but the trailing runs of empty rows
-  while (active_items < items.size() && items[active_items].row_begin < active) ++active_items;
-  if (slots > kMaxCsrSlots) return fail(TSN_ERR_ARGUMENT, "%u long-row chunks (at most %u)", slots, kMaxCsrSlots);
+  if (host.slots > kMaxCsrSlots)
+    return fail(TSN_ERR_ARGUMENT, "%u long-row chunks (at most %u)", host.slots, kMaxCsrSlots);
   auto* d = new tsn_direction();
   d->h = h;
   d->csr = true;
   (void)hipGetDevice(&d->device);
-  d->csr_rows = static_cast<uint32_t>(rows.size());
-  d->n_csr_items = static_cast<uint32_t>(items.size());
-  d->n_csr_active_items = active_items;
-  d->n_slots = slots;
-  d->n_counters = counters;
+  d->n_csr_blocks = static_cast<uint32_t>(host.blocks.size());
+  d->n_csr_active_blocks = active_blocks;
+  d->n_slots = host.slots;
+  d->n_counters = host.counters;
   size_t bytes = 0;
-  int rc = device_copy(ptr.data(), ptr.size(), &d->row_ptr, &bytes);
-  if (rc == TSN_OK) rc = device_copy(rows.data(), rows.size(), &d->row_ids, &bytes);
-  if (rc == TSN_OK) rc = device_copy(cols.data(), cols.size(), &d->cols, &bytes);
-  if (rc == TSN_OK) rc = device_copy(vals.data(), vals.size(), &d->vals, &bytes);
-  if (rc == TSN_OK) rc = device_copy(items.data(), items.size(), &d->csr_items, &bytes);
-  if (rc == TSN_OK && slots) {
-    const std::vector<float> zeros(static_cast<size_t>(slots) * 2 * kMaxCoils, 0.0f);
-    const std::vector<uint32_t> zero_counters(round_up(counters, 4u), 0u);
+  int rc = device_copy(host.row_ids.data(), host.row_ids.size(), &d->row_ids, &bytes);
+  if (rc == TSN_OK) rc = device_copy(host.cols.data(), host.cols.size(), &d->csr_cols, &bytes);
+  if (rc == TSN_OK) rc = device_copy(host.blocks.data(), host.blocks.size(), &d->csr_blocks, &bytes);
+  if (rc == TSN_OK) rc = device_copy(host.rounds.data(), host.rounds.size(), &d->csr_rounds, &bytes);
+  if (rc == TSN_OK) {
+    auto copy_parts = [&](auto** to, size_t count, auto part) -> int {
+      using T = std::remove_pointer_t<std::remove_pointer_t<decltype(to)>>;
+      if (count == 0) return TSN_OK;
+      TSN_HIP(hipMalloc(reinterpret_cast<void**>(to), count * sizeof(T)));
+      size_t at = 0;
+      for (const CsrHost& q : parts) {
+        const auto& v = part(q);
+        if (!v.empty()) TSN_HIP(hipMemcpy(*to + at, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+        at += v.size();
+      }
+      bytes += count * sizeof(T);
+      return TSN_OK;
+    };
+    rc = copy_parts(&d->vals, static_cast<size_t>(steps) * 64,
+                    [](const CsrHost& q) -> const std::vector<float2>& { return q.vals; });
+    if (rc == TSN_OK)
+      rc = copy_parts(&d->csr_idx, static_cast<size_t>(words) * 64,
+                      [](const CsrHost& q) -> const std::vector<uint32_t>& { return q.idx; });
+  }
+  if (rc == TSN_OK && host.slots) {
+    const std::vector<float> zeros(static_cast<size_t>(host.slots) * 2 * kMaxCoils, 0.0f);
+    const std::vector<uint32_t> zero_counters(round_up(host.counters, 4u), 0u);
     rc = device_copy(zeros.data(), zeros.size(), &d->partials, &bytes);
     if (rc == TSN_OK) rc = device_copy(zero_counters.data(), zero_counters.size(), &d->counters, &bytes);
   }

@@ -24,18 +24,16 @@ constexpr int kSplitAboveTiles = 16;  // tiles per unit at most; longer groups a
 // Interleaved-panel interpolation of 9..16 coils: waves per work entry, 1 (one
 // wave computes both coil blocks) or 2 (one wave per block, same entry).
 constexpr uint32_t kDefaultCoilWaves = 1;
-// FP32 CSR work items: runs of at most kCsrRowsPerItem consecutive rows of at
-// most kCsrShortEntries entries each, the first not empty; longer rows are
-// cut into chunks of at most kCsrChunkEntries entries; a run that would start
-// with an empty row takes the consecutive empty rows instead, at most
-// kCsrEmptyRunRows (no entries to stage).  A wave stages an item's entries in
-// LDS.
-constexpr int kCsrRowsPerItem = 8;
-constexpr int kCsrEmptyRunRows = 64;
-constexpr int kCsrShortEntries = 64;
-constexpr int kCsrChunkEntries = 256;
-constexpr int kCsrStageEntries = kCsrRowsPerItem * kCsrShortEntries;
-static_assert(kCsrChunkEntries <= kCsrStageEntries, "a chunk must fit the LDS stage");
+// FP32 path (interp_csr_kernel): distinct input rows of a round's LDS stage
+// (row 0 of the 256 is zero), entries of a short row (one quad, entry order)
+// and of a chunk of a longer one, rows of a run of empty rows, ranges of rows
+// that csr_build works on side by side (at most, and their entries at least).
+constexpr uint32_t kCsrCols = 255;
+constexpr uint32_t kCsrShortEntries = 64;
+constexpr uint32_t kCsrChunkEntries = 256;
+constexpr uint32_t kCsrEmptyRunRows = 64;
+constexpr uint32_t kCsrParts = 16;
+constexpr uint32_t kCsrPartEntries = 1u << 18;
 // Device column words of packed tiles hold column * 32 (a byte offset) below
 // bit 31, so a pack may have at most 2^26 columns.
 constexpr uint32_t kMaxDeviceCols = 1u << 26;
@@ -172,16 +170,38 @@ struct ChunkItem {
   uint32_t counter;  // arrival counter of the group (reset to 0 by the last arrival)
   uint32_t problem;  // batched launches: the problem table entry
 };
-// One work item of the FP32 CSR kernel: a run of short rows (n_chunks 0), or
-// chunk `chunk` of the n_chunks chunks of one long row.  A row of several
-// chunks has partial slots slot0 .. slot0 + n_chunks - 1 (kMaxCoils float2
-// each) and arrival counter `counter`.
-struct CsrItem {
-  uint32_t row_begin, row_end;  // CSR rows (a chunk: row_end = row_begin + 1)
-  uint32_t e_begin, e_end;      // the item's entries, contiguous in the CSR arrays
-  uint32_t chunk, n_chunks;
-  uint32_t slot0, counter;
+// One round of an FP32 block: n_cols distinct columns (cols from col0; local
+// column i + 1, 0 names a zero row), and byte w of `steps` steps of wave w.  At
+// a step lane 4q + k of a wave holds an entry of its quad q: entry i of the
+// quad sits at lane i mod 4 and the steps follow i / 4.  Values [step][64] from
+// ent0 (in steps, the waves one after the other), local columns one byte a step
+// in words [step / 4][64] from idx0.
+struct CsrRound {
+  uint32_t col0, n_cols, ent0, idx0, steps;
 };
+// One block of the FP32 kernel: n_rows rows (row_ids from row0) in n_rounds
+// rounds (first, then rounds[round0 ..]).  n_chunks 0: quad i is row i (rows of
+// up to kCsrShortEntries entries).  Else quads 4r .. 4r + 3 are chunk `chunk` of
+// the n_chunks chunks of row r, quad 4r + p its entries p mod 4; with several
+// chunks, chunk c's row r has partial slot slot0 + c n_rows + r, the rows
+// arrival counter `counter`.  n_rounds 0: a run of empty rows.
+struct CsrBlock {
+  CsrRound first;
+  uint32_t row0, n_rows, n_rounds, round0;
+  uint32_t n_chunks, chunk, slot0, counter;
+};
+// Host form of an FP32 direction's device arrays, or of one range of its rows.
+struct CsrHost {
+  std::vector<CsrBlock> blocks;
+  std::vector<CsrRound> rounds;
+  std::vector<uint32_t> cols, idx;
+  std::vector<int32_t> row_ids;
+  std::vector<float2> vals;
+  uint32_t slots = 0, counters = 0;
+};
+bool csr_build(const std::vector<uint32_t>& ptr, const std::vector<int32_t>& cols, const std::vector<float2>& vals,
+               const std::vector<int32_t>& rows, const std::vector<uint32_t>& perm, uint32_t n_cols,
+               std::vector<CsrHost>* out);
 // Floats of one partial slot: two coil blocks x (re, im) x 64 lanes x float4.
 constexpr uint32_t kSlotFloats = 2 * 2 * 64 * 4;
 // Launch order entries: a unit index, or kChunkTag | chunk index.  Units and
@@ -191,9 +211,6 @@ constexpr uint32_t kSlotFloats = 2 * 2 * 64 * 4;
 constexpr uint32_t kChunkTag = 0x80000000u;
 // Chunks of a direction's long groups with slots and counters numbered from
 // slot_base / counter_base (host side).
-// FP32 CSR work items of row pointers ptr (host side); slots and counters of
-// the rows of several chunks are numbered from 0.
-std::vector<CsrItem> csr_items(const std::vector<uint32_t>& ptr, uint32_t* slots, uint32_t* counters);
 // Slot offsets of CSR chunks are 32-bit buffer offsets of kMaxCoils float2.
 constexpr uint32_t kMaxCsrSlots = (1u << 31) / (kMaxCoils * 8);
 std::vector<ChunkItem> long_chunks(const std::vector<uint32_t>& group_offsets, uint32_t problem, uint32_t slot_base,
@@ -326,14 +343,14 @@ struct tsn_direction {
   std::vector<uint32_t> host_order;
   std::vector<void*> retired;          // earlier schedules (graphs may reference them)
   // ---- FP32 CSR (device)
-  uint32_t csr_rows = 0;
-  uint32_t* row_ptr = nullptr;   // [csr_rows + 1]
-  int32_t* row_ids = nullptr;    // [csr_rows] logical output row
-  int32_t* cols = nullptr;       // [nnz]
-  float2* vals = nullptr;        // [nnz]
-  tsn::CsrItem* csr_items = nullptr;  // [n_csr_items] work items in launch order
-  uint32_t n_csr_items = 0;
-  uint32_t n_csr_active_items = 0;  // leading items holding a row with entries (the rest zero empty rows)
+  int32_t* row_ids = nullptr;         // output rows of the blocks
+  uint32_t* csr_cols = nullptr;       // distinct columns of the blocks
+  float2* vals = nullptr;             // entry values, [steps][64] per wave
+  uint32_t* csr_idx = nullptr;        // local columns
+  tsn::CsrRound* csr_rounds = nullptr;  // rounds after the first of the blocks
+  tsn::CsrBlock* csr_blocks = nullptr;
+  uint32_t n_csr_blocks = 0;
+  uint32_t n_csr_active_blocks = 0;   // leading blocks holding rows with entries (the rest zero empty rows)
   // (partials / counters / n_slots / n_counters above hold the long-row chunk
   // scratch of a CSR direction: kMaxCoils float2 per slot)
   size_t bytes = 0;
