@@ -33,7 +33,7 @@ constexpr uint32_t kCsrShortEntries = 64;
 constexpr uint32_t kCsrChunkEntries = 256;
 constexpr uint32_t kCsrEmptyRunRows = 64;
 constexpr uint32_t kCsrParts = 16;
-constexpr uint32_t kCsrPartEntries = 1u << 18;
+constexpr uint32_t kCsrPartEntries = 1u << 15;
 // Device column words of packed tiles hold column * 32 (a byte offset) below
 // bit 31, so a pack may have at most 2^26 columns.
 constexpr uint32_t kMaxDeviceCols = 1u << 26;
