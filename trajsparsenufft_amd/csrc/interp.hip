@@ -41,7 +41,7 @@ namespace tsn {
 // kOutBlockRows (host side only): row-major float2 in blocks of 8 coils, block
 // b of rows at b * n_out * 8 (64-byte rows), launched as kOutRowMajor with
 // the block stride set.
-enum OutMode { kOutCoilMajor = 0, kOutRowMajor = 1, kOutSplit16 = 2, kOutSplit16IL = 3, kOutSplitBF16IL = 4,
+enum OutMode { kOutCoilMajor = 0, kOutRowMajor = 1, kOutSplit16IL = 3, kOutSplitBF16IL = 4,
                kOutBlockRows = 5 };
 // Tile kinds: FP16 tiles x FP16 hi + residual on smfmac, the same on dense
 // MFMA, FP16 hi only, and BF16 tiles x BF16 hi + residual on smfmac.
@@ -70,8 +70,6 @@ struct InterpArgs {
   uint32_t n_out;         // output rows (for layouts)
   float scale;
   float* out_f32;         // float2 output (coil- or row-major)
-  _Float16* out_hi;       // split output panel blocks
-  _Float16* out_res;
   uint32_t* out_il;       // interleaved split output panel blocks, or line rows
   uint32_t lines;         // one wave per coil block (WB = 2): the interleaved panels hold line rows, not blocks
   // row-major float2 output: (row, coil) at float2 (coil >> 3) * out_bs +
@@ -181,61 +179,102 @@ __device__ __forceinline__ float dc_apply(const InterpArgs& a, float v, uint32_t
   return dc_residual(v, y, a.dc_scale, w);
 }
 
+// Exchanges within the wave's 16-lane rows by DPP.  lane_xor: the value of lane
+// n ^ OFF.  swap_lanes: lanes with bit OFF of n clear take the partner's x into
+// y, the others the partner's y into x.
+constexpr int kRor8 = 0x128, kShl4 = 0x104, kShr4 = 0x114;  // row rotate by 8, lane n reads n + 4, n - 4
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float v) {
+  const int i = __builtin_bit_cast(int, v);
+  if constexpr (OFF == 8) return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(i, kRor8, 0xF, 0xF, true));
+  const int up = __builtin_amdgcn_update_dpp(i, i, kShl4, 0xF, 0x5, false);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, i, kShr4, 0xF, 0xA, false));
+}
+template <int OFF>
+__device__ __forceinline__ void swap_lanes(uint32_t& x, uint32_t& y) {
+  static_assert(OFF == 4 || OFF == 8, "lane bit 2 or 3");
+  const int x0 = static_cast<int>(x), y0 = static_cast<int>(y);
+  y = static_cast<uint32_t>(OFF == 8 ? __builtin_amdgcn_update_dpp(y0, x0, kRor8, 0xF, 0x3, false)
+                                     : __builtin_amdgcn_update_dpp(y0, x0, kShl4, 0xF, 0x5, false));
+  x = static_cast<uint32_t>(OFF == 8 ? __builtin_amdgcn_update_dpp(x0, y0, kRor8, 0xF, 0xC, false)
+                                     : __builtin_amdgcn_update_dpp(x0, y0, kShr4, 0xF, 0xA, false));
+}
+template <int OFF>
+__device__ __forceinline__ void swap_lanes(float& x, float& y) {
+  uint32_t u = __builtin_bit_cast(uint32_t, x), v = __builtin_bit_cast(uint32_t, y);
+  swap_lanes<OFF>(u, v);
+  x = __builtin_bit_cast(float, u);
+  y = __builtin_bit_cast(float, v);
+}
+
+// One float2 output value from the Re and the Im channel's sums.
+template <int OM, bool CONJ, bool ACC>
+__device__ __forceinline__ void store_value(const InterpArgs& a, int row, uint32_t coil, float rr, float ri, float ir,
+                                            float ii) {
+  float2_t v = {(CONJ ? rr + ii : rr - ii) * a.scale, (CONJ ? ir - ri : ir + ri) * a.scale};
+  if (row < 0 || coil >= a.coils) return;
+  size_t o;
+  if constexpr (OM == kOutCoilMajor) o = static_cast<size_t>(coil) * a.n_out + row;
+  else o = (coil >> 3) * a.out_bs + static_cast<size_t>(row) * a.out_rs + (coil & 7);
+  auto* out = glb(reinterpret_cast<float2_t*>(a.out_f32));
+  if constexpr (ACC) v += out[o];
+  out[o] = v;
+}
+
+// One coil block's rows from the wave's accumulators.  Lane n of a quarter
+// holds part n >> 3 (Re or Im) of coil n & 7 for four rows, lane n ^ 8 the
+// coil's other part.  Split outputs write a word a lane and row.  For float2
+// outputs the two lanes exchange accumulators, so that the Re lane holds both
+// parts of rows 0 and 1 and the Im lane those of rows 2 and 3: two 8-byte stores
+// a lane, where a store per part took four of 4 bytes (adjoint, 512^2 / 8 coils:
+// 17.9 -> 17.2 us).
 template <int OM, bool CONJ, bool ACC, int WB>
 __device__ __forceinline__ void interp_epilogue(const InterpArgs& a, const int4& rows, int b,
                                                 const float4_t& acc_re, const float4_t& acc_im,
                                                 int lane) {
   const int n = lane & 15;
-  const int rr[4] = {rows.x, rows.y, rows.z, rows.w};
   const uint32_t coil = a.coil_base + b * kCoilsPerBlock + (n & 7);
-  const int part = n >> 3;
+  if constexpr (OM == kOutSplitBF16IL || OM == kOutSplit16IL) {
+    const int rr[4] = {rows.x, rows.y, rows.z, rows.w};
+    const bool im = n & 8;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float other = __shfl_xor(acc_im[i], 8);
-    float v;
-    if (n < 8) v = CONJ ? acc_re[i] + other : acc_re[i] - other;
-    else v = CONJ ? acc_re[i] - other : acc_re[i] + other;
-    v *= a.scale;
-    const int row = rr[i];
-    if (row < 0) continue;
-    if constexpr (OM == kOutSplitBF16IL || OM == kOutSplit16IL) {
-      if (a.dc_meas) v = dc_apply(a, v, coil, row, part);
+    for (int i = 0; i < 4; ++i) {
+      const float x = lane_xor<8>(acc_im[i]);
+      float v = (im == CONJ ? acc_re[i] - x : acc_re[i] + x) * a.scale;
+      const int row = rr[i];
+      if (row < 0) continue;
+      if (a.dc_meas) v = dc_apply(a, v, coil, row, im ? 1 : 0);
       const size_t o = WB > 1 && a.lines ? (static_cast<size_t>(row) * 2 + b) * kN
                                          : (static_cast<size_t>(b) * a.n_out + row) * kN;
       glb(a.out_il)[o + n] = split_word<OM == kOutSplitBF16IL>(v);
-    } else if constexpr (OM == kOutSplit16) {
-      asm volatile("" : "+v"(v));  // split the FP32 value (see split_word)
-      const _Float16 hi = static_cast<_Float16>(v);
-      const _Float16 res = static_cast<_Float16>(v - static_cast<float>(hi));
-      const size_t o = (static_cast<size_t>(b) * a.n_out + row) * kN + n;
-      glb(a.out_hi)[o] = hi;
-      glb(a.out_res)[o] = res;
-    } else {
-      if (coil >= a.coils) continue;
-      size_t o;
-      if constexpr (OM == kOutCoilMajor) o = (static_cast<size_t>(coil) * a.n_out + row) * 2 + part;
-      else o = ((coil >> 3) * a.out_bs + static_cast<size_t>(row) * a.out_rs + (coil & 7)) * 2 + part;
-      if constexpr (ACC) v += glb(a.out_f32)[o];
-      glb(a.out_f32)[o] = v;
+    }
+  } else {
+    // rows.x and rows.y: rows 0 and 1 in the Re lane, 2 and 3 in the Im lane (group_rows_of)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float rr = acc_re[i], ir = acc_re[2 + i], ri = acc_im[i], ii = acc_im[2 + i];
+      swap_lanes<8>(rr, ir);
+      swap_lanes<8>(ri, ii);
+      store_value<OM, CONJ, ACC>(a, i ? rows.y : rows.x, coil, rr, ri, ir, ii);
     }
   }
 }
 
 // The epilogue of both coil blocks of kLines panels.  Accumulator b of lane n
-// of a quarter is word w = 4 (n & 7) + 2 (n >> 3) + b of the 32-word row (see
-// fetch_ops): part (n >> 1) & 1 (Re or Im) of coil 8 ((n >> 2) & 1) + 4 (n & 1)
-// + 2 (n >> 3) + b, and lane n ^ 2 holds the coil's other part.  Split outputs
-// write the two words with one 8-byte store (128 contiguous bytes a row);
-// float2 outputs exchange accumulators so that the Re lane holds both parts of
-// its b = 0 coil and the Im lane both parts of its b = 1 coil, one 8-byte store
-// each.
+// of a quarter is word 16 ((n >> 1) & 1) + 8 ((n >> 2) & 1) + 4 (n & 1) +
+// 2 (n >> 3) + b of the 32-word row (see fetch_ops): part (n >> 2) & 1 (Re or
+// Im) of coil 8 ((n >> 1) & 1) + 4 (n & 1) + 2 (n >> 3) + b, and lane n ^ 4
+// holds the coil's other part.  Split outputs write the two words with one
+// 8-byte store (128 contiguous bytes a row); float2 outputs exchange
+// accumulators so that the Re lane holds both parts of its b = 0 coil and the
+// Im lane both parts of its b = 1 coil, one 8-byte store each.
 template <int OM, bool CONJ, bool ACC>
 __device__ __forceinline__ void interp_epilogue_lines(const InterpArgs& a, const int4& rows,
                                                       const float4_t (&acc_re)[2], const float4_t (&acc_im)[2],
                                                       int lane) {
   const uint32_t n = lane & 15;
-  const bool im = (n >> 1) & 1u;
-  const uint32_t coil0 = a.coil_base + ((n >> 2) & 1u) * kCoilsPerBlock + 4 * (n & 1) + 2 * (n >> 3);
+  const bool im = n & 4u;
+  const uint32_t coil0 = a.coil_base + ((n >> 1) & 1u) * kCoilsPerBlock + 4 * (n & 1) + 2 * (n >> 3);
   const int rr[4] = {rows.x, rows.y, rows.z, rows.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -244,8 +283,8 @@ __device__ __forceinline__ void interp_epilogue_lines(const InterpArgs& a, const
       float v[2];
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        const float other = __shfl_xor(acc_im[b][i], 2);
-        v[b] = (im == CONJ ? acc_re[b][i] - other : acc_re[b][i] + other) * a.scale;
+        const float x = lane_xor<4>(acc_im[b][i]);
+        v[b] = (im == CONJ ? acc_re[b][i] - x : acc_re[b][i] + x) * a.scale;
       }
       if (row < 0) continue;
       if (a.dc_meas) {
@@ -253,22 +292,13 @@ __device__ __forceinline__ void interp_epilogue_lines(const InterpArgs& a, const
         for (int b = 0; b < 2; ++b) v[b] = dc_apply(a, v[b], coil0 + b, row, im ? 1 : 0);
       }
       const u32x2_t w = {split_word<OM == kOutSplitBF16IL>(v[0]), split_word<OM == kOutSplitBF16IL>(v[1])};
-      glb(reinterpret_cast<u32x2_t*>(a.out_il))[static_cast<size_t>(row) * kN + 2 * (n & 7) + (n >> 3)] = w;
+      glb(reinterpret_cast<u32x2_t*>(a.out_il))[static_cast<size_t>(row) * kN + 8 * ((n >> 1) & 1u) +
+                                                4 * ((n >> 2) & 1u) + 2 * (n & 1u) + (n >> 3)] = w;
     } else {
-      const float re = im ? acc_re[1][i] : acc_re[0][i], iv = im ? acc_im[1][i] : acc_im[0][i];
-      const float ore = __shfl_xor(im ? acc_re[0][i] : acc_re[1][i], 2);
-      const float oim = __shfl_xor(im ? acc_im[0][i] : acc_im[1][i], 2);
-      const float rr_ = im ? ore : re, ri = im ? oim : iv;  // the Re channel's sums
-      const float ir = im ? re : ore, ii = im ? iv : oim;   // the Im channel's sums
-      float2_t v = {(CONJ ? rr_ + ii : rr_ - ii) * a.scale, (CONJ ? ir - ri : ir + ri) * a.scale};
-      const uint32_t coil = coil0 + (im ? 1u : 0u);
-      if (row < 0 || coil >= a.coils) continue;
-      size_t o;
-      if constexpr (OM == kOutCoilMajor) o = static_cast<size_t>(coil) * a.n_out + row;
-      else o = (coil >> 3) * a.out_bs + static_cast<size_t>(row) * a.out_rs + (coil & 7);
-      auto* out = glb(reinterpret_cast<float2_t*>(a.out_f32));
-      if constexpr (ACC) v += out[o];
-      out[o] = v;
+      float re = acc_re[0][i], ir = acc_re[1][i], ri = acc_im[0][i], ii = acc_im[1][i];
+      swap_lanes<4>(re, ir);
+      swap_lanes<4>(ri, ii);
+      store_value<OM, CONJ, ACC>(a, row, coil0 + (im ? 1u : 0u), re, ri, ir, ii);
     }
   }
 }
@@ -328,15 +358,27 @@ __device__ __forceinline__ TileRsrc<NB> make_tile_rsrc(const InterpArgs& a, uint
   return r;
 }
 
-// Output rows of the lane's four accumulator rows (4q .. 4q+3) of group g.
-template <int NB>
+// Where a lane's output rows of a group start among its 16 (in bytes): the
+// quarter's four accumulator rows 4q .. 4q + 3, or, for one coil block's float2
+// output, the two of them that the lane stores (interp_epilogue).
+template <int IL, int OM>
+__device__ __forceinline__ int rows_offset(int lane) {
+  constexpr bool kPair = IL != kLines && (OM == kOutCoilMajor || OM == kOutRowMajor);
+  return (lane >> 4) * 16 + (kPair && (lane & 8) ? 8 : 0);
+}
+
+// Output rows of group g (x and y only where a lane stores two rows; past the
+// table's end the buffer range check returns zeros for the unused z and w).
+template <int NB, int IL, int OM>
 __device__ __forceinline__ int4 load_rows(const TileRsrc<NB>& r, int g, int lane) {
-  const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r.rows, (lane >> 4) * 16, g * 64, 0);
+  const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r.rows, rows_offset<IL, OM>(lane), g * 64, 0);
   return make_int4(static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z), static_cast<int>(v.w));
 }
 
+template <int IL, int OM>
 __device__ __forceinline__ int4 group_rows_of(const InterpArgs& a, uint32_t group, int lane) {
-  const auto* p = glb(a.group_rows + static_cast<size_t>(group) * 16 + (lane >> 4) * 4);
+  const auto* p = glb(a.group_rows + static_cast<size_t>(group) * 16) + rows_offset<IL, OM>(lane) / 4;
+  if constexpr (IL != kLines && (OM == kOutCoilMajor || OM == kOutRowMajor)) return make_int4(p[0], p[1], -1, -1);
   return make_int4(p[0], p[1], p[2], p[3]);
 }
 
@@ -392,7 +434,7 @@ template <int NB, int IL>
 struct TileOps {
   u32x4_t a0, a1;
   uint32_t idx, last;
-  uint32_t w[NB][IL ? 8 : 16];
+  uint32_t w[NB][IL == kHalves ? 16 : 8];
 };
 
 template <int KIND, int NB, int IL, int WB>
@@ -402,16 +444,17 @@ __device__ __forceinline__ void fetch_ops(const TileRsrc<NB>& r, int t, const Ti
   const uint32_t cw[8] = {c.c0.x, c.c0.y, c.c0.z, c.c0.w, c.c1.x, c.c1.y, c.c1.z, c.c1.w};
   if constexpr (IL == kLines) {
     // Whole 128-byte lines, 16 bytes a lane: lanes n < 8 of quarter q read its
-    // columns 8q .. 8q + 3, lanes n >= 8 columns 8q + 4 .. 8q + 7, words
-    // 4 (n & 7) .. + 3 of each (mma_tile exchanges half of them with lane
-    // n ^ 8).  Rows of 128 bytes in L2, 32 columns a step, 16 waves a CU: 80
+    // columns 8q .. 8q + 3, lanes n >= 8 columns 8q + 4 .. 8q + 7, 16-byte quad
+    // 4 ((n >> 1) & 1) + 2 ((n >> 2) & 1) + (n & 1) of each (block, part, coil
+    // half; mma_tile exchanges half of the words with lane n ^ 8).  Rows of 128 bytes in L2, 32 columns a step, 16 waves a CU: 80
     // cycles a CU, against 104 as two 64-byte halves in 4-byte loads and 140
     // in 8-byte loads.
     static_assert(NB == 2, "line rows hold two coil blocks");
+    const uint32_t quad = ((n & 2) << 5) | ((n & 4) << 3) | ((n & 1) << 4);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const u32x4_t v =
-          __builtin_amdgcn_raw_buffer_load_b128(r.hi[0], static_cast<int>((cw[j] << 2) | ((n & 7) << 4)), 0, 0);
+          __builtin_amdgcn_raw_buffer_load_b128(r.hi[0], static_cast<int>((cw[j] << 2) | quad), 0, 0);
       o.w[0][j] = v.x;
       o.w[1][j] = v.y;
       o.w[0][4 + j] = v.z;
@@ -458,29 +501,20 @@ __device__ __forceinline__ half8_t pack_halves(const uint32_t* w, uint32_t sel) 
 }
 constexpr uint32_t kSelLo = 0x05040100u, kSelHi = 0x07060302u;
 
-// Exchange between lanes n and n ^ 8 of each 16-lane row: lanes n < 8 take the
-// partner's x into y, lanes n >= 8 the partner's y into x.
-__device__ __forceinline__ void swap_halves(uint32_t& x, uint32_t& y) {
-  constexpr int kRor8 = 0x128;  // DPP row rotate by 8
-  const uint32_t x0 = x, y0 = y;
-  y = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(y0), static_cast<int>(x0), kRor8, 0xF, 0x3, false));
-  x = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(x0), static_cast<int>(y0), kRor8, 0xF, 0xC, false));
-}
-
 template <int KIND, int NB, int IL>
 __device__ __forceinline__ void mma_tile(TileOps<NB, IL>& o, float4_t (&acc_re)[NB],
                                          float4_t (&acc_im)[NB]) {
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     if constexpr (IL == kLines) {
-      // every lane gets words 4 (n & 7) + 2 (n >> 3) + b of all 8 columns
+      // every lane gets words 2 (n >> 3) + b of its quad of all 8 columns
 #pragma unroll
-      for (int j = 0; j < 4; ++j) swap_halves(o.w[b][j], o.w[b][4 + j]);
+      for (int j = 0; j < 4; ++j) swap_lanes<8>(o.w[b][j], o.w[b][4 + j]);
     }
     const half8_t hi = pack_halves(o.w[b], kSelLo);
     half8_t res;
-    if constexpr (IL) res = pack_halves(o.w[b], kSelHi);
-    else res = pack_halves(o.w[b] + 8, kSelLo);
+    if constexpr (IL == kHalves) res = pack_halves(o.w[b] + 8, kSelLo);
+    else res = pack_halves(o.w[b], kSelHi);
     if constexpr (KIND == kDenseSplit) {
       const half8_t dre = __builtin_bit_cast(half8_t, o.a0);
       const half8_t dim = __builtin_bit_cast(half8_t, o.a1);
@@ -518,8 +552,8 @@ __device__ __forceinline__ void mma_tile(TileOps<NB, IL>& o, float4_t (&acc_re)[
 // occupancy).
 template <int KIND, int NB, int IL>
 struct PipeDepth {
-  static constexpr int value = (IL && NB == 1 && KIND != kDenseSplit) ? 2
-                               : (NB == 2 && (!IL || KIND == kDenseSplit)) ? 0
+  static constexpr int value = (IL != kHalves && NB == 1 && KIND != kDenseSplit) ? 2
+                               : (NB == 2 && (IL == kHalves || KIND == kDenseSplit)) ? 0
                                                                           : 1;
 };
 
@@ -553,7 +587,7 @@ __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc
   auto tile = [&](int i) { return min(first + i, last); };
   auto cols_of = [&](int i) { return staged_cols<IL>(stage, tile(i) - first, lane); };
   last_mask = __builtin_amdgcn_readfirstlane(last_mask);
-  int4 rows = load_rows(r, g, lane);
+  int4 rows = load_rows<NB, IL, OM>(r, g, lane);
   TileCols cols[U];
   TileOps<NB, IL> ops[U];
   // The scheduler must keep the issue order: the wait counter is in order, and
@@ -586,7 +620,7 @@ __device__ __forceinline__ void stream_tiles(const InterpArgs& a, const TileRsrc
             acc_im[b] = float4_t{0.f, 0.f, 0.f, 0.f};
           }
           g = min(g + 1, g_last);
-          rows = load_rows(r, g, lane);
+          rows = load_rows<NB, IL, OM>(r, g, lane);
         }
       }
     }
@@ -643,7 +677,7 @@ __device__ __forceinline__ void chunk_finish(const InterpArgs& a, const ChunkIte
   asm volatile("" ::: "memory");
   if (lane == 0) __hip_atomic_store(a.counters + c.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int first = static_cast<int>(c.slot0 * kSlotFloats * 4);
-  const int4 rows = group_rows_of(a, static_cast<uint32_t>(c.group), lane);
+  const int4 rows = group_rows_of<IL, OM>(a, static_cast<uint32_t>(c.group), lane);
   const uint32_t n = c.n_chunks;
   float4_t sum_re[NB * WB], sum_im[NB * WB];
 #pragma unroll
@@ -735,11 +769,9 @@ __device__ __forceinline__ void tiles_entry(InterpArgs a) {
     vw.coil_base = v.coil_base + wb * kCoilsPerBlock;
     const size_t out_block = static_cast<size_t>(wb) * v.n_out * kN;
     vw.out_il = v.out_il ? v.out_il + (vw.lines ? static_cast<size_t>(wb) * kN : out_block) : nullptr;
-    vw.out_hi = v.out_hi ? v.out_hi + out_block : nullptr;
-    vw.out_res = v.out_res ? v.out_res + out_block : nullptr;
   }
   if (u.tile_begin == u.tile_end) {  // empty group: zero rows
-    const int4 rows = group_rows_of(vw, static_cast<uint32_t>(u.group), lane);
+    const int4 rows = group_rows_of<IL, OM>(vw, static_cast<uint32_t>(u.group), lane);
     write_group<NB, IL, OM, CONJ, ACC, WB>(vw, rows, acc_re, acc_im, lane);
     return;
   }
@@ -1144,7 +1176,7 @@ __global__ __launch_bounds__(256) void dc_residual_kernel(const float* __restric
 // for one coil block, 2 for two.
 template <int KIND, int NB, int IL, int OM, bool CONJ, bool ACC, int WB>
 struct AltDepths {
-  static constexpr bool kPlanLaunch = IL && KIND != kDenseSplit && !ACC && WB == 1 &&
+  static constexpr bool kPlanLaunch = (IL != kHalves) && KIND != kDenseSplit && !ACC && WB == 1 &&
                                       ((OM == kOutRowMajor && CONJ) ||
                                        ((OM == kOutSplit16IL || OM == kOutSplitBF16IL) && !CONJ));
 };
@@ -1179,7 +1211,7 @@ static void launch_both(const InterpArgs& a, hipStream_t s) {
 
 template <int KIND, int NB, int IL, int OM, int WB = 1>
 static void launch_tiles_om(const InterpArgs& a, bool conj, bool acc, hipStream_t s) {
-  constexpr bool kAccOk = OM != kOutSplit16 && OM != kOutSplit16IL && OM != kOutSplitBF16IL;
+  constexpr bool kAccOk = OM != kOutSplit16IL && OM != kOutSplitBF16IL;
   if (conj) {
     if (kAccOk && acc) launch_both<KIND, NB, IL, OM, true, kAccOk, WB>(a, s);
     else launch_both<KIND, NB, IL, OM, true, false, WB>(a, s);
@@ -1194,15 +1226,14 @@ static void launch_tiles_om(const InterpArgs& a, bool conj, bool acc, hipStream_
 // launch_interp).  WB = 2: two coil blocks, one wave each (NB = 1).
 template <int KIND, int NB, int IL, int WB = 1>
 static void launch_tiles_nb(const InterpArgs& a, int om, bool conj, bool acc, hipStream_t s) {
-  if constexpr (IL) {
+  if constexpr (IL != kHalves) {
     if (om == kOutCoilMajor) launch_tiles_om<KIND, NB, IL, kOutCoilMajor, WB>(a, conj, acc, s);
     else if (om == kOutRowMajor) launch_tiles_om<KIND, NB, IL, kOutRowMajor, WB>(a, conj, acc, s);
     else if (KIND == kSparseSplitBF16) launch_tiles_om<KIND, NB, IL, kOutSplitBF16IL, WB>(a, conj, false, s);
     else launch_tiles_om<KIND, NB, IL, kOutSplit16IL, WB>(a, conj, false, s);
   } else {
     if (om == kOutCoilMajor) launch_tiles_om<KIND, NB, IL, kOutCoilMajor>(a, conj, acc, s);
-    else if (om == kOutRowMajor) launch_tiles_om<KIND, NB, IL, kOutRowMajor>(a, conj, acc, s);
-    else launch_tiles_om<KIND, NB, IL, kOutSplit16>(a, conj, false, s);
+    else launch_tiles_om<KIND, NB, IL, kOutRowMajor>(a, conj, acc, s);
   }
 }
 
@@ -1242,7 +1273,7 @@ static int launch_tiles(const InterpArgs& a, int panels, int om, bool conj, bool
 
 static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                               int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                              _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
+                              hipStream_t stream, int panels,
                               uint32_t* out_il, const DcTerms* dc, const ChunkScratch* scratch) {
   const bool interleaved = panels != kHalves;
   if (!d || d->csr) return fail(TSN_ERR_ARGUMENT, "interpolation needs a packed (non-CSR) direction");
@@ -1252,10 +1283,10 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
     return fail(TSN_ERR_ARGUMENT, "missing input panel");
   const bool block_rows = out_mode == kOutBlockRows;
   if (block_rows) out_mode = kOutRowMajor;
-  const bool split_out = out_mode == kOutSplit16 || out_mode == kOutSplit16IL;
-  if (split_out ? (interleaved ? !out_il : (!out_hi || !out_res)) : !out_f32)
+  const bool split_out = out_mode == kOutSplit16IL;
+  if (split_out ? !out_il : !out_f32)
     return fail(TSN_ERR_ARGUMENT, "missing output");
-  if (interleaved ? out_mode == kOutSplit16 : out_mode == kOutSplit16IL)
+  if (split_out && !interleaved)
     return fail(TSN_ERR_ARGUMENT, "output mode %d does not match the panel layout", out_mode);
   if (kind == kDenseSplit && !d->tile_dense)
     return fail(TSN_ERR_ARGUMENT, "direction has no dense-control tiles");
@@ -1292,8 +1323,6 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
   a.lines = lines ? 1u : 0u;
   a.scale = scale;
   a.out_f32 = out_f32;
-  a.out_hi = out_hi;
-  a.out_res = out_res;
   a.out_il = out_il;
   a.out_rs = block_rows ? kCoilsPerBlock : coils;
   a.out_bs = block_rows ? static_cast<uint64_t>(a.n_out) * kCoilsPerBlock : kCoilsPerBlock;
@@ -1320,17 +1349,14 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
 // pointers sized by the caller; panels hold ceil(coils/8) blocks.
 int launch_interp(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                   int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
-                  uint32_t* out_il, const ChunkScratch* scratch) {
-  return launch_interp_impl(d, kind, hi, res, coils, out_mode, conj, accumulate, scale, out_f32, out_hi, out_res,
-                            stream, panels, out_il, nullptr, scratch);
+                  hipStream_t stream, int panels, uint32_t* out_il, const ChunkScratch* scratch) {
+  return launch_interp_impl(d, kind, hi, res, coils, out_mode, conj, accumulate, scale, out_f32, stream, panels, out_il, nullptr, scratch);
 }
 
 int launch_interp_dc(const tsn_direction* d, int kind, const uint32_t* panel, uint32_t coils, float scale,
                      const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch, int panels) {
   if (!dc.y) return fail(TSN_ERR_ARGUMENT, "missing measurements");
-  return launch_interp_impl(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, scale, nullptr, nullptr,
-                            nullptr, s, panels, out_il, &dc, scratch);
+  return launch_interp_impl(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, scale, nullptr, s, panels, out_il, &dc, scratch);
 }
 
 int launch_dc_residual(const float2* pred, uint32_t rows, uint32_t coils, const DcTerms& dc, bool bf16,
@@ -2269,7 +2295,7 @@ int tsn_interp_noalloc(const tsn_direction* d, const void* hi, const void* res, 
     TSN_HIP(hipGetLastError());
   }
   return launch_interp(d, res ? kSparseSplit : kSparseHi, hi, res, coils, out_layout, conjugate != 0,
-                       accumulate != 0, scale, static_cast<float*>(out), nullptr, nullptr, s, kHalves, nullptr,
+                       accumulate != 0, scale, static_cast<float*>(out), s, kHalves, nullptr,
                        d->n_chunks ? &chunk : nullptr);
 }
 
@@ -2363,8 +2389,8 @@ int tsn_direction_autotune(tsn_direction* d, uint32_t coils, void* stream, uint3
     d->pipe_depth = c.depth;
     rc = schedule_units(d, c.unit);
     auto launch = [&]() {
-      return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, 1.0f, nullptr, nullptr,
-                           nullptr, s, d->h.n_cols <= kMaxLineCols ? kLines : kBlocks, out);
+      return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, 1.0f, nullptr, s,
+                           d->h.n_cols <= kMaxLineCols ? kLines : kBlocks, out);
     };
     for (int i = 0; rc == TSN_OK && i < 3; ++i) rc = launch();
     if (rc != TSN_OK) break;
@@ -2601,8 +2627,7 @@ int tsn_interp(const tsn_direction* d, const void* hi, const void* res, void* ou
   if (out_layout != TSN_OUT_COIL_MAJOR && out_layout != TSN_OUT_ROW_MAJOR)
     return fail(TSN_ERR_ARGUMENT, "unknown output layout %d", out_layout);
   return launch_interp(d, res ? kSparseSplit : kSparseHi, hi, res, coils, out_layout, conjugate != 0,
-                       accumulate != 0, scale, static_cast<float*>(out), nullptr, nullptr,
-                       static_cast<hipStream_t>(stream), kHalves, nullptr);
+                       accumulate != 0, scale, static_cast<float*>(out), static_cast<hipStream_t>(stream), kHalves, nullptr);
 }
 
 int tsn_interp_dense(const tsn_direction* d, const void* hi, const void* res, void* out,
@@ -2613,8 +2638,7 @@ int tsn_interp_dense(const tsn_direction* d, const void* hi, const void* res, vo
   if (!res) return fail(TSN_ERR_ARGUMENT, "dense control needs hi and residual panels");
   TSN_CHECK(ensure_dense_tiles(d));
   return launch_interp(d, kDenseSplit, hi, res, coils, out_layout, conjugate != 0, accumulate != 0,
-                       scale, static_cast<float*>(out), nullptr, nullptr,
-                       static_cast<hipStream_t>(stream), kHalves, nullptr);
+                       scale, static_cast<float*>(out), static_cast<hipStream_t>(stream), kHalves, nullptr);
 }
 
 int tsn_interp_f32(const tsn_direction* d, const void* in, void* out, uint32_t coils, int conjugate,
@@ -2632,11 +2656,10 @@ int tsn_interp_il(const tsn_direction* d, const void* panel, void* out, uint32_t
   const int kind = d->values == TSN_VALUES_BF16 ? kSparseSplitBF16 : kSparseSplit;
   if (out_layout == TSN_OUT_SPLIT_IL) {
     if (accumulate) return fail(TSN_ERR_ARGUMENT, "a split-panel output cannot accumulate");
-    return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, conjugate != 0, false, scale, nullptr,
-                         nullptr, nullptr, static_cast<hipStream_t>(stream), kBlocks, static_cast<uint32_t*>(out));
+    return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, conjugate != 0, false, scale, nullptr, static_cast<hipStream_t>(stream), kBlocks, static_cast<uint32_t*>(out));
   }
   return launch_interp(d, kind, panel, nullptr, coils, out_layout, conjugate != 0, accumulate != 0, scale,
-                       static_cast<float*>(out), nullptr, nullptr, static_cast<hipStream_t>(stream), kBlocks, nullptr);
+                       static_cast<float*>(out), static_cast<hipStream_t>(stream), kBlocks, nullptr);
 }
 
 int tsn_interp_dc(const tsn_direction* d, const void* panel, const void* measurements, int measurement_layout,
@@ -2663,7 +2686,7 @@ int tsn_interp_dc(const tsn_direction* d, const void* panel, const void* measure
   auto* out = static_cast<uint32_t*>(out_panel);
   if (mode == TSN_DC_FUSED) return launch_interp_dc(d, kind, static_cast<const uint32_t*>(panel), coils, scale, dc, out, s);
   TSN_CHECK(launch_interp(d, kind, panel, nullptr, coils, kOutRowMajor, false, false, scale,
-                          static_cast<float*>(workspace), nullptr, nullptr, s, kBlocks, nullptr));
+                          static_cast<float*>(workspace), s, kBlocks, nullptr));
   return launch_dc_residual(static_cast<const float2*>(workspace), rows, coils, dc, bf16, out, s);
 }
 

@@ -146,10 +146,10 @@ int op_forward_samples(tsn_plan* pl, float2* out_coil_major, hipStream_t s) {
   }
   if (out_coil_major)
     return launch_interp(pl->fwd, interp_kind(pl), pl->pan_il, nullptr, pl->cfg.coils, 0, false, false, scale,
-                         reinterpret_cast<float*>(out_coil_major), nullptr, nullptr, s, pl->panels, nullptr,
+                         reinterpret_cast<float*>(out_coil_major), s, pl->panels, nullptr,
                          &pl->fwd_chunks);
   return launch_interp(pl->fwd, interp_kind(pl), pl->pan_il, nullptr, pl->cfg.coils, 3, false, false, scale,
-                       nullptr, nullptr, nullptr, s, pl->panels, pl->smp_il, &pl->fwd_chunks);
+                       nullptr, s, pl->panels, pl->smp_il, &pl->fwd_chunks);
 }
 
 // sample panels -> grid (conjugate transpose interpolation)
@@ -160,7 +160,7 @@ int op_adjoint_grid(tsn_plan* pl, hipStream_t s) {
   // row-major (mode 1) up to 8 coils, 8-coil blocks of rows (mode 5) above
   return launch_interp(pl->adj, interp_kind(pl), pl->smp_il, nullptr, pl->cfg.coils,
                        pl->cfg.coils > static_cast<uint32_t>(kCoilsPerBlock) ? 5 : 1, true, false, 1.0f, reinterpret_cast<float*>(pl->grid),
-                       nullptr, nullptr, s, pl->panels, nullptr, &pl->adj_chunks);
+                       s, pl->panels, nullptr, &pl->adj_chunks);
 }
 
 // grid -> image (column-major) with combine, scale, regulariser, dot partial

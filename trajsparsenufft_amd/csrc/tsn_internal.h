@@ -279,8 +279,7 @@ int launch_interp_csr(const tsn_direction* d, const float2* in, uint32_t coils, 
 // kBlocks); scratch null: the direction's own.
 int launch_interp(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                   int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
-                  _Float16* out_hi, _Float16* out_res, hipStream_t stream, int panels,
-                  uint32_t* out_il, const ChunkScratch* scratch = nullptr);
+                  hipStream_t stream, int panels, uint32_t* out_il, const ChunkScratch* scratch = nullptr);
 
 // Data-consistency terms: residual (prediction - scale * y) * w per sample
 // row, y read at row * row_stride + coil * coil_stride + part (floats).
