@@ -162,6 +162,8 @@ FftArgs batch_fft_args(const tsn_batch* bt) {
   a.tw1 = bt->tw1;
   a.smaps_t = bt->smaps_t;
   a.apod_t = bt->apod_t;
+  a.image_s0 = 1;  // column-major vectors
+  a.image_s1 = a.n0;
   a.t_fwd = bt->t_fwd;
   a.panel_il = bt->pan_il;
   a.grid = bt->grid_buf;

@@ -105,26 +105,6 @@ __global__ __launch_bounds__(kVecThreads) void cg_final_out_kernel(
   }
 }
 
-// [rows][cols] -> [cols][rows] complex, 32x32 tiles, optional scale.
-__global__ __launch_bounds__(256) void transpose_kernel(const float2* __restrict__ in, uint32_t rows,
-                                                        uint32_t cols, float scale,
-                                                        float2* __restrict__ out) {
-  __shared__ float2 tile[32][33];
-  const uint32_t bx = blockIdx.x * 32, by = blockIdx.y * 32;
-  for (uint32_t i = threadIdx.y; i < 32; i += 8) {
-    const uint32_t r = by + i, c = bx + threadIdx.x;
-    if (r < rows && c < cols) tile[i][threadIdx.x] = in[static_cast<size_t>(r) * cols + c];
-  }
-  __syncthreads();
-  for (uint32_t i = threadIdx.y; i < 32; i += 8) {
-    const uint32_t c = bx + i, r = by + threadIdx.x;
-    if (r < rows && c < cols) {
-      const float2 v = tile[threadIdx.x][i];
-      out[static_cast<size_t>(c) * rows + r] = make_float2(v.x * scale, v.y * scale);
-    }
-  }
-}
-
 // [coils][n0][n1] -> [n1][cstride][n0]
 __global__ __launch_bounds__(256) void smaps_transpose_kernel(const float2* __restrict__ in, uint32_t coils,
                                                               uint32_t n0, uint32_t n1, uint32_t cstride,

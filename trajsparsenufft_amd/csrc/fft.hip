@@ -33,13 +33,20 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T* gmem(const
 // ---------------------------------------------------------------- kernels
 
 // Forward, first axis: image column n1 (all n0 < N0) of x*S_c*apod for eight
-// coils -> T[k0][n1][c].  Image-space arrays are column-major ([n1][n0]).
-template <int R>
+// coils -> T[k0][n1][c].  CG: the input is the next search direction, formed
+// here from column-major ([n1][n0]) vectors; else image_t at its strides, so
+// that an operator reads a caller's row-major image in place.  A line of it
+// holds 16 columns, so a wave's load touches 64 lines: the block loads the
+// column once, for its eight coils, through LDS.  Against a transpose launch
+// before and behind: a normal call of 64x128 with 5 coils 37.4 -> 31.4 us, of
+// 384^2 with 16 coils 260 -> 253 us (264 us where each coil loads for itself).
+template <int R, bool CG>
 __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   const FftArgs a = problem_view(args, blockIdx.z);
   if (blockIdx.y * 8 >= a.coils) return;  // coil chunk beyond this problem (batched launches)
   extern __shared__ float2 lds[];
   __shared__ double red[24];
+  __shared__ float2 column[CG ? 1 : 32 * R];
   constexpr int K = 64 * R;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // neighbouring columns on one XCD: their 64-byte rows of T fill whole L2 lines
@@ -53,7 +60,10 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   // (branch-free: selected sources, a zero array for the absent ones, so no
   // wait is forced where branches would merge; threads past dot_count load
   // its last entry and drop it below)
-  const bool cg = a.cg_r != nullptr;
+  // (a runtime test although CG launches always set cg_r: without the branch
+  // the compiler moves the update into the loads and takes 131 instead of 114
+  // registers at R = 8, three waves per SIMD instead of four)
+  const bool cg = CG && a.cg_r != nullptr;
   const bool sums = cg || a.rho0_dots != nullptr;
   const uint32_t qi = sums ? min(threadIdx.x, a.dot_count - 1) : 0u;
   const uint32_t qs = cg ? a.dot_count : 0u;
@@ -70,13 +80,17 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   // would be waited for at the branch's end); out-of-range values are zeroed
   // afterwards.  Only j < JN can hold pixels: N0 = K/2.
   constexpr int JN = R >= 2 ? R / 2 : 1;
-  const float2* src_r = a.cg_r ? a.cg_r : a.image_t;
-  const float2* src_p = a.cg_r ? a.cg_p_old : a.image_t;
-  const float2* src_a = a.cg_r ? a.cg_ap : a.image_t;
+  const float2* src_r = cg ? a.cg_r : a.image_t;
+  const float2* src_p = cg ? a.cg_p_old : a.image_t;
+  const float2* src_a = cg ? a.cg_ap : a.image_t;
   const float2* src_s = a.smaps_t + (static_cast<size_t>(n1) * a.cstride + min(c, a.coils - 1)) * a.n0;
-  const bool x_wave = a.cg_r && !a.x_zero && __builtin_amdgcn_readfirstlane(store_vec ? 1 : 0);
+  const bool x_wave = cg && !a.x_zero && __builtin_amdgcn_readfirstlane(store_vec ? 1 : 0);
   float2 img[R], sm[R], pv[R], av[R], xv[R];
   float ap[R];
+  // (one load of the column per block, shared by its eight coils: rows of a
+  // row-major image are a line each)
+  float2 pixel;
+  if constexpr (!CG) pixel = a.image_t[min(threadIdx.x, a.n0 - 1) * a.image_s0 + n1 * a.image_s1];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
     img[j] = pv[j] = sm[j] = av[j] = xv[j] = make_float2(0.f, 0.f);
@@ -84,9 +98,11 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
     if (j >= JN) continue;
     const uint32_t n0 = min(lane + 64u * j, a.n0 - 1);
     const size_t pix = static_cast<size_t>(n1) * a.n0 + n0;
-    img[j] = src_r[pix];
-    pv[j] = src_p[pix];
-    av[j] = src_a[pix];
+    if constexpr (CG) {
+      img[j] = src_r[pix];
+      pv[j] = src_p[pix];
+      av[j] = src_a[pix];
+    }
     sm[j] = src_s[n0];
     ap[j] = a.apod_t[pix];
     if (x_wave) xv[j] = a.cg_x[pix];
@@ -109,8 +125,13 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
       *a.cg_status = 1;
     }
   }
+  if constexpr (!CG) {
+    if (threadIdx.x < a.n0) column[threadIdx.x] = pixel;
+    __syncthreads();
+  }
 #pragma unroll
   for (int j = 0; j < JN; ++j) {
+    if constexpr (!CG) img[j] = column[min(lane + 64u * j, a.n0 - 1)];
     if (!active || lane + 64u * j >= a.n0) {
       img[j] = pv[j] = sm[j] = av[j] = xv[j] = make_float2(0.f, 0.f);
       ap[j] = 0.f;
@@ -143,8 +164,10 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   float2 x[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const float2 v = cmul(img[j], sm[j]);
-    x[j] = make_float2(v.x * ap[j], v.y * ap[j]);
+    // (the roundings spelled out, so that both kernels form the same bits)
+    const float vx = __builtin_fmaf(img[j].x, sm[j].x, -(img[j].y * sm[j].y));
+    const float vy = __builtin_fmaf(img[j].y, sm[j].x, img[j].x * sm[j].y);
+    x[j] = make_float2(vx * ap[j], vy * ap[j]);
   }
   constexpr int TPL = (R * 8 + 63) / 64;
   float2 out[TPL][8];
@@ -299,15 +322,19 @@ __global__ __launch_bounds__(512) void inv_axis0_kernel(FftArgs args) {
   __shared__ double red[24];
   constexpr int K = 64 * R;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint32_t n1 = blockIdx.x;
+  // neighbouring columns on one XCD where their pixels share lines (a caller's
+  // row-major image); column-major vectors have no such lines, and a solve's
+  // pass takes 7.3 us in launch order against 7.8 us (256^2 / 8 coils)
+  const uint32_t n1 = a.image_s0 == 1 ? blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
   constexpr int TPL = (R * 8 + 63) / 64;
   // the epilogue's operands are loaded first, so their latency overlaps the transforms
   // (at a clamped pixel, unconditionally: a load under a lane-dependent branch
   // would be waited for at the branch's end)
   const bool pixel = threadIdx.x < a.n0;
-  const size_t pix = static_cast<size_t>(n1) * a.n0 + min(threadIdx.x, a.n0 - 1);
+  const uint32_t row = min(threadIdx.x, a.n0 - 1);
+  const size_t pix = row * a.image_s0 + n1 * a.image_s1;
   // (an absent input reads the output column instead, unused)
-  const float apv = a.apod_t[pix];
+  const float apv = a.apod_t[static_cast<size_t>(n1) * a.n0 + row];
   const float2 regv = (a.reg_in ? a.reg_in : a.image_out)[pix];
   const float2 rv = (a.dot_r ? a.dot_r : a.image_out)[pix];
   float2 acc = make_float2(0.f, 0.f);
@@ -414,8 +441,13 @@ static int radix_of(uint32_t k) {
 int fft_forward(const FftArgs& a, int out_kind, hipStream_t s, uint32_t problems) {
   const int r0 = radix_of(a.k0), r1 = radix_of(a.k1);
   const uint32_t chunks = (a.cstride + 7) / 8;
-  TSN_DISPATCH_R(r0, hipLaunchKernelGGL(fwd_axis0_kernel<R>, dim3(a.n1, chunks, problems), dim3(512),
-                                        lds_bytes_for<R>(), s, a));
+  if (a.cg_r) {
+    TSN_DISPATCH_R(r0, hipLaunchKernelGGL((fwd_axis0_kernel<R, true>), dim3(a.n1, chunks, problems), dim3(512),
+                                          lds_bytes_for<R>(), s, a));
+  } else {
+    TSN_DISPATCH_R(r0, hipLaunchKernelGGL((fwd_axis0_kernel<R, false>), dim3(a.n1, chunks, problems), dim3(512),
+                                          lds_bytes_for<R>(), s, a));
+  }
   if (out_kind == 0) {
     TSN_DISPATCH_R(r1, hipLaunchKernelGGL((fwd_axis1_kernel<R, 0>), dim3(div_up(a.k0, rows_per_block<R>()), chunks, problems), dim3(512),
                                           lds_bytes_for<R>(), s, a));

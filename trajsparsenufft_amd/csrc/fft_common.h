@@ -16,7 +16,8 @@ struct FftArgs {
                            // launch, row width of the legacy grid layout
   const float2* tw0;       // W_K0^k, k < K0
   const float2* tw1;       // W_K1^k
-  const float2* image_t;   // [n1][n0]
+  const float2* image_t;   // pixel (n0, n1) at n0 * image_s0 + n1 * image_s1, as image_out, reg_in and dot_r
+  uint64_t image_s0, image_s1;
   const float2* smaps_t;   // [n1][coil][n0]
   const float* apod_t;     // [n1][n0]
   // Channel layouts (float2; see chunk_rows): t_fwd, t_inv and, with
@@ -31,8 +32,8 @@ struct FftArgs {
   const float2* grid;      // rows [K0*K1]
   float2* t_inv;           // rows [n1][K0]
   uint32_t grid_blocked;
-  float2* image_out;       // [n1][n0]
-  const float2* reg_in;    // [n1][n0] or null
+  float2* image_out;
+  const float2* reg_in;    // or null
   float lambda;
   float out_scale;
   double* dot_partial;     // [n1] partials of Re<reg_in, out>, or null

@@ -45,7 +45,7 @@ struct tsn_plan {
   uint32_t *pan_il = nullptr, *smp_il = nullptr;  // interleaved hi | res << 16 panels
   float2* y_rows = nullptr;                         // measurement rows [M][coils] (data consistency)
   float2 *pan32 = nullptr, *smp32 = nullptr, *grid = nullptr;
-  float2 *x = nullptr, *r = nullptr, *r2 = nullptr, *p = nullptr, *p2 = nullptr, *ap = nullptr, *tmp = nullptr;
+  float2 *x = nullptr, *r = nullptr, *r2 = nullptr, *p = nullptr, *p2 = nullptr, *ap = nullptr;
   // [3][image1] partials of <p, Ap>, Re<r, Ap>, <Ap, Ap> per image column (first: <b, b> in the third)
   double* partial = nullptr;
   // chunk slots and counters of the two directions' long groups, the plan's
@@ -90,6 +90,8 @@ FftArgs fft_args(const tsn_plan* pl) {
   a.tw1 = pl->tw1;
   a.smaps_t = pl->smaps_t;
   a.apod_t = pl->apod_t;
+  a.image_s0 = 1;  // column-major vectors
+  a.image_s1 = a.n0;
   a.t_fwd = pl->t_fwd;
   a.panel_il = pl->pan_il;
   a.panel32 = pl->pan32;
@@ -127,10 +129,17 @@ float grid_norm(const tsn_plan* pl) {
   return static_cast<float>(1.0 / std::sqrt(static_cast<double>(pl->cfg.grid0) * pl->cfg.grid1));
 }
 
-// p (column-major image) -> gridded panels
-int op_forward_grid(tsn_plan* pl, const float2* image_t, hipStream_t s) {
+// A caller's image, [n0][n1].
+void row_major(FftArgs& a) {
+  a.image_s0 = a.n1;
+  a.image_s1 = 1;
+}
+
+// a caller's image -> gridded panels
+int op_forward_grid(tsn_plan* pl, const float2* image, hipStream_t s) {
   FftArgs a = fft_args(pl);
-  a.image_t = image_t;
+  a.image_t = image;
+  row_major(a);
   return fft_forward(a, fft_out_kind(pl), s);
 }
 
@@ -163,25 +172,18 @@ int op_adjoint_grid(tsn_plan* pl, hipStream_t s) {
                        s, pl->panels, nullptr, &pl->adj_chunks);
 }
 
-// grid -> image (column-major) with combine, scale, regulariser, dot partial
-int op_adjoint_image(tsn_plan* pl, float2* out_t, const float2* reg, float lambda, float out_scale,
-                     double* dot_partial, hipStream_t s, const float2* dot_r = nullptr) {
+// grid -> image (column-major, or a caller's) with combine, scale, regulariser, dot partial
+int op_adjoint_image(tsn_plan* pl, float2* out, const float2* reg, float lambda, float out_scale,
+                     double* dot_partial, hipStream_t s, const float2* dot_r = nullptr, bool callers = false) {
   FftArgs a = fft_args(pl);
-  a.image_out = out_t;
+  if (callers) row_major(a);
+  a.image_out = out;
   a.reg_in = reg;
   a.lambda = lambda;
   a.out_scale = out_scale * grid_norm(pl);
   a.dot_partial = dot_partial;
   a.dot_r = dot_r;
   return fft_inverse(a, s);
-}
-
-int op_normal(tsn_plan* pl, const float2* in_t, float2* out_t, float inv_scale_sq, float lambda,
-              double* dot_partial, hipStream_t s) {
-  TSN_CHECK(op_forward_grid(pl, in_t, s));
-  TSN_CHECK(op_forward_samples(pl, nullptr, s));
-  TSN_CHECK(op_adjoint_grid(pl, s));
-  return op_adjoint_image(pl, out_t, in_t, lambda, inv_scale_sq, dot_partial, s);
 }
 
 // measurement (raw, coil-major) -> scaled sample panels of the adjoint input
@@ -195,13 +197,6 @@ int op_load_samples(tsn_plan* pl, const float2* samples, float scale, hipStream_
   }
   return launch_split_panel_il(samples, pl->m, pl->cfg.coils, scale, pl->smp_il, s,
                                is_bf16(pl) ? TSN_VALUES_BF16 : TSN_VALUES_FP16, pl->panels == kLines);
-}
-
-int transpose_image(const float2* in, uint32_t rows, uint32_t cols, float scale, float2* out, hipStream_t s) {
-  hipLaunchKernelGGL(transpose_kernel, dim3(div_up(cols, 32), div_up(rows, 32)), dim3(32, 8), 0, s, in,
-                     rows, cols, scale, out);
-  TSN_HIP(hipGetLastError());
-  return TSN_OK;
 }
 
 int enqueue_cg(tsn_plan* pl, const float2* measurement, uint32_t iterations, float operator_scale,
@@ -355,7 +350,7 @@ int tsn_plan_create(const tsn_plan_config* cfg, const tsn_direction* fwd, const 
     A(&pl->smp_il, static_cast<size_t>(pl->blocks) * pl->m * kN);
     A(&pl->y_rows, static_cast<size_t>(pl->m) * c.coils);
   }
-  for (float2** v : {&pl->x, &pl->r, &pl->r2, &pl->p, &pl->p2, &pl->ap, &pl->tmp}) A(v, px);
+  for (float2** v : {&pl->x, &pl->r, &pl->r2, &pl->p, &pl->p2, &pl->ap}) A(v, px);
   A(&pl->partial, 3 * static_cast<size_t>(c.image1));
   // slots: kSlotFloats floats per packed chunk, kMaxCoils float2 per CSR chunk
   const size_t slot_floats = fp32 ? 2 * kMaxCoils : kSlotFloats;
@@ -404,8 +399,7 @@ size_t tsn_plan_bytes(const tsn_plan* pl) { return pl ? pl->bytes : 0; }
 int tsn_forward(tsn_plan* pl, const void* image, void* samples, void* stream) {
   if (!pl || !image || !samples) return fail(TSN_ERR_ARGUMENT, "null argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  TSN_CHECK(transpose_image(static_cast<const float2*>(image), pl->cfg.image0, pl->cfg.image1, 1.0f, pl->tmp, s));
-  TSN_CHECK(op_forward_grid(pl, pl->tmp, s));
+  TSN_CHECK(op_forward_grid(pl, static_cast<const float2*>(image), s));
   return op_forward_samples(pl, static_cast<float2*>(samples), s);
 }
 
@@ -414,17 +408,19 @@ int tsn_adjoint(tsn_plan* pl, const void* samples, void* image, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   TSN_CHECK(op_load_samples(pl, static_cast<const float2*>(samples), 1.0f, s));
   TSN_CHECK(op_adjoint_grid(pl, s));
-  TSN_CHECK(op_adjoint_image(pl, pl->tmp, nullptr, 0.0f, 1.0f, nullptr, s));
-  return transpose_image(pl->tmp, pl->cfg.image1, pl->cfg.image0, 1.0f, static_cast<float2*>(image), s);
+  return op_adjoint_image(pl, static_cast<float2*>(image), nullptr, 0.0f, 1.0f, nullptr, s, nullptr, true);
 }
 
 int tsn_normal(tsn_plan* pl, const void* image, void* out, float inv_scale_sq, float scaled_lambda,
                void* stream) {
   if (!pl || !image || !out) return fail(TSN_ERR_ARGUMENT, "null argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  TSN_CHECK(transpose_image(static_cast<const float2*>(image), pl->cfg.image0, pl->cfg.image1, 1.0f, pl->tmp, s));
-  TSN_CHECK(op_normal(pl, pl->tmp, pl->ap, inv_scale_sq, scaled_lambda, nullptr, s));
-  return transpose_image(pl->ap, pl->cfg.image1, pl->cfg.image0, 1.0f, static_cast<float2*>(out), s);
+  // (out may be image: each pixel's lambda term is read by the thread that writes it)
+  TSN_CHECK(op_forward_grid(pl, static_cast<const float2*>(image), s));
+  TSN_CHECK(op_forward_samples(pl, nullptr, s));
+  TSN_CHECK(op_adjoint_grid(pl, s));
+  return op_adjoint_image(pl, static_cast<float2*>(out), static_cast<const float2*>(image), scaled_lambda, inv_scale_sq,
+                          nullptr, s, nullptr, true);
 }
 
 int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measurement, const float* density,
@@ -436,8 +432,7 @@ int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measuremen
   DcTerms dc;
   dc.density = density;
   dc.scale = measurement_scale;
-  TSN_CHECK(transpose_image(static_cast<const float2*>(image), pl->cfg.image0, pl->cfg.image1, 1.0f, pl->tmp, s));
-  TSN_CHECK(op_forward_grid(pl, pl->tmp, s));
+  TSN_CHECK(op_forward_grid(pl, static_cast<const float2*>(image), s));
   if (is_fp32(pl)) {
     // CSR forward into the FP32 sample rows, then the residual in place (y coil-major)
     dc.y = static_cast<const float*>(measurement);
@@ -459,8 +454,7 @@ int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measuremen
                                &pl->fwd_chunks, pl->panels));
   }
   TSN_CHECK(op_adjoint_grid(pl, s));
-  TSN_CHECK(op_adjoint_image(pl, pl->ap, nullptr, 0.0f, 1.0f, nullptr, s));
-  return transpose_image(pl->ap, pl->cfg.image1, pl->cfg.image0, 1.0f, static_cast<float2*>(out), s);
+  return op_adjoint_image(pl, static_cast<float2*>(out), nullptr, 0.0f, 1.0f, nullptr, s, nullptr, true);
 }
 
 int tsn_cg(tsn_plan* pl, const void* measurement, uint32_t iterations, float operator_scale, float lambda,
