@@ -131,15 +131,39 @@ __global__ __launch_bounds__(256) void fill_zero_kernel(float4* __restrict__ p, 
   if (e < n4) p[e] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// [coils][m] -> [m][coils] * scale (FP32 path sample layout)
+// [coils][m] -> [m][coils] * scale (FP32 path sample layout).  Memory bound: a
+// block turns 128 rows of all coils through LDS, so that a wave reads 512
+// contiguous bytes of a coil and writes 512 of the rows, with one 64-bit index
+// a block (a thread per output with its own 64-bit division and 64-byte reads:
+// 206 K rows of 8 coils 8.3 -> 6.5 us).  The pitch keeps the rows that 32
+// lanes read on banks of their own.
+constexpr uint32_t kRowTile = 128;
 __global__ __launch_bounds__(256) void samples_to_rows_kernel(const float2* __restrict__ in, uint32_t coils,
                                                               uint32_t m, float scale,
                                                               float2* __restrict__ out) {
-  const uint64_t e = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= static_cast<uint64_t>(coils) * m) return;
-  const uint32_t c = static_cast<uint32_t>(e % coils), row = static_cast<uint32_t>(e / coils);
-  const float2 v = in[static_cast<size_t>(c) * m + row];
-  out[e] = make_float2(v.x * scale, v.y * scale);
+  __shared__ float2 tile[tsn::kMaxCoils * kRowTile + 2 * 32];
+  const uint32_t row0 = blockIdx.x * kRowTile, rows = min(kRowTile, m - row0);
+  const uint32_t pitch = kRowTile + (32 + coils - 1) / coils;
+  const uint32_t r = threadIdx.x % kRowTile;
+#pragma unroll 4
+  for (uint32_t c = threadIdx.x / kRowTile; c < coils; c += 256 / kRowTile) {
+    if (r < rows) tile[c * pitch + r] = in[static_cast<size_t>(c) * m + row0 + r];
+  }
+  __syncthreads();
+  out += static_cast<size_t>(row0) * coils;
+  const uint32_t inv = 65536 / coils + 1;  // e / coils = e * inv >> 16 for e < 65536 / coils
+  for (uint32_t e = threadIdx.x; e < rows * coils; e += 256) {
+    const uint32_t row = (e * inv) >> 16, c = e - row * coils;
+    const float2 v = tile[c * pitch + row];
+    out[e] = make_float2(v.x * scale, v.y * scale);
+  }
+}
+
+inline int launch_samples_to_rows(const float2* in, uint32_t coils, uint32_t m, float scale, float2* out,
+                                  hipStream_t s) {
+  hipLaunchKernelGGL(samples_to_rows_kernel, dim3(div_up(m, kRowTile)), dim3(256), 0, s, in, coils, m, scale, out);
+  TSN_HIP(hipGetLastError());
+  return TSN_OK;
 }
 
 // a fill kernel (not hipMemsetAsync) so the work can sit inside a captured graph

@@ -189,11 +189,7 @@ int op_adjoint_image(tsn_plan* pl, float2* out, const float2* reg, float lambda,
 // measurement (raw, coil-major) -> scaled sample panels of the adjoint input
 int op_load_samples(tsn_plan* pl, const float2* samples, float scale, hipStream_t s) {
   if (is_fp32(pl)) {
-    const uint64_t n = static_cast<uint64_t>(pl->cfg.coils) * pl->m;
-    hipLaunchKernelGGL(samples_to_rows_kernel, dim3(div_up(n, 256)), dim3(256), 0, s, samples,
-                       pl->cfg.coils, pl->m, scale, pl->smp32);
-    TSN_HIP(hipGetLastError());
-    return TSN_OK;
+    return launch_samples_to_rows(samples, pl->cfg.coils, pl->m, scale, pl->smp32, s);
   }
   return launch_split_panel_il(samples, pl->m, pl->cfg.coils, scale, pl->smp_il, s,
                                is_bf16(pl) ? TSN_VALUES_BF16 : TSN_VALUES_FP16, pl->panels == kLines);
@@ -443,10 +439,7 @@ int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measuremen
     TSN_CHECK(launch_dc_residual_rows(pl->smp32, pl->m, coils, dc, s));
   } else {
     // y to rows (one 64-byte read per sample row in the epilogue), residual fused
-    const uint64_t n = static_cast<uint64_t>(coils) * pl->m;
-    hipLaunchKernelGGL(samples_to_rows_kernel, dim3(div_up(n, 256)), dim3(256), 0, s,
-                       static_cast<const float2*>(measurement), coils, pl->m, 1.0f, pl->y_rows);
-    TSN_HIP(hipGetLastError());
+    TSN_CHECK(launch_samples_to_rows(static_cast<const float2*>(measurement), coils, pl->m, 1.0f, pl->y_rows, s));
     dc.y = reinterpret_cast<const float*>(pl->y_rows);
     dc.row_stride = 2 * coils;
     dc.coil_stride = 2;
