@@ -321,7 +321,7 @@ __global__ __launch_bounds__(512) void inv_axis0_kernel(FftArgs args) {
   extern __shared__ float2 lds[];
   __shared__ double red[24];
   constexpr int K = 64 * R;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int w = threadIdx.x >> 6;
   // neighbouring columns on one XCD where their pixels share lines (a caller's
   // row-major image); column-major vectors have no such lines, and a solve's
   // pass takes 7.3 us in launch order against 7.8 us (256^2 / 8 coils)
@@ -340,19 +340,28 @@ __global__ __launch_bounds__(512) void inv_axis0_kernel(FftArgs args) {
   float2 acc = make_float2(0.f, 0.f);
   const uint32_t chunks = (a.coils + 7) / 8;
   for (uint32_t chunk = 0; chunk < chunks; ++chunk) {
+    // R = 12: an opaque lane keeps the loop's twiddles and addresses from being
+    // held in registers across it, and the maps are loaded behind the
+    // transform: 124 registers instead of 241 let two blocks share a compute
+    // unit (768^2 grid, 16 coils, 8 frames: 174 -> 151 us)
+    int lane = threadIdx.x & 63;
+    if constexpr (R > 8) asm volatile("" : "+v"(lane));
     const uint32_t cw = min(8u, a.coils - chunk * 8);
-    // conj(S_c[n0]) of the wave's outputs, loaded with the chunk's data
+    // conj(S_c[n0]) of the wave's outputs, loaded with the chunk's data (R <= 8)
     const uint32_t c = chunk * 8 + w;
     const float2* sm = a.smaps_t + (static_cast<size_t>(n1) * a.cstride + min(c, a.coils - 1)) * a.n0;
     float2 smv[TPL][4];
+    const auto load_maps = [&] {
 #pragma unroll
-    for (int s = 0; s < TPL; ++s) {
-      const int task = lane + 64 * s;
-      const int k1 = task >> 3, k2a = task & 7;
+      for (int s = 0; s < TPL; ++s) {
+        const int task = lane + 64 * s;
+        const int k1 = task >> 3, k2a = task & 7;
 #pragma unroll
-      for (int k2b = 0; k2b < 4; ++k2b)
-        smv[s][k2b] = task < R * 8 ? sm[k1 + R * (k2a + 8 * k2b)] : make_float2(0.f, 0.f);
-    }
+        for (int k2b = 0; k2b < 4; ++k2b)
+          smv[s][k2b] = task < R * 8 ? sm[k1 + R * (k2a + 8 * k2b)] : make_float2(0.f, 0.f);
+      }
+    };
+    if constexpr (R <= 8) load_maps();
     const ChunkRows tl = chunk_rows(a.coils, static_cast<uint64_t>(a.n1) * a.k0);
     fill_exchange<K>(a.t_inv + chunk * tl.cs + static_cast<size_t>(n1) * K * tl.rs, tl.rs, cw, lds);
     __syncthreads();
@@ -362,6 +371,7 @@ __global__ __launch_bounds__(512) void inv_axis0_kernel(FftArgs args) {
     __syncthreads();
     float2 out[TPL][8];
     wave_fft<R, true, false, true>(x, lds + w * wave_lds_elems<R>(), a.tw0, twp, lane, out);
+    if constexpr (R > 8) load_maps();
     // multiply by conj(S_c[n0]) before the coil sum
 #pragma unroll
     for (int s = 0; s < TPL; ++s) {

@@ -340,9 +340,26 @@ __device__ __forceinline__ void wave_lds_sync() {
 // banks (stride 65, 1 mod 32, made two lanes of each group share a bank);
 // pass C reads task * 9 + b0, consecutive tasks 9 apart.
 constexpr int kRowA = 72;
+//
+// R = 12 swizzles both layouts in 64-element rows instead (slot_a, slot_b: for
+// each access 32 neighbouring lanes still touch distinct banks): without the
+// padding a block holds 48 KB, and a compute unit's 160 KB three blocks
+// instead of two (768^2 grid, 16 coils, one problem: inv_axis0 34.4 -> 29.1,
+// inv_axis1 32.0 -> 30.1, fwd_axis1 30.6 -> 28.2 us).  The shorter radices have
+// four either way and keep the padding, whose addresses are base + constant.
 template <int R>
 __host__ __device__ constexpr int wave_lds_elems() {
-  return R * kRowA > R * 8 * 9 ? R * kRowA : R * 8 * 9;
+  return R > 8 ? R * 64 : R * kRowA > R * 8 * 9 ? R * kRowA : R * 8 * 9;
+}
+// element i = b0 + 8 b1 of pass A's row k1
+template <int R>
+__host__ __device__ constexpr int slot_a(int k1, int i) {
+  return R > 8 ? k1 * 64 + (i ^ ((k1 & 3) << 3)) : k1 * kRowA + i;
+}
+// element b0 of pass C's task (k1, k2a)
+template <int R>
+__host__ __device__ constexpr int slot_b(int k1, int k2a, int b0) {
+  return R > 8 ? k1 * 64 + ((k2a ^ (k1 & 3)) << 3) + (b0 ^ ((k2a & 6) | (k1 & 1))) : (k1 * 8 + k2a) * 9 + b0;
 }
 
 // Twiddles of one lane for wave_fft, loaded before the data so their latency
@@ -399,7 +416,7 @@ __device__ __forceinline__ void wave_fft(float2 (&x)[R], float2* buf, const floa
 #pragma unroll
   for (int k1 = 1; k1 < R; ++k1) y[k1] = twiddle<INV>(y[k1], R <= 8 ? twp.a[k1] : tw[lane * k1]);
 #pragma unroll
-  for (int k1 = 0; k1 < R; ++k1) buf[k1 * kRowA + lane] = y[k1];
+  for (int k1 = 0; k1 < R; ++k1) buf[slot_a<R>(k1, lane)] = y[k1];
   wave_lds_sync();
   // pass B: task (k1, b0): radix-8 over b1, twiddle W_64^{b0*k2a}
   float2 u[TPL][8];
@@ -409,7 +426,7 @@ __device__ __forceinline__ void wave_fft(float2 (&x)[R], float2* buf, const floa
     if (task < R * 8) {
       const int k1 = task >> 3, b0 = task & 7;
 #pragma unroll
-      for (int b1 = 0; b1 < 8; ++b1) u[s][b1] = buf[k1 * kRowA + b0 + 8 * b1];
+      for (int b1 = 0; b1 < 8; ++b1) u[s][b1] = buf[slot_a<R>(k1, b0 + 8 * b1)];
     }
   }
   wave_lds_sync();
@@ -423,7 +440,7 @@ __device__ __forceinline__ void wave_fft(float2 (&x)[R], float2* buf, const floa
 #pragma unroll
       for (int k2a = 1; k2a < 8; ++k2a) v[k2a] = twiddle<INV>(v[k2a], R <= 8 ? twp.b[k2a] : tw[R * b0 * k2a]);
 #pragma unroll
-      for (int k2a = 0; k2a < 8; ++k2a) buf[(k1 * 8 + k2a) * 9 + b0] = v[k2a];
+      for (int k2a = 0; k2a < 8; ++k2a) buf[slot_b<R>(k1, k2a, b0)] = v[k2a];
     }
   }
   wave_lds_sync();
@@ -434,7 +451,7 @@ __device__ __forceinline__ void wave_fft(float2 (&x)[R], float2* buf, const floa
     if (task < R * 8) {
       float2 v[8];
 #pragma unroll
-      for (int b0 = 0; b0 < 8; ++b0) v[b0] = buf[task * 9 + b0];
+      for (int b0 = 0; b0 < 8; ++b0) v[b0] = buf[slot_b<R>(task >> 3, task & 7, b0)];
       dft8<INV, 8>(v, out[s]);
     }
   }
