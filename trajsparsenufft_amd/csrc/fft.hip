@@ -46,7 +46,7 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   if (blockIdx.y * 8 >= a.coils) return;  // coil chunk beyond this problem (batched launches)
   extern __shared__ float2 lds[];
   __shared__ double red[24];
-  __shared__ float2 column[CG ? 1 : 32 * R];
+  __shared__ float2 column[32 * R];
   constexpr int K = 64 * R;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // neighbouring columns on one XCD: their 64-byte rows of T fill whole L2 lines
@@ -60,52 +60,46 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   // (branch-free: selected sources, a zero array for the absent ones, so no
   // wait is forced where branches would merge; threads past dot_count load
   // its last entry and drop it below)
-  // (a runtime test although CG launches always set cg_r: without the branch
-  // the compiler moves the update into the loads and takes 131 instead of 114
-  // registers at R = 8, three waves per SIMD instead of four)
-  const bool cg = CG && a.cg_r != nullptr;
-  const bool sums = cg || a.rho0_dots != nullptr;
+  const bool sums = CG || a.rho0_dots != nullptr;
   const uint32_t qi = sums ? min(threadIdx.x, a.dot_count - 1) : 0u;
-  const uint32_t qs = cg ? a.dot_count : 0u;
-  const double* q_src = cg ? a.cg_dots : (a.rho0_dots ? a.rho0_dots : kZeroPartials);
-  const double* q_more = cg ? a.cg_dots : kZeroPartials;
+  const uint32_t qs = CG ? a.dot_count : 0u;
+  const double* q_src = CG ? a.cg_dots : (a.rho0_dots ? a.rho0_dots : kZeroPartials);
+  const double* q_more = CG ? a.cg_dots : kZeroPartials;
   double q0 = gmem(q_src)[qi];
-  double q1 = gmem(q_more)[qs + (cg ? qi : 0u)];
-  double q2 = gmem(q_more)[2 * qs + (cg ? qi : 0u)];
-  const double rho_old = *gmem(cg ? a.rho_hist + (a.iter - 1) : kZeroPartials);
+  double q1 = gmem(q_more)[qs + (CG ? qi : 0u)];
+  double q2 = gmem(q_more)[2 * qs + (CG ? qi : 0u)];
+  const double rho_old = *gmem(CG ? a.rho_hist + (a.iter - 1) : kZeroPartials);
   __builtin_amdgcn_sched_barrier(0);  // keep these loads ahead of the data loads
-  const bool store_vec = chunk == 0 && w == 0;  // the wave that writes x, r and p_new
+  // the column's pixels, one a thread, for the block's eight coils: each wave
+  // forming the direction for itself took 9.1 instead of 8.3 us at 256^2 / 8
+  // coils, 180 instead of 138 us for 8 frames of 384^2 / 16 coils (106 instead
+  // of 88 registers), and rows of a row-major image are a line each
+  const bool pixel = threadIdx.x < a.n0;
+  const uint32_t row = min(threadIdx.x, a.n0 - 1);
+  const size_t pix = static_cast<size_t>(n1) * a.n0 + row;
+  float2 v = CG ? a.cg_r[pix] : a.image_t[row * a.image_s0 + n1 * a.image_s1];
+  float2 pv = make_float2(0.f, 0.f), av = pv, xv = pv;
+  if constexpr (CG) {
+    pv = a.cg_p_old[pix];
+    av = a.cg_ap[pix];
+    xv = (a.x_zero ? a.cg_p_old : a.cg_x)[pix];
+  }
   // Loads are unconditional, at clamped indices (straight-line code lets every
   // load issue before the first wait; a load under a lane-dependent branch
   // would be waited for at the branch's end); out-of-range values are zeroed
   // afterwards.  Only j < JN can hold pixels: N0 = K/2.
   constexpr int JN = R >= 2 ? R / 2 : 1;
-  const float2* src_r = cg ? a.cg_r : a.image_t;
-  const float2* src_p = cg ? a.cg_p_old : a.image_t;
-  const float2* src_a = cg ? a.cg_ap : a.image_t;
   const float2* src_s = a.smaps_t + (static_cast<size_t>(n1) * a.cstride + min(c, a.coils - 1)) * a.n0;
-  const bool x_wave = cg && !a.x_zero && __builtin_amdgcn_readfirstlane(store_vec ? 1 : 0);
-  float2 img[R], sm[R], pv[R], av[R], xv[R];
+  float2 img[R], sm[R];
   float ap[R];
-  // (one load of the column per block, shared by its eight coils: rows of a
-  // row-major image are a line each)
-  float2 pixel;
-  if constexpr (!CG) pixel = a.image_t[min(threadIdx.x, a.n0 - 1) * a.image_s0 + n1 * a.image_s1];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    img[j] = pv[j] = sm[j] = av[j] = xv[j] = make_float2(0.f, 0.f);
+    img[j] = sm[j] = make_float2(0.f, 0.f);
     ap[j] = 0.f;
     if (j >= JN) continue;
     const uint32_t n0 = min(lane + 64u * j, a.n0 - 1);
-    const size_t pix = static_cast<size_t>(n1) * a.n0 + n0;
-    if constexpr (CG) {
-      img[j] = src_r[pix];
-      pv[j] = src_p[pix];
-      av[j] = src_a[pix];
-    }
     sm[j] = src_s[n0];
-    ap[j] = a.apod_t[pix];
-    if (x_wave) xv[j] = a.cg_x[pix];
+    ap[j] = a.apod_t[static_cast<size_t>(n1) * a.n0 + n0];
   }
   // the partials' sums (every block, same order), while the data loads are in
   // flight: the previous step's <p, Ap>, Re<r, Ap>, <Ap, Ap>, or rho0 = <b, b>
@@ -114,30 +108,18 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
     if (threadIdx.x >= a.dot_count) q0 = q1 = q2 = 0.0;
     for (uint32_t i = threadIdx.x + 512; i < a.dot_count; i += 512) {
       q0 += gmem(q_src)[i];
-      if (cg) {
+      if (CG) {
         q1 += gmem(a.cg_dots)[a.dot_count + i];
         q2 += gmem(a.cg_dots)[2 * a.dot_count + i];
       }
     }
     block_sum3<8>(q0, q1, q2, red);
-    if (!cg && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    if (!CG && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
       a.rho_hist[0] = q0;
       *a.cg_status = 1;
     }
   }
-  if constexpr (!CG) {
-    if (threadIdx.x < a.n0) column[threadIdx.x] = pixel;
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < JN; ++j) {
-    if constexpr (!CG) img[j] = column[min(lane + 64u * j, a.n0 - 1)];
-    if (!active || lane + 64u * j >= a.n0) {
-      img[j] = pv[j] = sm[j] = av[j] = xv[j] = make_float2(0.f, 0.f);
-      ap[j] = 0.f;
-    }
-  }
-  if (cg) {
+  if constexpr (CG) {
     const double pap = q0, rap = q1, apap = q2;
     const bool first_block = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
     double alpha = 0.0;
@@ -146,19 +128,23 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
     const double rho_new = fmax(rho_old - 2.0 * alpha * rap + alpha * alpha * apap, 0.0);
     const double beta = rho_new / fmax(rho_old, 1e-30);
     if (first_block) a.rho_hist[a.iter] = rho_new;
+    const float2 r_new = make_float2(static_cast<float>(v.x - alpha * av.x), static_cast<float>(v.y - alpha * av.y));
+    v = make_float2(static_cast<float>(r_new.x + beta * pv.x), static_cast<float>(r_new.y + beta * pv.y));
+    if (chunk == 0 && pixel) {
+      if (a.x_zero) xv = make_float2(0.f, 0.f);
+      a.cg_x[pix] = make_float2(static_cast<float>(xv.x + alpha * pv.x), static_cast<float>(xv.y + alpha * pv.y));
+      a.cg_r_new[pix] = r_new;
+      a.cg_p_new[pix] = v;
+    }
+  }
+  if (pixel) column[threadIdx.x] = v;
+  __syncthreads();
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const uint32_t n0 = lane + 64 * j;
-      const float2 r_new = make_float2(static_cast<float>(img[j].x - alpha * av[j].x),
-                                       static_cast<float>(img[j].y - alpha * av[j].y));
-      img[j] = make_float2(static_cast<float>(r_new.x + beta * pv[j].x), static_cast<float>(r_new.y + beta * pv[j].y));
-      if (active && n0 < a.n0 && store_vec) {
-        const size_t pix = static_cast<size_t>(n1) * a.n0 + n0;
-        a.cg_x[pix] = make_float2(static_cast<float>(xv[j].x + alpha * pv[j].x),
-                                  static_cast<float>(xv[j].y + alpha * pv[j].y));
-        a.cg_r_new[pix] = r_new;
-        a.cg_p_new[pix] = img[j];
-      }
+  for (int j = 0; j < JN; ++j) {
+    img[j] = column[min(lane + 64u * j, a.n0 - 1)];
+    if (!active || lane + 64u * j >= a.n0) {
+      img[j] = sm[j] = make_float2(0.f, 0.f);
+      ap[j] = 0.f;
     }
   }
   float2 x[R];
