@@ -292,7 +292,8 @@ size_t tsn_plan_bytes(const tsn_plan* plan);
 int tsn_forward(tsn_plan* plan, const void* image, void* samples, void* stream);
 /* A^H y (exact adjoint of tsn_forward). */
 int tsn_adjoint(tsn_plan* plan, const void* samples, void* image, void* stream);
-/* (A^H A) x * inv_scale_sq + scaled_lambda * x (launch_normal). */
+/* (A^H A) x * inv_scale_sq + scaled_lambda * x (launch_normal); out may be
+ * image or overlap it at any offset. */
 int tsn_normal(tsn_plan* plan, const void* image, void* out, float inv_scale_sq,
                float scaled_lambda, void* stream);
 

@@ -126,6 +126,11 @@ __global__ __launch_bounds__(256) void apod_transpose_kernel(const float* __rest
   out[static_cast<size_t>(x1) * n0 + x0] = in[e];
 }
 
+__global__ __launch_bounds__(256) void copy_kernel(const float2* __restrict__ in, uint32_t n, float2* __restrict__ out) {
+  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n) out[e] = in[e];
+}
+
 __global__ __launch_bounds__(256) void fill_zero_kernel(float4* __restrict__ p, uint64_t n4) {
   const uint64_t e = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (e < n4) p[e] = make_float4(0.f, 0.f, 0.f, 0.f);

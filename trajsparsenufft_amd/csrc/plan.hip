@@ -411,12 +411,21 @@ int tsn_normal(tsn_plan* pl, const void* image, void* out, float inv_scale_sq, f
                void* stream) {
   if (!pl || !image || !out) return fail(TSN_ERR_ARGUMENT, "null argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // (out may be image: each pixel's lambda term is read by the thread that writes it)
-  TSN_CHECK(op_forward_grid(pl, static_cast<const float2*>(image), s));
+  const auto* x = static_cast<const float2*>(image);
+  // The last pass reads image again for the lambda term.  Where out is image,
+  // each pixel is read by the thread that writes it; where they overlap at an
+  // offset, the term comes from a copy (pl->ap is free outside a solve).
+  const auto at = reinterpret_cast<uintptr_t>(image), to = reinterpret_cast<uintptr_t>(out);
+  const bool offset_overlap = at != to && (at < to ? to - at : at - to) < pl->pixels * sizeof(float2);
+  TSN_CHECK(op_forward_grid(pl, x, s));
   TSN_CHECK(op_forward_samples(pl, nullptr, s));
   TSN_CHECK(op_adjoint_grid(pl, s));
-  return op_adjoint_image(pl, static_cast<float2*>(out), static_cast<const float2*>(image), scaled_lambda, inv_scale_sq,
-                          nullptr, s, nullptr, true);
+  if (offset_overlap) {
+    hipLaunchKernelGGL(copy_kernel, dim3(div_up(pl->pixels, 256)), dim3(256), 0, s, x, pl->pixels, pl->ap);
+    TSN_HIP(hipGetLastError());
+    x = pl->ap;
+  }
+  return op_adjoint_image(pl, static_cast<float2*>(out), x, scaled_lambda, inv_scale_sq, nullptr, s, nullptr, true);
 }
 
 int tsn_data_consistency(tsn_plan* pl, const void* image, const void* measurement, const float* density,
