@@ -82,7 +82,8 @@ __global__ __launch_bounds__(512) void fwd_axis0_kernel(FftArgs args) {
   if constexpr (CG) {
     pv = a.cg_p_old[pix];
     av = a.cg_ap[pix];
-    xv = (a.x_zero ? a.cg_p_old : a.cg_x)[pix];
+    // (x only where chunk 0 reads and stores it; a select of addresses, no branch)
+    xv = (chunk != 0 || a.x_zero ? a.cg_p_old : a.cg_x)[pix];
   }
   // Loads are unconditional, at clamped indices (straight-line code lets every
   // load issue before the first wait; a load under a lane-dependent branch

@@ -46,9 +46,9 @@ struct FftArgs {
   // (= ||r - alpha Ap||^2), beta = rho_new / max(rho_old, 1e-30); then
   // x += alpha p_old, r_new = r - alpha Ap, and the input is p_new = r_new +
   // beta p_old.  rho_hist[iter - 1] is read and rho_hist[iter] written by
-  // block (0, 0); coil chunk 0's first wave stores x (in place: it alone reads
-  // it), r_new and p_new (other buffers than r and p_old, which every chunk
-  // and wave of the column reads).
+  // block (0, 0); coil chunk 0 stores x (in place: it alone reads x, each pixel
+  // in the thread that stores it), r_new and p_new (other buffers than r and
+  // p_old, which every chunk of the column reads).
   const float2* cg_r;
   float2* cg_r_new;
   float2* cg_x;
