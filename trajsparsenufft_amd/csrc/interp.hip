@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <numeric>
@@ -1878,10 +1879,11 @@ bool tsn::csr_build(const std::vector<uint32_t>& ptr, const std::vector<int32_t>
   };
   const uint32_t threads = std::clamp(std::thread::hardware_concurrency(), 1u, parts);
   std::vector<std::thread> pool;
+  pool.reserve(threads);  // nothing may throw past a running helper
   try {
     for (uint32_t i = 1; i < threads; ++i) pool.emplace_back(work);
-  } catch (const std::system_error&) {
-    // fewer helpers
+  } catch (const std::system_error&) {  // fewer helpers
+  } catch (const std::bad_alloc&) {
   }
   work();
   for (std::thread& t : pool) t.join();
@@ -2450,9 +2452,7 @@ int tsn_direction_load(const char* real_dir, const char* imag_dir, tsn_direction
   return rc;
 }
 
-int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
-  if (!kb || !out || (view != 0 && view != 1)) return fail(TSN_ERR_ARGUMENT, "bad argument");
-  *out = nullptr;
+static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   const uint32_t m = kb->rows, w = kb->width;
   const uint32_t grid = kb->grid0 * kb->grid1;
   std::vector<uint32_t> ptr;
@@ -2578,7 +2578,8 @@ int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** 
   }
   if (host.slots > kMaxCsrSlots)
     return fail(TSN_ERR_ARGUMENT, "%u long-row chunks (at most %u)", host.slots, kMaxCsrSlots);
-  auto* d = new tsn_direction();
+  std::unique_ptr<tsn_direction, void (*)(tsn_direction*)> owner(new tsn_direction(), release);
+  tsn_direction* d = owner.get();
   d->h = h;
   d->csr = true;
   (void)hipGetDevice(&d->device);
@@ -2617,13 +2618,20 @@ int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** 
     rc = device_copy(zeros.data(), zeros.size(), &d->partials, &bytes);
     if (rc == TSN_OK) rc = device_copy(zero_counters.data(), zero_counters.size(), &d->counters, &bytes);
   }
-  if (rc != TSN_OK) {
-    release(d);
-    return rc;
-  }
+  if (rc != TSN_OK) return rc;
   d->bytes = bytes;
-  *out = d;
+  *out = owner.release();
   return TSN_OK;
+}
+
+int tsn_direction_upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
+  if (!kb || !out || (view != 0 && view != 1)) return fail(TSN_ERR_ARGUMENT, "bad argument");
+  *out = nullptr;
+  try {
+    return upload_csr(kb, view, out);
+  } catch (const std::bad_alloc&) {
+    return fail(TSN_ERR_RUNTIME, "out of host memory");
+  }
 }
 
 int tsn_direction_header(const tsn_direction* d, tsn_pack_header* out) {
