@@ -26,12 +26,16 @@ constexpr int kSplitAboveTiles = 16;  // tiles per unit at most; longer groups a
 constexpr uint32_t kDefaultCoilWaves = 1;
 // FP32 path (interp_csr_kernel): distinct input rows of a round's LDS stage
 // (row 0 of the 256 is zero), entries of a short row (one quad, entry order)
-// and of a chunk of a longer one, rows of a run of empty rows, ranges of rows
-// that csr_build works on side by side (at most, and their entries at least).
+// and of a chunk of a longer one, rows of a run of empty rows, compute units
+// that a direction's blocks should cover, blocks up to which a launch splits the
+// coils, ranges of rows that csr_build works on side by side (at most, and their
+// entries at least).
 constexpr uint32_t kCsrCols = 255;
 constexpr uint32_t kCsrShortEntries = 64;
 constexpr uint32_t kCsrChunkEntries = 256;
 constexpr uint32_t kCsrEmptyRunRows = 64;
+constexpr uint32_t kCsrUnits = 256;
+constexpr uint32_t kCsrFewBlocks = 512;
 constexpr uint32_t kCsrParts = 16;
 constexpr uint32_t kCsrPartEntries = 1u << 15;
 // Device column words of packed tiles hold column * 32 (a byte offset) below
