@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <cstdlib>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -1559,8 +1560,7 @@ static int device_copy(const T* host, size_t count, T** out, size_t* bytes) {
 static void release(tsn_direction* d) {
   if (!d) return;
   void* ptrs[] = {d->group_offsets, d->group_rows, d->tile_cols, d->tile_a, d->tile_idx,
-                  d->tile_dense, d->items, d->order, d->chunks, d->partials, d->counters, d->row_ids,
-                  d->csr_cols, d->vals, d->csr_idx, d->csr_rounds, d->csr_blocks};
+                  d->tile_dense, d->items, d->order, d->chunks, d->partials, d->counters, d->csr_data};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (void* p : d->retired) (void)hipFree(p);
@@ -1686,107 +1686,218 @@ static int schedule_units(tsn_direction* d, uint32_t unit_tiles) {
 
 namespace {
 
-// One lane quad of an FP32 block: entries base + stride i, i < count.
+// The entries of an FP32 direction's rows, ascending columns: G as the matrix
+// holds them, or its transpose.  (Plain pointers: loops copy a view, so that
+// their stores cannot alias it.)
+struct CsrForward {
+  uint32_t width;
+  const int32_t* cols;
+  const float *re, *im;
+  uint32_t begin(uint32_t t) const { return t * width; }
+  uint32_t column(uint32_t e) const { return static_cast<uint32_t>(cols[e]); }
+  float2 value(uint32_t e) const { return make_float2(re[e], im[e]); }
+};
+struct CsrTranspose {
+  struct Entry {
+    uint32_t sample, at;  // column, and the entry's place in the matrix
+  };
+  const uint32_t* ptr;
+  const Entry* entries;
+  const float *re, *im;
+  uint32_t begin(uint32_t t) const { return ptr[t]; }
+  uint32_t column(uint32_t e) const { return entries[e].sample; }
+  float2 value(uint32_t e) const { return make_float2(re[entries[e].at], im[entries[e].at]); }
+};
+
+// One lane quad of an FP32 block: entries base + stride i, i < count, whose
+// columns' numbers in uniq are at local + stride i of the block's list.
 struct CsrQuad {
-  uint32_t base, stride, count;
+  uint32_t base, stride, count, local;
 };
 
 // Builds the blocks of one range of a direction's rows (csr_build).
+template <typename View>
 struct CsrBuilder {
-  const std::vector<uint32_t>& ptr;
-  const std::vector<int32_t>& cols;
-  const std::vector<float2>& vals;
+  // the group that last named a column, and its number there
+  struct Slot {
+    uint32_t group, place;
+  };
+  const View view;
   const std::vector<int32_t>& rows;
   uint32_t short_rows, long_rows;  // rows of a block of either kind, at most
+  Slot* slots;                     // [n_cols]
+  uint32_t group = 1;
   tsn::CsrHost h;
-  std::vector<uint32_t> mark, place;  // group that last named a column; its index in uniq
-  std::vector<uint32_t> uniq;
-  uint32_t group = 0;
+  // the group's entries and their columns' numbers, its columns as first named
+  // (one place more: name() writes before it knows), their place in ascending order
+  static constexpr uint32_t kEntries = 65 * tsn::kCsrShortEntries;
+  static_assert(16 * tsn::kCsrChunkEntries <= kEntries, "entries of a group of long rows");
+  uint32_t n_local = 0, n_uniq = 0;
+  std::vector<uint16_t> local = std::vector<uint16_t>(kEntries), rank = std::vector<uint16_t>(kEntries);
+  std::vector<uint32_t> uniq = std::vector<uint32_t>(kEntries + 1);
 
-  // The distinct columns of entries [b, e) that the group has not named yet.
-  uint32_t fresh(uint32_t b, uint32_t e) const {
-    uint32_t n = 0;
-    for (uint32_t k = b; k < e; ++k) n += mark[cols[k]] != group;
-    return n;
-  }
-  void name(uint32_t b, uint32_t e) {
-    for (uint32_t k = b; k < e; ++k)
-      if (mark[cols[k]] != group) {
-        mark[cols[k]] = group;
-        uniq.push_back(static_cast<uint32_t>(cols[k]));
-      }
+  uint32_t length(uint32_t t) const { return view.begin(t + 1) - view.begin(t); }
+
+  // Names entries [b, e) in the group; where their first is in local.  (Without
+  // a branch: whether a column is new is a coin toss.)
+  uint32_t name(uint32_t b, uint32_t e) {
+    const View v = view;
+    const uint32_t at = n_local, g = group;
+    Slot* const table = slots;
+    uint16_t* to = local.data() + at;
+    uint32_t* const named = uniq.data();
+    uint32_t n = n_uniq;
+    for (uint32_t k = b; k < e; ++k) {
+      const uint32_t c = v.column(k);
+      const Slot s = table[c];
+      const bool fresh = s.group != g;
+      const uint32_t place = fresh ? n : s.place;
+      table[c] = {g, place};
+      named[n] = c;
+      n += fresh;
+      *to++ = static_cast<uint16_t>(place);
+    }
+    n_uniq = n;
+    n_local = at + (e - b);
+    return at;
   }
 
   // One block of the quads (16 to a wave), whose entries name the columns uniq.
   void emit(tsn::CsrBlock b, const CsrQuad* quads, uint32_t n_quads) {
-    std::sort(uniq.begin(), uniq.end());
-    const uint32_t u = static_cast<uint32_t>(uniq.size());
-    for (uint32_t i = 0; i < u; ++i) place[uniq[i]] = i;
-    b.n_rounds = tsn::div_up(u, tsn::kCsrCols);
+    b.n_rounds = tsn::div_up(n_uniq, tsn::kCsrCols);
     b.round0 = static_cast<uint32_t>(h.rounds.size());
-    uint32_t at[64] = {};
-    for (uint32_t k = 0; k < b.n_rounds; ++k) {
-      const uint32_t u0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * k / b.n_rounds);
-      const uint32_t u1 = static_cast<uint32_t>(static_cast<uint64_t>(u) * (k + 1) / b.n_rounds);
-      tsn::CsrRound rd{};
-      rd.col0 = static_cast<uint32_t>(h.cols.size());
-      rd.n_cols = u1 - u0;
-      h.cols.insert(h.cols.end(), uniq.begin() + u0, uniq.begin() + u1);
-      rd.ent0 = static_cast<uint32_t>(h.vals.size() / 64);
-      rd.idx0 = static_cast<uint32_t>(h.idx.size() / 64);
-      for (uint32_t w = 0; w < 4; ++w) {
-        const uint32_t q0 = 16 * w, q1 = std::min(n_quads, q0 + 16);
-        // entry i of a quad sits at step i / 4 - at / 4, lane i mod 4 of the quad
-        uint32_t end[16] = {}, n = 0;
-        for (uint32_t q = q0; q < q1; ++q) {
-          const CsrQuad& qd = quads[q];
-          uint32_t i = at[q];
-          if (u1 == u) i = qd.count;
-          else
-            while (i < qd.count && place[cols[qd.base + qd.stride * i]] < u1) ++i;
-          end[q - q0] = i;
-          if (i > at[q]) n = std::max(n, (i - 1) / 4 - at[q] / 4 + 1);
-        }
-        rd.steps |= n << (8 * w);
-        const size_t v0 = h.vals.size(), i0 = h.idx.size();
-        h.vals.resize(v0 + static_cast<size_t>(n) * 64, make_float2(0.f, 0.f));
-        h.idx.resize(i0 + static_cast<size_t>(tsn::div_up(n, 4)) * 64, 0u);
-        for (uint32_t q = q0; q < q1; ++q) {
-          const CsrQuad& qd = quads[q];
-          const uint32_t first = at[q] / 4;
-          for (uint32_t i = at[q]; i < end[q - q0]; ++i) {
-            const uint32_t e = qd.base + qd.stride * i, t = i / 4 - first, lane = (q - q0) * 4 + (i & 3u);
-            h.vals[v0 + static_cast<size_t>(t) * 64 + lane] = vals[e];
-            h.idx[i0 + static_cast<size_t>(t / 4) * 64 + lane] |= (place[cols[e]] - u0 + 1) << (8 * (t & 3u));
-          }
-          at[q] = end[q - q0];
-        }
-      }
-      if (k == 0) b.first = rd;
-      else h.rounds.push_back(rd);
-    }
+    if (b.n_rounds == 1) b.first = one_round(quads, n_quads);
+    else if (b.n_rounds > 1) b.first = rounds(b.n_rounds, quads, n_quads);
     h.blocks.push_back(b);
-    uniq.clear();
+    n_uniq = n_local = 0;
     ++group;
   }
 
-  uint32_t length(uint32_t t) const { return ptr[t + 1] - ptr[t]; }
+  // The wave's n steps, entry i of a quad at step i / 4 and lane i mod 4 of it.
+  struct Wave {
+    float2* vals;
+    uint8_t* idx;  // one byte a step
+    float2& value(uint32_t q, uint32_t i) { return vals[(i / 4) * 64 + q * 4 + (i & 3u)]; }
+    uint8_t& column(uint32_t q, uint32_t i) { return idx[((i / 16) * 64 + q * 4 + (i & 3u)) * 4 + (i / 4 & 3u)]; }
+  };
+  Wave wave(uint32_t n) {
+    const size_t words = static_cast<size_t>(tsn::div_up(n, 4)) * 64;
+    const Wave w{h.vals.grow(static_cast<size_t>(n) * 64), reinterpret_cast<uint8_t*>(h.idx.grow(words))};
+    std::memset(w.idx, 0, words * 4);
+    return w;
+  }
+  tsn::CsrRound round_at(uint32_t u0, uint32_t u1) {
+    tsn::CsrRound rd{};
+    rd.col0 = static_cast<uint32_t>(h.cols.size());
+    rd.n_cols = u1 - u0;
+    rd.ent0 = static_cast<uint32_t>(h.vals.size() / 64);
+    rd.idx0 = static_cast<uint32_t>(h.idx.size() / 64);
+    h.cols.insert(h.cols.end(), uniq.begin() + u0, uniq.begin() + u1);
+    return rd;
+  }
+
+  // All columns in one round, in the order in which they were named.
+  tsn::CsrRound one_round(const CsrQuad* quads, uint32_t n_quads) {
+    const View v = view;
+    tsn::CsrRound rd = round_at(0, n_uniq);
+    for (uint32_t q0 = 0; q0 < n_quads; q0 += 16) {
+      const uint32_t in_wave = std::min(n_quads - q0, 16u);
+      uint32_t n = 0;
+      for (uint32_t q = 0; q < in_wave; ++q) n = std::max(n, tsn::div_up(quads[q0 + q].count, 4));
+      if (n == 0) continue;
+      rd.steps |= n << (q0 / 2);  // byte q0 / 16
+      Wave w = wave(n);
+      for (uint32_t q = 0; q < 16; ++q) {
+        const CsrQuad qd = q < in_wave ? quads[q0 + q] : CsrQuad{};
+        const uint16_t* from = local.data() + qd.local;
+        uint32_t e = qd.base, i = 0;
+        auto put = [&, v, stride = qd.stride](float2* value, uint8_t* column) {
+          *value = v.value(e);
+          *column = static_cast<uint8_t>(*from + 1);
+          e += stride;
+          from += stride;
+        };
+        for (; i + 4 <= qd.count; i += 4)
+          for (uint32_t l = 0; l < 4; ++l) put(&w.value(q, i) + l, &w.column(q, i) + 4 * l);
+        for (; i < qd.count; ++i) put(&w.value(q, i), &w.column(q, i));
+        for (; i < 4 * n; ++i) w.value(q, i) = make_float2(0.f, 0.f);  // (and local column 0)
+      }
+    }
+    return rd;
+  }
+
+  // The columns in ascending order cut into n_rounds rounds: a quad's entries
+  // (ascending too) follow the rounds.  The first round; the rest in h.rounds.
+  tsn::CsrRound rounds(uint32_t n_rounds, const CsrQuad* quads, uint32_t n_quads) {
+    const uint32_t u = n_uniq;
+    std::sort(uniq.begin(), uniq.begin() + u);
+    for (uint32_t i = 0; i < u; ++i) rank[slots[uniq[i]].place] = static_cast<uint16_t>(i);
+    tsn::CsrRound head{};
+    uint32_t at[64] = {};
+    for (uint32_t k = 0; k < n_rounds; ++k) {
+      const uint32_t u0 = static_cast<uint32_t>(static_cast<uint64_t>(u) * k / n_rounds);
+      const uint32_t u1 = static_cast<uint32_t>(static_cast<uint64_t>(u) * (k + 1) / n_rounds);
+      tsn::CsrRound rd = round_at(u0, u1);
+      for (uint32_t q0 = 0; q0 < n_quads; q0 += 16) {
+        const uint32_t in_wave = std::min(n_quads - q0, 16u);
+        // a quad's entries at .. end of this round, from step 0 on (lane i mod 4)
+        uint32_t end[16] = {}, n = 0;
+        for (uint32_t q = 0; q < in_wave; ++q) {
+          const CsrQuad& qd = quads[q0 + q];
+          uint32_t i = at[q0 + q];
+          while (i < qd.count && rank[local[qd.local + qd.stride * i]] < u1) ++i;
+          end[q] = i;
+          if (i > at[q0 + q]) n = std::max(n, (i - 1) / 4 - at[q0 + q] / 4 + 1);
+        }
+        if (n == 0) continue;
+        rd.steps |= n << (q0 / 2);
+        Wave w = wave(n);
+        std::fill_n(w.vals, static_cast<size_t>(n) * 64, make_float2(0.f, 0.f));
+        for (uint32_t q = 0; q < in_wave; ++q) {
+          const CsrQuad& qd = quads[q0 + q];
+          const uint32_t s0 = at[q0 + q] & ~3u;
+          for (uint32_t i = at[q0 + q]; i < end[q]; ++i) {
+            w.value(q, i - s0) = view.value(qd.base + qd.stride * i);
+            w.column(q, i - s0) = static_cast<uint8_t>(rank[local[qd.local + qd.stride * i]] - u0 + 1);
+          }
+          at[q0 + q] = end[q];
+        }
+      }
+      if (k == 0) head = rd;
+      else h.rounds.push_back(rd);
+    }
+    return head;
+  }
 
   // The rows of perm[lo .. hi): long rows and short rows each form groups of
   // consecutive rows, the long ones (blocks of several rounds) first.
   void build(const std::vector<uint32_t>& perm, uint32_t lo, uint32_t hi) {
-    std::vector<uint32_t> small, large;
+    struct Row {
+      uint32_t row, length, local;
+    };
+    std::vector<Row> small;
+    std::vector<uint32_t> large;
     CsrQuad quads[64];
+    // (about a fifth of the steps' lanes hold no entry)
+    size_t entries = 0;
+    for (uint32_t i = lo; i < hi; ++i) entries += length(perm[i]);
+    h.vals.reserve(entries + entries / 4);
+    h.idx.reserve(entries / 4 + entries / 16);
     auto flush_small = [&]() {
       if (small.empty()) return;
       // longest first, so that the 16 rows of a wave are of similar length
-      std::stable_sort(small.begin(), small.end(), [&](uint32_t p, uint32_t q) { return length(p) > length(q); });
+      // (stable, by counting)
+      uint32_t first[tsn::kCsrShortEntries + 2] = {};
+      for (const Row& r : small) ++first[tsn::kCsrShortEntries - r.length + 1];
+      for (uint32_t i = 1; i < tsn::kCsrShortEntries + 2; ++i) first[i] += first[i - 1];
       tsn::CsrBlock b{};
       b.row0 = static_cast<uint32_t>(h.row_ids.size());
       b.n_rows = static_cast<uint32_t>(small.size());
-      for (uint32_t r = 0; r < b.n_rows; ++r) {
-        h.row_ids.push_back(rows[small[r]]);
-        quads[r] = {ptr[small[r]], 1, length(small[r])};
+      h.row_ids.resize(b.row0 + b.n_rows);
+      for (const Row& r : small) {
+        const uint32_t q = first[tsn::kCsrShortEntries - r.length]++;
+        h.row_ids[b.row0 + q] = rows[r.row];
+        quads[q] = {view.begin(r.row), 1, r.length, r.local};
       }
       emit(b, quads, b.n_rows);
       small.clear();
@@ -1807,11 +1918,11 @@ struct CsrBuilder {
       for (uint32_t c = 0; c < b.n_chunks; ++c) {
         b.chunk = c;
         for (uint32_t r = 0; r < b.n_rows; ++r) {
-          const uint32_t n = length(large[r]), t = ptr[large[r]];
+          const uint32_t n = length(large[r]), t = view.begin(large[r]);
           const uint32_t e0 = t + static_cast<uint32_t>(static_cast<uint64_t>(n) * c / b.n_chunks);
           const uint32_t e1 = t + static_cast<uint32_t>(static_cast<uint64_t>(n) * (c + 1) / b.n_chunks);
-          name(e0, e1);
-          for (uint32_t p = 0; p < 4; ++p) quads[4 * r + p] = {e0 + p, 4, (e1 - e0 + 3 - p) / 4};
+          const uint32_t at = name(e0, e1);
+          for (uint32_t p = 0; p < 4; ++p) quads[4 * r + p] = {e0 + p, 4, (e1 - e0 + 3 - p) / 4, at + p};
         }
         emit(b, quads, 4 * b.n_rows);
       }
@@ -1829,9 +1940,15 @@ struct CsrBuilder {
     for (uint32_t i = lo; i < hi; ++i) {
       const uint32_t t = perm[i], n = length(t);
       if (n > tsn::kCsrShortEntries) continue;
-      if (small.size() == short_rows || uniq.size() + fresh(ptr[t], ptr[t + 1]) > tsn::kCsrCols) flush_small();
-      name(ptr[t], ptr[t + 1]);
-      small.push_back(t);
+      if (small.size() == short_rows) flush_small();
+      const uint32_t named = n_uniq;
+      uint32_t at = name(view.begin(t), view.begin(t) + n);
+      if (n_uniq > tsn::kCsrCols && !small.empty()) {  // the row starts the next block
+        n_uniq = named;
+        flush_small();  // (and with it the row's names)
+        at = name(view.begin(t), view.begin(t) + n);
+      }
+      small.push_back({t, n, at});
     }
     flush_small();
   }
@@ -1877,40 +1994,42 @@ static void csr_balance(std::vector<tsn::CsrBlock>* blocks, const std::vector<ts
   }
 }
 
-// Blocks of an FP32 direction.  Rows in the order `perm` (entries of row t:
-// ptr[t] .. ptr[t + 1] of cols and vals, ascending columns), cut into
-// up to kCsrParts ranges built side by side (false: out of memory).  In a range, short rows form groups of
-// up to 64 rows naming at most kCsrCols distinct columns (one round), long rows
-// groups of up to 16 rows of equally many chunks, one block per chunk.
-bool tsn::csr_build(const std::vector<uint32_t>& ptr, const std::vector<int32_t>& cols,
-                    const std::vector<float2>& vals, const std::vector<int32_t>& rows,
-                    const std::vector<uint32_t>& perm, uint32_t n_cols, std::vector<CsrHost>* out) {
+// Blocks of an FP32 direction: the rows of the view in the order `perm` (row t
+// is output row rows[t]), cut into up to kCsrParts ranges built side by side
+// (false: out of memory).  In a range, short rows form groups of up to 64 rows
+// naming at most kCsrCols distinct columns (one round), long rows groups of up
+// to 16 rows of equally many chunks, one block per chunk.
+template <typename View>
+static bool csr_build(const View& view, const std::vector<int32_t>& rows, const std::vector<uint32_t>& perm,
+                      uint32_t entries, uint32_t n_cols, std::vector<tsn::CsrHost>* out) {
   const uint32_t n = static_cast<uint32_t>(perm.size());
   // a range holds at least kCsrPartEntries entries: smaller ones cost more in
   // groups cut short at their ends and in threads than they save
-  const uint32_t parts = static_cast<uint32_t>(
-      std::clamp<size_t>(cols.size() / kCsrPartEntries, 1, kCsrParts));
-  out->assign(parts, CsrHost{});
+  const uint32_t parts = std::clamp(entries / tsn::kCsrPartEntries, 1u, tsn::kCsrParts);
+  out->clear();
+  out->resize(parts);
   // blocks hold fewer rows where full ones would not give every compute unit
   // one, down to one wave's quads (24 x 64 samples, 32^2 image, 8 coils: a solve
   // of 6 steps 190 -> 187 us)
   uint32_t n_long = 0;
-  for (uint32_t t = 0; t < n; ++t) n_long += ptr[t + 1] - ptr[t] > kCsrShortEntries;
-  const uint32_t short_rows = std::clamp((n - n_long) / kCsrUnits / 16 * 16, 16u, 64u);
-  const uint32_t long_rows = std::clamp(n_long / kCsrUnits / 4 * 4, 4u, 16u);
+  for (uint32_t t = 0; t < n; ++t) n_long += view.begin(t + 1) - view.begin(t) > tsn::kCsrShortEntries;
+  const uint32_t short_rows = std::clamp((n - n_long) / tsn::kCsrUnits / 16 * 16, 16u, 64u);
+  const uint32_t long_rows = std::clamp(n_long / tsn::kCsrUnits / 4 * 4, 4u, 16u);
   std::atomic<uint32_t> next{0};
   std::atomic<bool> done{true};
+  using Builder = CsrBuilder<View>;
   auto work = [&]() {
     try {
-      std::vector<uint32_t> mark(n_cols, 0xFFFFFFFFu), place(n_cols, 0u);
-      uint32_t group = 0;
+      // (zeros from calloc: only the pages that the thread's rows name are ever touched)
+      std::unique_ptr<typename Builder::Slot, decltype(&std::free)> slots(
+          static_cast<typename Builder::Slot*>(std::calloc(n_cols, sizeof(typename Builder::Slot))), &std::free);
+      if (!slots) throw std::bad_alloc();
+      uint32_t group = 1;
       for (uint32_t k; (k = next++) < parts;) {
-        CsrBuilder b{ptr, cols, vals, rows, short_rows, long_rows, {}, std::move(mark), std::move(place), {}, group};
+        Builder b{view, rows, short_rows, long_rows, slots.get(), group};
         b.build(perm, static_cast<uint32_t>(static_cast<uint64_t>(n) * k / parts),
                 static_cast<uint32_t>(static_cast<uint64_t>(n) * (k + 1) / parts));
         (*out)[k] = std::move(b.h);
-        mark = std::move(b.mark);
-        place = std::move(b.place);
         group = b.group;
       }
     } catch (const std::bad_alloc&) {
@@ -2492,12 +2611,28 @@ int tsn_direction_load(const char* real_dir, const char* imag_dir, tsn_direction
   return rc;
 }
 
+// The indices of the keys in ascending order, equal keys in order of index
+// (by counting, 11 bits at a time).
+static std::vector<uint32_t> stable_order(const std::vector<uint32_t>& key) {
+  std::vector<uint32_t> order(key.size()), next(key.size());
+  std::iota(order.begin(), order.end(), 0u);
+  const uint32_t most = key.empty() ? 0 : *std::max_element(key.begin(), key.end());
+  for (uint32_t shift = 0; shift < 32 && most >> shift; shift += 11) {
+    uint32_t first[2049] = {};
+    for (uint32_t k : key) ++first[(k >> shift & 2047u) + 1];
+    for (uint32_t d = 1; d < 2049; ++d) first[d] += first[d - 1];
+    for (uint32_t i : order) next[first[key[i] >> shift & 2047u]++] = i;
+    order.swap(next);
+  }
+  return order;
+}
+
 static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   const uint32_t m = kb->rows, w = kb->width;
   const uint32_t grid = kb->grid0 * kb->grid1;
   std::vector<uint32_t> ptr;
-  std::vector<int32_t> rows, cols;
-  std::vector<float2> vals;
+  std::vector<int32_t> rows;
+  std::vector<CsrTranspose::Entry> entries;
   tsn_pack_header h{};
   h.magic = kMagic;
   h.version = kVersion;
@@ -2506,13 +2641,8 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   h.k_tile = kK;
   h.nnz = m * w;
   if (view == 0) {
-    ptr.resize(m + 1);
-    for (uint32_t i = 0; i <= m; ++i) ptr[i] = i * w;
     rows.resize(m);
     std::iota(rows.begin(), rows.end(), 0);
-    cols = kb->cols;
-    vals.resize(static_cast<size_t>(m) * w);
-    for (size_t k = 0; k < vals.size(); ++k) vals[k] = make_float2(kb->re[k], kb->im[k]);
     h.output_size = m;
     h.n_cols = grid;
     h.active_rows = m;
@@ -2522,24 +2652,16 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
     for (int32_t c : kb->cols) ++count[c + 1];
     std::vector<uint32_t> start(grid + 1, 0);
     for (uint32_t g = 0; g < grid; ++g) start[g + 1] = start[g] + count[g + 1];
-    std::vector<int32_t> tcols(static_cast<size_t>(m) * w);
-    std::vector<float2> tvals(tcols.size());
+    entries.resize(static_cast<size_t>(m) * w);
     std::vector<uint32_t> fill(start.begin(), start.end() - 1);
-    for (uint32_t i = 0; i < m; ++i)
-      for (uint32_t j = 0; j < w; ++j) {
-        const size_t k = static_cast<size_t>(i) * w + j;
-        const uint32_t pos = fill[kb->cols[k]]++;
-        tcols[pos] = static_cast<int32_t>(i);
-        tvals[pos] = make_float2(kb->re[k], kb->im[k]);
-      }
+    for (uint32_t i = 0, k = 0; i < m; ++i)
+      for (uint32_t j = 0; j < w; ++j, ++k) entries[fill[kb->cols[k]]++] = {i, k};
     ptr.push_back(0);
     for (uint32_t g = 0; g < grid; ++g) {
       if (count[g + 1] == 0) continue;
       rows.push_back(static_cast<int32_t>(g));
       ptr.push_back(start[g + 1]);
     }
-    cols.swap(tcols);
-    vals.swap(tvals);
     h.output_size = grid;
     h.n_cols = m;
     h.active_rows = static_cast<uint32_t>(rows.size());
@@ -2548,25 +2670,21 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   // coordinate; grid points: their own): a block's rows share columns, and the
   // contiguous range of blocks each XCD runs covers a compact k-space region
   // whose input rows stay in that XCD's L2.
-  std::vector<uint32_t> perm;
-  {
-    const uint32_t n = static_cast<uint32_t>(rows.size());
-    std::vector<uint32_t> key(n);
-    for (uint32_t t = 0; t < n; ++t) {
-      if (view == 0) {
-        const double c0 = std::nearbyint(kb->coord0[t]), c1 = std::nearbyint(kb->coord1[t]);
-        key[t] = morton_key(static_cast<uint32_t>(std::max(0.0, c0)), static_cast<uint32_t>(std::max(0.0, c1)));
-      } else {
-        const uint32_t g = static_cast<uint32_t>(rows[t]);
-        key[t] = morton_key(g % kb->grid1, g / kb->grid1);
-      }
+  const uint32_t n = static_cast<uint32_t>(rows.size());
+  std::vector<uint32_t> key(n);
+  for (uint32_t t = 0; t < n; ++t) {
+    if (view == 0) {
+      const double c0 = std::nearbyint(kb->coord0[t]), c1 = std::nearbyint(kb->coord1[t]);
+      key[t] = morton_key(static_cast<uint32_t>(std::max(0.0, c0)), static_cast<uint32_t>(std::max(0.0, c1)));
+    } else {
+      const uint32_t g = static_cast<uint32_t>(rows[t]);
+      key[t] = morton_key(g % kb->grid1, g / kb->grid1);
     }
-    perm.resize(n);
-    std::iota(perm.begin(), perm.end(), 0u);
-    std::stable_sort(perm.begin(), perm.end(), [&](uint32_t a, uint32_t b) { return key[a] < key[b]; });
   }
+  const std::vector<uint32_t> perm = stable_order(key);
   std::vector<CsrHost> parts;
-  if (!csr_build(ptr, cols, vals, rows, perm, h.n_cols, &parts))
+  if (!(view == 0 ? csr_build(CsrForward{w, kb->cols.data(), kb->re.data(), kb->im.data()}, rows, perm, h.nnz, h.n_cols, &parts)
+                  : csr_build(CsrTranspose{ptr.data(), entries.data(), kb->re.data(), kb->im.data()}, rows, perm, h.nnz, h.n_cols, &parts)))
     return fail(TSN_ERR_RUNTIME, "out of host memory");
   // the parts one after the other: every block's offsets move by what precedes it
   CsrHost host;  // blocks, rounds, row ids and columns of all parts; values and local columns stay in parts
@@ -2627,39 +2745,57 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   d->n_csr_active_blocks = active_blocks;
   d->n_slots = host.slots;
   d->n_counters = host.counters;
-  size_t bytes = 0;
-  int rc = device_copy(host.row_ids.data(), host.row_ids.size(), &d->row_ids, &bytes);
-  if (rc == TSN_OK) rc = device_copy(host.cols.data(), host.cols.size(), &d->csr_cols, &bytes);
-  if (rc == TSN_OK) rc = device_copy(host.blocks.data(), host.blocks.size(), &d->csr_blocks, &bytes);
-  if (rc == TSN_OK) rc = device_copy(host.rounds.data(), host.rounds.size(), &d->csr_rounds, &bytes);
-  if (rc == TSN_OK) {
-    auto copy_parts = [&](auto** to, size_t count, auto part) -> int {
-      using T = std::remove_pointer_t<std::remove_pointer_t<decltype(to)>>;
-      if (count == 0) return TSN_OK;
-      TSN_HIP(hipMalloc(reinterpret_cast<void**>(to), count * sizeof(T)));
-      size_t at = 0;
-      for (const CsrHost& q : parts) {
-        const auto& v = part(q);
-        if (!v.empty()) TSN_HIP(hipMemcpy(*to + at, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-        at += v.size();
-      }
-      bytes += count * sizeof(T);
-      return TSN_OK;
-    };
-    rc = copy_parts(&d->vals, static_cast<size_t>(steps) * 64,
-                    [](const CsrHost& q) -> const std::vector<float2>& { return q.vals; });
-    if (rc == TSN_OK)
-      rc = copy_parts(&d->csr_idx, static_cast<size_t>(words) * 64,
-                      [](const CsrHost& q) -> const std::vector<uint32_t>& { return q.idx; });
+  // one allocation for all arrays, each array's parts one after the other
+  struct Piece {
+    const void* data;
+    size_t bytes, at;
+  };
+  std::vector<Piece> pieces;
+  size_t total = 0;
+  auto add = [&](const auto& v) {
+    const size_t bytes = v.size() * sizeof(*v.data());
+    if (bytes) pieces.push_back({v.data(), bytes, total});
+    total += bytes;
+  };
+  auto begin = [&] { return total = (total + 255) / 256 * 256; };
+  const size_t vals_at = begin();
+  for (const CsrHost& q : parts) add(q.vals);
+  const size_t idx_at = begin();
+  for (const CsrHost& q : parts) add(q.idx);
+  const size_t rows_at = begin();
+  add(host.row_ids);
+  const size_t cols_at = begin();
+  add(host.cols);
+  const size_t blocks_at = begin();
+  add(host.blocks);
+  const size_t rounds_at = begin();
+  add(host.rounds);
+  TSN_HIP(hipMalloc(reinterpret_cast<void**>(&d->csr_data), std::max<size_t>(total, 1)));
+  std::vector<unsigned char> stage(total <= kCsrStagedBytes ? total : 0);
+  if (!stage.empty()) {
+    for (const Piece& p : pieces) std::memcpy(stage.data() + p.at, p.data, p.bytes);
+    pieces = {Piece{stage.data(), total, 0}};
   }
-  if (rc == TSN_OK && host.slots) {
-    const std::vector<float> zeros(static_cast<size_t>(host.slots) * 2 * kMaxCoils, 0.0f);
-    const std::vector<uint32_t> zero_counters(round_up(host.counters, 4u), 0u);
-    rc = device_copy(zeros.data(), zeros.size(), &d->partials, &bytes);
-    if (rc == TSN_OK) rc = device_copy(zero_counters.data(), zero_counters.size(), &d->counters, &bytes);
+  hipError_t copied = hipSuccess;
+  for (const Piece& p : pieces)
+    if (copied == hipSuccess) copied = hipMemcpyAsync(d->csr_data + p.at, p.data, p.bytes, hipMemcpyHostToDevice, nullptr);
+  const hipError_t done = hipStreamSynchronize(nullptr);  // (also after a failure: the copies read this call's memory)
+  TSN_HIP(copied);
+  TSN_HIP(done);
+  d->vals = reinterpret_cast<float2*>(d->csr_data + vals_at);
+  d->csr_idx = reinterpret_cast<uint32_t*>(d->csr_data + idx_at);
+  d->row_ids = reinterpret_cast<int32_t*>(d->csr_data + rows_at);
+  d->csr_cols = reinterpret_cast<uint32_t*>(d->csr_data + cols_at);
+  d->csr_blocks = reinterpret_cast<CsrBlock*>(d->csr_data + blocks_at);
+  d->csr_rounds = reinterpret_cast<CsrRound*>(d->csr_data + rounds_at);
+  d->bytes = total;
+  if (host.slots) {
+    const std::vector<uint32_t> zeros(round_up(host.counters, 4u), 0u);
+    const size_t slot_bytes = static_cast<size_t>(host.slots) * kMaxCoils * sizeof(float2);
+    TSN_HIP(hipMalloc(reinterpret_cast<void**>(&d->partials), slot_bytes));
+    TSN_CHECK(device_copy(zeros.data(), zeros.size(), &d->counters, &d->bytes));
+    d->bytes += slot_bytes;
   }
-  if (rc != TSN_OK) return rc;
-  d->bytes = bytes;
   *out = owner.release();
   return TSN_OK;
 }

@@ -3,8 +3,12 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -38,6 +42,7 @@ constexpr uint32_t kCsrUnits = 256;
 constexpr uint32_t kCsrFewBlocks = 512;
 constexpr uint32_t kCsrParts = 16;
 constexpr uint32_t kCsrPartEntries = 1u << 15;
+constexpr size_t kCsrStagedBytes = 1u << 20;
 // Device column words of packed tiles hold column * 32 (a byte offset) below
 // bit 31, so a pack may have at most 2^26 columns.
 constexpr uint32_t kMaxDeviceCols = 1u << 26;
@@ -194,18 +199,43 @@ struct CsrBlock {
   uint32_t row0, n_rows, n_rounds, round0;
   uint32_t n_chunks, chunk, slot0, counter;
 };
+// A growing host array whose new elements are not initialised.
+template <typename T>
+class HostBuffer {
+ public:
+  T* grow(size_t n) {
+    if (size_ + n > capacity_) reserve(std::max(size_ + n, capacity_ * 2));
+    size_ += n;
+    return data_.get() + (size_ - n);
+  }
+  void reserve(size_t capacity) {
+    if (capacity <= capacity_) return;
+    void* p = std::realloc(data_.get(), capacity * sizeof(T));
+    if (!p) throw std::bad_alloc();
+    (void)data_.release();
+    data_.reset(static_cast<T*>(p));
+    capacity_ = capacity;
+  }
+  const T* data() const { return data_.get(); }
+  size_t size() const { return size_; }
+
+ private:
+  struct Free {
+    void operator()(T* p) const { std::free(p); }
+  };
+  std::unique_ptr<T, Free> data_;
+  size_t size_ = 0, capacity_ = 0;
+};
 // Host form of an FP32 direction's device arrays, or of one range of its rows.
 struct CsrHost {
   std::vector<CsrBlock> blocks;
   std::vector<CsrRound> rounds;
-  std::vector<uint32_t> cols, idx;
+  std::vector<uint32_t> cols;
   std::vector<int32_t> row_ids;
-  std::vector<float2> vals;
+  HostBuffer<float2> vals;
+  HostBuffer<uint32_t> idx;
   uint32_t slots = 0, counters = 0;
 };
-bool csr_build(const std::vector<uint32_t>& ptr, const std::vector<int32_t>& cols, const std::vector<float2>& vals,
-               const std::vector<int32_t>& rows, const std::vector<uint32_t>& perm, uint32_t n_cols,
-               std::vector<CsrHost>* out);
 // Floats of one partial slot: two coil blocks x (re, im) x 64 lanes x float4.
 constexpr uint32_t kSlotFloats = 2 * 2 * 64 * 4;
 // Launch order entries: a unit index, or kChunkTag | chunk index.  Units and
@@ -346,6 +376,7 @@ struct tsn_direction {
   std::vector<uint32_t> host_order;
   std::vector<void*> retired;          // earlier schedules (graphs may reference them)
   // ---- FP32 CSR (device)
+  unsigned char* csr_data = nullptr;  // the arrays below, one allocation
   int32_t* row_ids = nullptr;         // output rows of the blocks
   uint32_t* csr_cols = nullptr;       // distinct columns of the blocks
   float2* vals = nullptr;             // entry values, [steps][64] per wave
