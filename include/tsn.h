@@ -169,10 +169,15 @@ uint32_t tsn_direction_pipe_depth(const tsn_direction* dir);
  * the candidate unit sizes {2,3,4,5,6,8,10,12,14,16} x pipeline depths
  * (default and alternatives), and for 9..16 coils over both coil-wave
  * settings, writing 64-byte rows per coil block as plans do (scratch panels
- * allocated and freed here, the stream synchronized; two passes, the faster
- * of each candidate counts), and keep the fastest schedule.  Results do not
- * depend on the schedule (bitwise).  No counterpart in the reference; run
- * once per trajectory and coil count. */
+ * allocated and freed here, the stream synchronized; two passes, the second
+ * over the candidates within 5% of the best; the faster of each candidate
+ * counts), and keep the fastest schedule.  For 9..16 coils plans and batches
+ * hold both coil blocks of a panel row in one line and the calls on a
+ * caller's panels separate blocks: each layout is timed and keeps a schedule
+ * of its own, and best_unit_tiles, best_us and the getters above name that of
+ * plans and batches (the setters and tsn_direction_schedule set both).
+ * Results do not depend on the schedule (bitwise).  No counterpart in the
+ * reference; run once per trajectory and coil count. */
 int tsn_direction_autotune(tsn_direction* dir, uint32_t coils, void* stream, uint32_t* best_unit_tiles,
                            float* best_us);
 /* Device bytes the direction occupies (pack + index arrays, plus the

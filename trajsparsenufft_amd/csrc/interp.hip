@@ -18,6 +18,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <initializer_list>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -1348,11 +1349,12 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
   if (lines && d->h.n_cols > kMaxLineCols)
     return fail(TSN_ERR_ARGUMENT, "line-row panels hold at most %u columns (got %u)", kMaxLineCols, d->h.n_cols);
   InterpArgs a{};
-  a.items = d->items;
-  a.n_items = d->n_items;
+  const TileSchedule& schedule = lines ? d->line_rows : d->block_rows;
+  a.items = schedule.items;
+  a.n_items = schedule.n_items;
   a.chunks = d->chunks;
   a.n_chunks = d->n_chunks;
-  a.order = d->order;
+  a.order = schedule.order;
   a.partials = scratch ? scratch->partials : d->partials;
   a.counters = scratch ? scratch->counters : d->counters;
   if (d->n_chunks && (!a.partials || !a.counters)) return fail(TSN_ERR_ARGUMENT, "missing chunk scratch");
@@ -1383,8 +1385,8 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
     a.dc_row_stride = dc->row_stride;
     a.dc_coil_stride = dc->coil_stride;
   }
-  a.depth = d->pipe_depth;
-  const uint32_t cw = d->coil_waves;
+  a.depth = schedule.pipe_depth;
+  const uint32_t cw = schedule.coil_waves;
   if (kind == kSparseSplit) TSN_CHECK(launch_tiles<kSparseSplit>(a, panels, out_mode, conj, accumulate, cw, stream));
   else if (kind == kDenseSplit)
     TSN_CHECK(launch_tiles<kDenseSplit>(a, panels, out_mode, conj, accumulate, cw, stream));
@@ -1564,10 +1566,10 @@ static int device_copy(const T* host, size_t count, T** out, size_t* bytes) {
 static void release(tsn_direction* d) {
   if (!d) return;
   void* ptrs[] = {d->group_offsets, d->group_rows, d->tile_cols, d->tile_a, d->tile_idx,
-                  d->tile_dense, d->items, d->order, d->chunks, d->partials, d->counters, d->csr_data};
+                  d->tile_dense, d->chunks, d->partials, d->counters, d->csr_data};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  for (void* p : d->retired) (void)hipFree(p);
+  for (void* p : d->schedules) (void)hipFree(p);
   delete d;
 }
 
@@ -1600,7 +1602,7 @@ static void lpt_order(std::vector<uint32_t>& order, F tiles_of) {
 // samples / 512^2 grid / 8 coils: G 17.9 us with 14-tile units against 18.0
 // (16) and 18.1 (12); G^T 18.3 us against 18.4 (16) and 20.1 (12); smaller
 // units start more waves than the CUs hold at once.
-static int schedule_units(tsn_direction* d, uint32_t unit_tiles) {
+static int schedule_units(tsn_direction* d, uint32_t unit_tiles, std::initializer_list<TileSchedule*> into) {
   const std::vector<uint32_t>& off = d->host_offsets;
   const uint32_t groups = d->h.groups;
   uint64_t regular_tiles = 0;
@@ -1674,14 +1676,16 @@ static int schedule_units(tsn_direction* d, uint32_t unit_tiles) {
   }
   // Earlier schedules stay allocated until the direction is freed: a captured
   // graph may still hold their addresses in its kernel arguments.
-  if (d->items) d->retired.push_back(d->items);
-  if (d->order) d->retired.push_back(d->order);
-  d->items = new_items;
-  d->order = new_order;
-  d->n_items = static_cast<uint32_t>(items.size());
-  d->unit_tiles = static_cast<uint32_t>(target);
-  d->host_items = items;
-  d->host_order = order;
+  for (void* p : {static_cast<void*>(new_items), static_cast<void*>(new_order)})
+    if (p) d->schedules.push_back(p);
+  for (TileSchedule* to : into) {
+    to->items = new_items;
+    to->order = new_order;
+    to->n_items = static_cast<uint32_t>(items.size());
+    to->unit_tiles = static_cast<uint32_t>(target);
+    to->host_items = items;
+    to->host_order = order;
+  }
   d->bytes += bytes;
   return TSN_OK;
 }
@@ -2213,7 +2217,7 @@ static int upload_pack(const HostPack& p, tsn_direction** out) {
   if (rc == TSN_OK) rc = device_copy(tile_a.data(), tile_a.size(), &d->tile_a, &bytes);
   if (rc == TSN_OK) rc = device_copy(tile_idx.data(), tile_idx.size(), &d->tile_idx, &bytes);
   d->bytes = bytes;
-  if (rc == TSN_OK) rc = schedule_units(d, 0);
+  if (rc == TSN_OK) rc = schedule_units(d, 0, {&d->line_rows, &d->block_rows});
   if (rc == TSN_OK) rc = upload_chunks(d);
   if (rc != TSN_OK) {
     release(d);
@@ -2290,13 +2294,14 @@ int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* o
     // every part has its own slots and counters
     uint32_t ns = 0, nc = 0;
     const std::vector<ChunkItem> dc = long_chunks(d->host_offsets, 0, 0, 0, &ns, &nc);
-    const uint32_t nd = static_cast<uint32_t>(d->host_order.size());
+    const TileSchedule& schedule = lines ? d->line_rows : d->block_rows;
+    const uint32_t nd = static_cast<uint32_t>(schedule.host_order.size());
     for (uint32_t x = 0; x < 8; ++x) {
       const uint32_t lo = xcd_remap(x, nd), hi = x == 7 ? nd : xcd_remap(x + 1, nd);
       const uint32_t nm = static_cast<uint32_t>(members.size());
       for (uint32_t k0 = 0; k0 < nm; k0 += member_group)
       for (uint32_t i = lo; i < hi; ++i) {
-        const uint32_t e = d->host_order[i];
+        const uint32_t e = schedule.host_order[i];
         for (uint32_t k = k0; k < std::min(nm, k0 + member_group); ++k) {
           if (e & kChunkTag) {
             ChunkItem c = dc[e & ~kChunkTag];
@@ -2307,7 +2312,7 @@ int interp_batch_build(const std::vector<InterpBatchPart>& parts, InterpBatch* o
             chunks.push_back(c);
           } else {
             xcd_entries[x].push_back(static_cast<uint32_t>(items.size()));
-            items.push_back(d->host_items[e]);
+            items.push_back(schedule.host_items[e]);
             item_problem.push_back(members[k]);
           }
         }
@@ -2500,28 +2505,28 @@ int tsn_direction_schedule(tsn_direction* d, uint32_t unit_tiles) {
   if (unit_tiles > (1u << 20)) return fail(TSN_ERR_ARGUMENT, "unit_tiles %u is out of range", unit_tiles);
   TSN_HIP(hipSetDevice(d->device));
   TSN_HIP(hipDeviceSynchronize());
-  return schedule_units(d, unit_tiles);
+  return schedule_units(d, unit_tiles, {&d->line_rows, &d->block_rows});
 }
 
-uint32_t tsn_direction_unit_tiles(const tsn_direction* d) { return d ? d->unit_tiles : 0; }
+uint32_t tsn_direction_unit_tiles(const tsn_direction* d) { return d ? d->line_rows.unit_tiles : 0; }
 
 int tsn_direction_set_coil_waves(tsn_direction* d, uint32_t waves) {
   if (!d) return fail(TSN_ERR_ARGUMENT, "null direction");
   if (waves != 1 && waves != 2) return fail(TSN_ERR_ARGUMENT, "coil waves must be 1 or 2 (got %u)", waves);
-  d->coil_waves = waves;
+  d->line_rows.coil_waves = d->block_rows.coil_waves = waves;
   return TSN_OK;
 }
 
-uint32_t tsn_direction_coil_waves(const tsn_direction* d) { return d ? d->coil_waves : 0; }
+uint32_t tsn_direction_coil_waves(const tsn_direction* d) { return d ? d->line_rows.coil_waves : 0; }
 
 int tsn_direction_set_pipe_depth(tsn_direction* d, uint32_t depth) {
   if (!d) return fail(TSN_ERR_ARGUMENT, "null direction");
   if (depth > 3) return fail(TSN_ERR_ARGUMENT, "pipeline depth must be 0 (default) or 1..3");
-  d->pipe_depth = depth;
+  d->line_rows.pipe_depth = d->block_rows.pipe_depth = depth;
   return TSN_OK;
 }
 
-uint32_t tsn_direction_pipe_depth(const tsn_direction* d) { return d ? d->pipe_depth : 0; }
+uint32_t tsn_direction_pipe_depth(const tsn_direction* d) { return d ? d->line_rows.pipe_depth : 0; }
 
 int tsn_direction_autotune(tsn_direction* d, uint32_t coils, void* stream, uint32_t* best_unit_tiles,
                            float* best_us) {
@@ -2551,35 +2556,50 @@ int tsn_direction_autotune(tsn_direction* d, uint32_t coils, void* stream, uint3
   const int kind = d->values == TSN_VALUES_BF16 ? kSparseSplitBF16 : kSparseSplit;
   // candidates: unit sizes x, for 9..16 coils, one wave for both coil blocks
   // or one per block x pipeline depths (the default and the alternatives of
-  // the launch: 1 or 3 tiles ahead for one block per wave, 2 for two)
+  // the launch: 1 or 3 tiles ahead for one block per wave, 2 for two); for
+  // 9..16 coils each on line rows (plans, batches) and on separate blocks
+  // (tsn_interp_il), whose best schedules differ: 512^2 / 11 coils adjoint on
+  // blocks 33 us, 37 us with the one that is best on line rows
   struct Candidate {
+    TileSchedule* of;
     uint32_t waves, unit, depth;
   };
-  std::vector<Candidate> cands;
   const bool two = coils > static_cast<uint32_t>(kCoilsPerBlock);
-  for (uint32_t cw : two ? std::vector<uint32_t>{1u, 2u} : std::vector<uint32_t>{d->coil_waves})
-    for (uint32_t u : {2u, 3u, 4u, 5u, 6u, 8u, 10u, 12u, 14u, 16u}) {
-      std::vector<uint32_t> depths = {0u};
-      if (two && cw == 1) depths.push_back(2u);
-      if (!two) depths.insert(depths.end(), {1u, 3u});
-      for (uint32_t dp : depths) cands.push_back({cw, u, dp});
-    }
-  // two passes over the candidates, each candidate's faster pass counts
-  // (neighbouring unit sizes differ by a few percent, about the spread of
-  // one timing)
+  const bool line_rows = two && d->h.n_cols <= kMaxLineCols;
+  std::vector<Candidate> cands;
+  for (uint32_t u : {2u, 3u, 4u, 5u, 6u, 8u, 10u, 12u, 14u, 16u})
+    for (TileSchedule* of : line_rows ? std::vector<TileSchedule*>{&d->line_rows, &d->block_rows}
+                                      : std::vector<TileSchedule*>{&d->block_rows})
+      for (uint32_t cw : two ? std::vector<uint32_t>{1u, 2u} : std::vector<uint32_t>{of->coil_waves}) {
+        std::vector<uint32_t> depths = {0u};
+        if (two && cw == 1) depths.push_back(2u);
+        if (!two) depths.insert(depths.end(), {1u, 3u});
+        for (uint32_t dp : depths) cands.push_back({of, cw, u, dp});
+      }
+  // two passes, the second over the candidates within 5% of their layout's best
+  // (neighbouring unit sizes differ by a few percent, about the spread of one
+  // timing); each candidate's faster pass counts
+  struct Best {
+    Candidate c;
+    float ms;
+  };
+  Best best_lines{{&d->line_rows, d->line_rows.coil_waves, 0, d->line_rows.pipe_depth}, 0.0f};
+  Best best_blocks{{&d->block_rows, d->block_rows.coil_waves, 0, d->block_rows.pipe_depth}, 0.0f};
   std::vector<float> times(cands.size(), 0.0f);
-  Candidate best{d->coil_waves, 0, d->pipe_depth};
-  float best_ms = 0.0f;
+  uint32_t unit = 0;
   for (int pass = 0; pass < 2; ++pass)
   for (size_t ci = 0; ci < cands.size(); ++ci) {
     if (rc != TSN_OK) break;
     const Candidate& c = cands[ci];
-    d->coil_waves = c.waves;
-    d->pipe_depth = c.depth;
-    rc = schedule_units(d, c.unit);
+    Best& best = c.of == &d->line_rows ? best_lines : best_blocks;
+    if (pass == 1 && times[ci] > 1.05f * best.ms) continue;
+    if (c.unit != unit) rc = schedule_units(d, c.unit, {&d->line_rows, &d->block_rows});
+    unit = c.unit;
+    c.of->coil_waves = c.waves;
+    c.of->pipe_depth = c.depth;
     auto launch = [&]() {
       return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, 1.0f, nullptr, s,
-                           d->h.n_cols <= kMaxLineCols ? kLines : kBlocks, out);
+                           c.of == &d->line_rows ? kLines : kBlocks, out);
     };
     for (int i = 0; rc == TSN_OK && i < 3; ++i) rc = launch();
     if (rc != TSN_OK) break;
@@ -2594,22 +2614,29 @@ int tsn_direction_autotune(tsn_direction* d, uint32_t coils, void* stream, uint3
     if (rc != TSN_OK) break;
     if (pass == 1) ms = std::min(ms, times[ci]);
     times[ci] = ms;
-    if (pass == 1 && (best.unit == 0 || ms < best_ms)) {
-      best = c;
-      best_ms = ms;
-    }
+    if (best.c.unit == 0 || ms < best.ms) best = {c, ms};
+  }
+  if (!line_rows) {
+    best_lines = best_blocks;
+    best_lines.c.of = &d->line_rows;
+    if (!two) best_lines.c.waves = d->line_rows.coil_waves;
   }
   (void)hipStreamSynchronize(s);
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   if (panel) (void)hipFree(panel);
   if (out) (void)hipFree(out);
-  d->coil_waves = best.waves;
-  d->pipe_depth = best.depth;
-  if (rc == TSN_OK) rc = schedule_units(d, best.unit);
+  for (const Best& best : {best_lines, best_blocks}) {
+    best.c.of->coil_waves = best.c.waves;
+    best.c.of->pipe_depth = best.c.depth;
+  }
+  // (first both at the one, then the blocks at theirs)
+  if (rc == TSN_OK) rc = schedule_units(d, best_lines.c.unit, {&d->line_rows, &d->block_rows});
+  if (rc == TSN_OK && best_blocks.c.unit != best_lines.c.unit)
+    rc = schedule_units(d, best_blocks.c.unit, {&d->block_rows});
   if (rc != TSN_OK) return rc;
-  if (best_unit_tiles) *best_unit_tiles = best.unit;
-  if (best_us) *best_us = best_ms * 1000.0f;
+  if (best_unit_tiles) *best_unit_tiles = best_lines.c.unit;
+  if (best_us) *best_us = best_lines.ms * 1000.0f;
   return TSN_OK;
 }
 

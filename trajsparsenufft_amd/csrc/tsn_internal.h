@@ -349,6 +349,21 @@ struct tsn_kb_matrix {
   std::vector<double> coord0, coord1;    // mod(traj*grid + grid/2, grid), float64
 };
 
+namespace tsn {
+// A work schedule of a packed direction and how its launches run (device
+// arrays owned by the direction).
+struct TileSchedule {
+  const WorkItem* items = nullptr;  // runs of groups with <= kSplitAboveTiles tiles each
+  const uint32_t* order = nullptr;  // [n_items + n_chunks] launch order (kChunkTag marks chunks)
+  uint32_t n_items = 0;
+  uint32_t unit_tiles = 0;                  // tile budget of one regular unit
+  uint32_t coil_waves = kDefaultCoilWaves;  // interleaved launches of 9..16 coils: waves per entry (1 or 2)
+  uint32_t pipe_depth = 0;  // tiles in flight ahead of the multiply: 0 = the kernel's default, 1..3
+  std::vector<WorkItem> host_items;         // (batched launches merge schedules)
+  std::vector<uint32_t> host_order;
+};
+}  // namespace tsn
+
 struct tsn_direction {
   tsn_pack_header h{};
   int device = 0;
@@ -361,20 +376,16 @@ struct tsn_direction {
   uint4* tile_a = nullptr;           // [tiles * 64] per lane {re 4xf16, im 4xf16}
   uint16_t* tile_idx = nullptr;      // [tiles * 64] per lane sparse index byte re | im << 8
   uint4* tile_dense = nullptr;       // [tiles * 64 * 2] per lane {re 8xf16}, {im 8xf16}; built on first use
-  tsn::WorkItem* items = nullptr;    // runs of groups with <= kSplitAboveTiles tiles each
   tsn::ChunkItem* chunks = nullptr;  // chunks of the longer groups (fixed by the pack)
   float* partials = nullptr;         // [slots][kSlotFloats] partial sums of the chunks
   uint32_t* counters = nullptr;      // [long groups] arrival counters, zero between launches
-  uint32_t n_items = 0, n_chunks = 0;
+  uint32_t n_chunks = 0;
   uint32_t n_slots = 0, n_counters = 0;  // sizes of the chunk scratch (ChunkScratch)
-  uint32_t unit_tiles = 0;           // tile budget of one regular unit
-  uint32_t coil_waves = tsn::kDefaultCoilWaves;  // interleaved launches of 9..16 coils: waves per entry (1 or 2)
-  uint32_t pipe_depth = 0;  // tiles in flight ahead of the multiply: 0 = the kernel's default, 1..3
   std::vector<uint32_t> host_offsets;  // group_offsets kept for rescheduling
-  uint32_t* order = nullptr;         // [n_items + n_chunks] launch order (kChunkTag marks chunks)
-  std::vector<tsn::WorkItem> host_items;  // the current schedule (batched launches merge it)
-  std::vector<uint32_t> host_order;
-  std::vector<void*> retired;          // earlier schedules (graphs may reference them)
+  // schedules of launches on line rows (9..16 coils in plans and batches) and of
+  // the others: the autotuner finds different ones
+  tsn::TileSchedule line_rows, block_rows;
+  std::vector<void*> schedules;        // every schedule's arrays, earlier ones too (graphs may reference them)
   // ---- FP32 CSR (device)
   unsigned char* csr_data = nullptr;  // the arrays below, one allocation
   int32_t* row_ids = nullptr;         // output rows of the blocks

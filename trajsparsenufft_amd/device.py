@@ -93,8 +93,9 @@ class Direction:
 
     def autotune(self, coils: int = 8) -> tuple[int, float]:
         """Time the interpolation over the candidate unit sizes, pipeline depths
-        and (9..16 coils) waves per entry, and keep the fastest; returns
-        (unit_tiles, microseconds per launch)."""
+        and (9..16 coils) waves per entry, and keep the fastest, for 9..16
+        coils one each for plans and batches and for calls on a caller's panels;
+        returns (unit_tiles, microseconds per launch) of the former."""
 
         best, us = C.c_uint32(), C.c_float()
         check(lib().tsn_direction_autotune(self._h, int(coils), _stream(), C.byref(best), C.byref(us)))
