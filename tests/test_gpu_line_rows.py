@@ -45,3 +45,21 @@ def test_line_rows_are_bitwise_invariant(coils, precision):
     one = build_plan(packs, dev(smaps[:8]), precision).forward(x)
     torch.cuda.synchronize()
     assert np.array_equal(np.ascontiguousarray(torch.view_as_real(one).cpu().numpy()).view(np.uint32), ref[0][:8])
+
+
+@pytest.mark.parametrize("precision", ["split16", "splitbf16", "dense16", "hi16"])
+@pytest.mark.parametrize("coils", [9, 11, 16])
+def test_second_block_of_line_rows_matches_the_one_block_layout(coils, precision):
+    """Coils 8 .. are the second half of every line: their samples have the bits
+    of a plan that holds them alone in the one-block layout."""
+
+    need_gpu()
+    from trajsparsenufft_amd import synth
+    from trajsparsenufft_amd.recon import build_plan
+    _, packs = small_case(32, 120)
+    smaps = synth.coil_maps(coils, 32)
+    x = dev(synth.phantom(32, seed=coils))
+    both = build_plan(packs, dev(smaps), precision).forward(x)
+    second = build_plan(packs, dev(smaps[8:]), precision).forward(x)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.view_as_real(both[8:]), torch.view_as_real(second))
