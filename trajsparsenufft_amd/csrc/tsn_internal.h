@@ -57,9 +57,11 @@ constexpr uint32_t kMaxDeviceCols = 1u << 26;
 // is left moves 5.1 TB/s past L2); eight such frames 701 -> 488 and 608 -> 500
 // us per step; 512^2 / 11 coils / spiral 30.7 -> 24.9 and 20.4 -> 19.0 us.
 enum PanelMode { kHalves = 0, kBlocks = 1, kLines = 2 };
-// Byte offsets of line rows (column * 128) are 32-bit; plans and batches with
-// more columns keep separate blocks.
-constexpr uint32_t kMaxLineCols = 1u << 25;
+// Byte offsets of line rows (column * 128) and the size of the buffer that
+// checks them are 32-bit, so a panel stays below 4 GiB (at 4 GiB the clamped
+// size would cut its last word off); plans and batches with more columns keep
+// separate blocks.
+constexpr uint32_t kMaxLineCols = (1u << 25) - 1;
 // Per-tile operand offsets are signed 32-bit buffer offsets: sparse operands
 // (1 KiB per tile) hold 2^21 tiles, expanded dense-control tiles (2 KiB) 2^20.
 constexpr uint32_t kMaxDeviceTiles = 1u << 21;
