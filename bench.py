@@ -148,7 +148,9 @@ def batch_workloads(torch, log, reps=3):
         img = outs[f].image.cpu().numpy()
         nrmse.append(magnitude_nrmse(img, ref.image.cpu().numpy()))
         truth_err.append(magnitude_nrmse(img, truth[f]))
-    # interpolation HBM rate at this shape (16 coils: two coil blocks per launch)
+    # HBM rate of the interpolation calls at this shape (16 coils: two coil
+    # blocks per launch) on a caller's panels, which hold separate coil blocks;
+    # plans and batches hold both blocks of a panel row in one line
     fh = packs.forward.header
     m, g, nnz = fh["output_size"], fh["n_cols"], fh["nnz"]
     fwd, adj = Direction.upload(packs.forward), Direction.upload(packs.adjoint)
@@ -162,8 +164,7 @@ def batch_workloads(torch, log, reps=3):
     gp, sp = panel(g), panel(m)
     out_s = torch.empty((2, m, 16), dtype=torch.int32, device="cuda")
     out_g = torch.zeros((g, nc), dtype=torch.complex64, device="cuda")
-    tuned = {"forward": fwd.coil_waves, "adjoint": adj.coil_waves}
-    interp = {}
+    interp = {"panels": "separate coil blocks (tsn_interp_il); plans and batches use line rows"}
     for waves in (1, 2):
         fwd.coil_waves = adj.coil_waves = waves
         f_ms = time_launches(torch, lambda: device.interp_il(fwd, gp, out_s, nc, False, False, 1.0, "split_il"), 20, 5)
@@ -172,11 +173,12 @@ def batch_workloads(torch, log, reps=3):
             b = nnz * 8 + 2 * n_in * 2 * nc * 2 + n_out * nc * 8
             row = {"us": ms * 1e3, "bytes": b, "GBs": b / (ms * 1e-3) / 1e9,
                    "frac_of_peak": b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS}
-            interp.setdefault(name, {})[f"coil_waves_{waves}"] = row
-            if waves == tuned[name]:
-                interp[name].update(row)
-        log(f"[bench] frames interp, {waves} wave(s) per entry: forward {f_ms * 1e3:.1f} us, adjoint {a_ms * 1e3:.1f} us")
-    interp["tuned_coil_waves"] = tuned
+            both = interp.setdefault(name, {})
+            if row["us"] < both.get("us", float("inf")):
+                both.update(row, coil_waves=waves)
+            both[f"coil_waves_{waves}"] = row
+        log(f"[bench] frames interp (separate coil blocks), {waves} wave(s) per entry: forward {f_ms * 1e3:.1f} us, "
+            f"adjoint {a_ms * 1e3:.1f} us")
     out["frames"] = {"workload": "24 frames 384x384 / 768x768, 16 coils, shared golden-angle radial 600x768 pack, "
                                  "35 dB, 30 CG batched across frames, split16",
                      "frames_per_s": frames * 1000.0 / frames_ms, "batched_ms": frames_ms,
@@ -416,7 +418,7 @@ def interp_roofline(torch, packs, steps, warmup, log):
                            steps, warmup)
     for name, ms, n_in, n_out, conj in (("fp32_forward", f32_ms, g, m, "false"), ("fp32_adjoint", a32_ms, m, g, "true")):
         b = nnz * 12 + n_in * COILS * 8 + n_out * COILS * 8
-        kernel = f"interp_csr_kernel<2, 1, {conj}, false>"
+        kernel = f"interp_csr_kernel<2, 2, 1, {conj}, false>"
         res[name] = {"kernel": kernel, "us": ms * 1e3, "bytes": b, "GBs": b / (ms * 1e-3) / 1e9,
                      "frac": b / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": measured_traffic(kernel)}
         log(f"[bench] FP32 CSR {name[5:]} {ms * 1e3:.1f} us ({res[name]['GBs']:.0f} GB/s algorithmic)")
