@@ -449,9 +449,9 @@ __device__ __forceinline__ void fetch_ops(const TileRsrc<NB>& r, int t, const Ti
     // Whole 128-byte lines, 16 bytes a lane: lanes n < 8 of quarter q read its
     // columns 8q .. 8q + 3, lanes n >= 8 columns 8q + 4 .. 8q + 7, 16-byte quad
     // 4 ((n >> 1) & 1) + 2 ((n >> 2) & 1) + (n & 1) of each (block, part, coil
-    // half; mma_tile exchanges half of the words with lane n ^ 8).  Rows of 128 bytes in L2, 32 columns a step, 16 waves a CU: 80
-    // cycles a CU, against 104 as two 64-byte halves in 4-byte loads and 140
-    // in 8-byte loads.
+    // half; mma_tile exchanges half of the words with lane n ^ 8).  Rows of 128
+    // bytes in L2, 32 columns a step, 16 waves a CU: 80 cycles a CU, against
+    // 104 as two 64-byte halves in 4-byte loads and 140 in 8-byte loads.
     static_assert(NB == 2, "line rows hold two coil blocks");
     const uint32_t quad = ((n & 2) << 5) | ((n & 4) << 3) | ((n & 1) << 4);
 #pragma unroll
@@ -844,8 +844,8 @@ struct CsrArgs {
 // 5.4 -> 5.0, 456 blocks (128^2, 8 coils) 6.0 -> 5.8; 584 blocks 7.8 -> 7.7 at 8
 // coils, 11.6 -> 11.9 at 16; 960 blocks 7.8 -> 8.1, 1392 blocks 8.6 -> 9.5.
 // Measured against one lane group per row that gathered every entry from memory
-// (512^2 / 8 coils): forward 43-46 -> 21 us, adjoint
-// 59-65 -> 27.5 us, sums bit for bit the same.
+// (512^2 / 8 coils): forward 43-46 -> 20 us, adjoint 59-65 -> 26 us, sums bit
+// for bit the same.
 template <int CTRL>
 __device__ __forceinline__ float quad_bcast(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
@@ -1402,13 +1402,15 @@ static int launch_interp_impl(const tsn_direction* d, int kind, const void* hi, 
 int launch_interp(const tsn_direction* d, int kind, const void* hi, const void* res, uint32_t coils,
                   int out_mode, bool conj, bool accumulate, float scale, float* out_f32,
                   hipStream_t stream, int panels, uint32_t* out_il, const ChunkScratch* scratch) {
-  return launch_interp_impl(d, kind, hi, res, coils, out_mode, conj, accumulate, scale, out_f32, stream, panels, out_il, nullptr, scratch);
+  return launch_interp_impl(d, kind, hi, res, coils, out_mode, conj, accumulate, scale, out_f32, stream, panels,
+                            out_il, nullptr, scratch);
 }
 
 int launch_interp_dc(const tsn_direction* d, int kind, const uint32_t* panel, uint32_t coils, float scale,
                      const DcTerms& dc, uint32_t* out_il, hipStream_t s, const ChunkScratch* scratch, int panels) {
   if (!dc.y) return fail(TSN_ERR_ARGUMENT, "missing measurements");
-  return launch_interp_impl(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, scale, nullptr, s, panels, out_il, &dc, scratch);
+  return launch_interp_impl(d, kind, panel, nullptr, coils, kOutSplit16IL, false, false, scale, nullptr, s, panels,
+                            out_il, &dc, scratch);
 }
 
 int launch_dc_residual(const float2* pred, uint32_t rows, uint32_t coils, const DcTerms& dc, bool bf16,
@@ -2004,9 +2006,10 @@ static void csr_balance(std::vector<tsn::CsrBlock>* blocks, const std::vector<ts
 
 // Blocks of an FP32 direction: the rows of the view in the order `perm` (row t
 // is output row rows[t]), cut into up to kCsrParts ranges of equally many
-// entries (to within a row) built side by side (false: out of memory).  In a range, short rows form groups of up to 64 rows
-// naming at most kCsrCols distinct columns (one round), long rows groups of up
-// to 16 rows of equally many chunks, one block per chunk.
+// entries (to within a row) built side by side (false: out of memory).  In a
+// range, short rows form groups of up to 64 rows naming at most kCsrCols
+// distinct columns (one round), long rows groups of up to 16 rows of equally
+// many chunks, one block per chunk.
 template <typename View>
 static bool csr_build(const View& view, const std::vector<int32_t>& rows, const std::vector<uint32_t>& perm,
                       uint32_t entries, uint32_t n_cols, std::vector<tsn::CsrHost>* out) {
@@ -2722,8 +2725,10 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   }
   const std::vector<uint32_t> perm = stable_order(key);
   std::vector<CsrHost> parts;
-  if (!(view == 0 ? csr_build(CsrForward{w, kb->cols.data(), kb->re.data(), kb->im.data()}, rows, perm, h.nnz, h.n_cols, &parts)
-                  : csr_build(CsrTranspose{ptr.data(), entries.data(), kb->re.data(), kb->im.data()}, rows, perm, h.nnz, h.n_cols, &parts)))
+  const CsrForward forward{w, kb->cols.data(), kb->re.data(), kb->im.data()};
+  const CsrTranspose transpose{ptr.data(), entries.data(), kb->re.data(), kb->im.data()};
+  if (!(view == 0 ? csr_build(forward, rows, perm, h.nnz, h.n_cols, &parts)
+                  : csr_build(transpose, rows, perm, h.nnz, h.n_cols, &parts)))
     return fail(TSN_ERR_RUNTIME, "out of host memory");
   // the parts one after the other: every block's offsets move by what precedes it
   CsrHost host;  // blocks, rounds, row ids and columns of all parts; values and local columns stay in parts
@@ -2817,7 +2822,8 @@ static int upload_csr(const tsn_kb_matrix* kb, int view, tsn_direction** out) {
   }
   hipError_t copied = hipSuccess;
   for (const Piece& p : pieces)
-    if (copied == hipSuccess) copied = hipMemcpyAsync(d->csr_data + p.at, p.data, p.bytes, hipMemcpyHostToDevice, nullptr);
+    if (copied == hipSuccess)
+      copied = hipMemcpyAsync(d->csr_data + p.at, p.data, p.bytes, hipMemcpyHostToDevice, nullptr);
   const hipError_t done = hipStreamSynchronize(nullptr);  // (also after a failure: the copies read this call's memory)
   TSN_HIP(copied);
   TSN_HIP(done);
@@ -2895,7 +2901,8 @@ int tsn_interp_il(const tsn_direction* d, const void* panel, void* out, uint32_t
   const int kind = d->values == TSN_VALUES_BF16 ? kSparseSplitBF16 : kSparseSplit;
   if (out_layout == TSN_OUT_SPLIT_IL) {
     if (accumulate) return fail(TSN_ERR_ARGUMENT, "a split-panel output cannot accumulate");
-    return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, conjugate != 0, false, scale, nullptr, static_cast<hipStream_t>(stream), kBlocks, static_cast<uint32_t*>(out));
+    return launch_interp(d, kind, panel, nullptr, coils, kOutSplit16IL, conjugate != 0, false, scale, nullptr,
+                         static_cast<hipStream_t>(stream), kBlocks, static_cast<uint32_t*>(out));
   }
   return launch_interp(d, kind, panel, nullptr, coils, out_layout, conjugate != 0, accumulate != 0, scale,
                        static_cast<float*>(out), static_cast<hipStream_t>(stream), kBlocks, nullptr);

@@ -33,7 +33,7 @@ constexpr uint32_t kDefaultCoilWaves = 1;
 // and of a chunk of a longer one, rows of a run of empty rows, compute units
 // that a direction's blocks should cover, blocks up to which a launch splits the
 // coils, ranges of rows that csr_build works on side by side (at most, and their
-// entries at least).
+// entries at least), bytes up to which an upload is one copy.
 constexpr uint32_t kCsrCols = 255;
 constexpr uint32_t kCsrShortEntries = 64;
 constexpr uint32_t kCsrChunkEntries = 256;
